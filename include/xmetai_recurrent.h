@@ -264,8 +264,10 @@ int xm_softmax_cpu(const float *in, const int64_t *shape, int32_t rank, int64_t 
  *   "gdn2_rows"      1, 2, 4: rows of 16 lanes per value column of the fused kernel
  *   "m3_path"        1: Mamba3SisoFn token-by-token kernel
  *   "ss_lpc"         1, 2, 4, 8, 16: SelectiveScanFn lanes per channel (d_state <= 16)
- *   "ss_split"       1: SelectiveScanFn channel-block kernel only; 2: the
- *                    sequence-split kernel wherever it applies
+ *   "ss_split"       1: SelectiveScanFn channel-block kernel over the whole
+ *                    sequence only; 2: the sequence-parallel kernel wherever it
+ *                    applies; 3: the channel-block kernel in segments of the
+ *                    sequence wherever the output rows hold their records
  *   "gdn2_kpw4"      1: chunked GDN-2 above 128 keys with 4 key tiles per wave
  *   "gdn2_windowed"  1: chunked GDN-2 in windows of 128 chunks
  *   "gdn2_split"     1: chunked GDN-2 never split along the sequence; 2: split

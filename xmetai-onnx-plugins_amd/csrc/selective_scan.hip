@@ -41,10 +41,21 @@ namespace {
 using namespace ssdev;
 
 constexpr int kThreads = 256;
-// Sequence-split selection: single-pass workgroups below this count (one per
-// CU), sequences at least this long.
+// The kernel's part of the work (described at the kernel).
+enum Mode { kWhole, kSegState, kSegOut };
+struct SegSplit {
+    int count, len;   // segments, tokens per segment (the last may be shorter)
+};
+// Sequence-split selection (ChoosePlan): considered below this many channel
+// blocks (workgroups of the whole pass), for sequences at least this long.
 constexpr long long kSegMaxChannelBlocks = 256;
 constexpr int kSegMinSeqlen = 256;
+constexpr long long kSplitMaxChannelBlocks = 320;
+// Segments: enough workgroups for five per CU (what the VGPRs admit), of 128
+// tokens or more.
+constexpr long long kSplitTarget = 1280;
+constexpr int kSplitMax = 16;
+constexpr int kSplitMinLen = 128;
 
 // Tokens per tile: 32 fp32 = one 128-byte line per (channel, tile), so every
 // line of u and delta is consumed by the load that fetched it (rows are
@@ -71,14 +82,27 @@ __device__ __forceinline__ float LaneGroupSum(float x) {
     return x;
 }
 
-// FAST: seqlen % 4 == 0, 16-byte aligned rows, dim_per_group % CPW == 0 and a
-// workgroup's rows under 2 GiB.
+// FAST: rows on 4-byte boundaries, dim_per_group % CPW == 0 and a workgroup's
+// rows under 2 GiB.
 // Full tiles then move as float4 with no guards, and the one-tile-ahead
 // prefetch of u/delta/B/C stays in flight through the recurrence.  A ragged
 // last tile (seqlen % 32 != 0) is peeled off the loop and loaded with guards.
 // Without FAST every load is guarded (clamped address + select).
-template <typename IT, int LPC, int SPL, bool BVAR, bool CVAR, bool FAST>
-__global__ __launch_bounds__(kThreads) void SelectiveScanFwdKernel(SelectiveScanParams p) {
+//
+// MODE kWhole: the whole sequence.  The sequence split runs two launches of
+// split.count segments of split.len tokens (a multiple of the tile) per
+// channel block, so that few channel blocks still fill the chip:
+//  * kSegState: segments 0 .. count - 2 from a zero state, the state alone (no
+//    C, no y): 5.4 of the 8.2 issue slots per state and token of a whole
+//    pass.  Writes each channel's sum of delta' and end state.
+//  * kSegOut: every segment from its true start state, the composition of the
+//    records of the segments before it (h <- exp2(A sum delta') h + h_end).
+// The records live in the output rows that the later segments will write:
+// segment s's go into slot s of every later segment's rows, so a workgroup of
+// the second launch reads only rows that it alone overwrites, before its
+// first store, and no scratch is needed.
+template <typename IT, int LPC, int SPL, bool BVAR, bool CVAR, bool FAST, int MODE>
+__global__ __launch_bounds__(kThreads) void SelectiveScanFwdKernel(SelectiveScanParams p, SegSplit split) {
     constexpr int CPW = kThreads / LPC;      // channels per workgroup
     constexpr int NP = LPC * SPL;            // padded state count
     constexpr int kTile = Tile<CPW, NP>::T;
@@ -86,14 +110,16 @@ __global__ __launch_bounds__(kThreads) void SelectiveScanFwdKernel(SelectiveScan
     constexpr int kQ4 = Tile<CPW, NP>::Q4;
     constexpr int ITEMS = CPW * kQ4;         // (channel, 4-token) items per tile
     constexpr int IPT = (ITEMS + kThreads - 1) / kThreads;
-    constexpr int NBC = (BVAR ? 1 : 0) + (CVAR ? 1 : 0);
+    constexpr bool kState = MODE == kSegState;
+    constexpr bool CLOAD = CVAR && !kState;   // C rows are read
+    constexpr int NBC = (BVAR ? 1 : 0) + (CLOAD ? 1 : 0);
     constexpr int BCPT = NBC == 0 ? 1 : (NBC * NP * kQ4 + kThreads - 1) / kThreads;
 
     __shared__ __attribute__((aligned(16))) float sDl[CPW * kRow];        // delta' per (channel, token)
     __shared__ __attribute__((aligned(16))) float sDu[CPW * kRow];        // delta' * u
     __shared__ __attribute__((aligned(16))) float sB[BVAR ? NP * kRow : 1];
-    __shared__ __attribute__((aligned(16))) float sC[CVAR ? NP * kRow : 1];
-    __shared__ __attribute__((aligned(16))) float sY[CPW * kRow];         // sum over states per (channel, token)
+    __shared__ __attribute__((aligned(16))) float sC[CLOAD ? NP * kRow : 1];
+    __shared__ __attribute__((aligned(16))) float sY[kState ? 1 : CPW * kRow];   // sum over states per (channel, token)
 
     const int tid = threadIdx.x;
     const int L = p.seqlen;
@@ -101,6 +127,14 @@ __global__ __launch_bounds__(kThreads) void SelectiveScanFwdKernel(SelectiveScan
     const int dpg = p.dim_per_group;
     const int ncb = (dpg + CPW - 1) / CPW;
     int wg = blockIdx.x;
+    int seg = 0, tb = 0, te = L;             // this workgroup's segment, its tokens [tb, te)
+    if constexpr (MODE != kWhole) {
+        const int blocks = ncb * p.groups_b * p.batch;
+        seg = wg / blocks;
+        wg -= seg * blocks;
+        tb = seg * split.len;
+        te = min(L, tb + split.len);
+    }
     const int cb = wg % ncb;
     wg /= ncb;
     const int g = wg % p.groups_b;
@@ -149,10 +183,34 @@ __global__ __launch_bounds__(kThreads) void SelectiveScanFwdKernel(SelectiveScan
     // Zero the padded state rows once; tiles only overwrite rows < N.
     if (BVAR)
         for (int i = tid; i < (NP - N) * kRow; i += kThreads) sB[N * kRow + i] = 0.0f;
-    if (CVAR)
+    if (CLOAD)
         for (int i = tid; i < (NP - N) * kRow; i += kThreads) sC[N * kRow + i] = 0.0f;
 
-    float bias[IPT], dsk[IPT];
+    // The records in channel c's rows of segment s2: slot s holds segment s's
+    // sum of delta' and its N end states, from the first 4-byte boundary on.
+    auto record = [&](int c, int s2, int s) __attribute__((always_inline)) {
+        const uintptr_t a = reinterpret_cast<uintptr_t>(ob + static_cast<size_t>(c) * L + static_cast<size_t>(s2) * split.len);
+        return reinterpret_cast<float *>((a + 3) & ~static_cast<uintptr_t>(3)) + static_cast<size_t>(s) * (N + 1);
+    };
+    if constexpr (MODE == kSegOut) {
+        if (lane_ok)
+            for (int s = 0; s < seg; ++s) {
+                const float *rec = record(lc, seg, s);
+                const float sum = rec[0];
+#pragma unroll
+                for (int j = 0; j < SPL; ++j) {
+                    const int n = lq * SPL + j;
+                    const float end = n < N ? rec[1 + n] : 0.0f;
+                    // the decay in two halves: it may leave the range of a
+                    // float where its product with h does not; a zero state
+                    // stays zero under any growth
+                    const float half = __builtin_amdgcn_exp2f(0.5f * (sum * A2[j]));
+                    h[j] = h[j] == 0.0f ? end : fmaf(half * h[j], half, end);
+                }
+            }
+    }
+
+    float bias[IPT], dsk[IPT], dsum[IPT];
 #pragma unroll
     for (int k = 0; k < IPT; ++k) {
         const int it = tid + k * kThreads;
@@ -160,6 +218,7 @@ __global__ __launch_bounds__(kThreads) void SelectiveScanFwdKernel(SelectiveScan
         const bool ok = it < ITEMS && c < nvalid;
         bias[k] = (ok && p.delta_bias) ? p.delta_bias[cbase + c] : 0.0f;
         dsk[k] = (ok && p.D) ? p.D[cbase + c] : 0.0f;
+        dsum[k] = 0.0f;   // kSegState: sum of delta' over this item's tokens
     }
 
     // ---- tile loads (global -> registers) ----------------------------------
@@ -178,8 +237,9 @@ __global__ __launch_bounds__(kThreads) void SelectiveScanFwdKernel(SelectiveScan
     }
     // Two register sets of a tile's loads, used in turn by consecutive full
     // tiles, so a prefetch lands where it is consumed (no register copies).
-    F4 uA[IPT], dA[IPT], bcA[BCPT], uB[IPT], dB[IPT], bcB[BCPT];
-    auto load_full = [&](int t0, F4 (&ureg)[IPT], F4 (&dreg)[IPT], F4 (&bcreg)[BCPT])
+    using R4 = Raw4<IT>;
+    R4 uA[IPT], dA[IPT], bcA[BCPT], uB[IPT], dB[IPT], bcB[BCPT];
+    auto load_full = [&](int t0, R4 (&ureg)[IPT], R4 (&dreg)[IPT], R4 (&bcreg)[BCPT])
                          __attribute__((always_inline)) {   // FAST, whole tile in range: no guards
 #pragma unroll
         for (int k = 0; k < IPT; ++k) {
@@ -192,8 +252,8 @@ __global__ __launch_bounds__(kThreads) void SelectiveScanFwdKernel(SelectiveScan
             for (int k = 0; k < BCPT; ++k) {
                 const int it = min(tid + k * kThreads, NBC * per - 1);
                 const int r = it % per;
-                const IT *row = ((BVAR && it < per) ? Bb : Cb) + static_cast<size_t>(r / kQ4) * L;
-                bcreg[k] = LoadRow4Fast(row, t0 + (r % kQ4) * 4);
+                const IT *row = ((BVAR && (!CLOAD || it < per)) ? Bb : Cb) + static_cast<size_t>(r / kQ4) * L;
+                bcreg[k] = LoadRaw4(row, t0 + (r % kQ4) * 4);
             }
         }
     };
@@ -213,7 +273,7 @@ __global__ __launch_bounds__(kThreads) void SelectiveScanFwdKernel(SelectiveScan
             for (int k = 0; k < BCPT; ++k) {
                 const int it = min(tid + k * kThreads, NBC * per - 1);
                 const int r = it % per;
-                const IT *row = ((BVAR && it < per) ? Bb : Cb) + static_cast<size_t>(r / kQ4) * L;
+                const IT *row = ((BVAR && (!CLOAD || it < per)) ? Bb : Cb) + static_cast<size_t>(r / kQ4) * L;
                 bcreg[k] = LoadRow4Guarded(row, t0 + (r % kQ4) * 4, L, true);
             }
         }
@@ -249,6 +309,7 @@ __global__ __launch_bounds__(kThreads) void SelectiveScanFwdKernel(SelectiveScan
                     duv.v[e] = x * ureg[k].v[e];
                     skip[k].v[e] = dsk[k] * ureg[k].v[e];
                 }
+                if constexpr (kState) dsum[k] += (dlv.v[0] + dlv.v[1]) + (dlv.v[2] + dlv.v[3]);
                 *reinterpret_cast<float4 *>(&sDl[c * kRow + q4 * 4]) = make_float4(dlv.v[0], dlv.v[1], dlv.v[2], dlv.v[3]);
                 *reinterpret_cast<float4 *>(&sDu[c * kRow + q4 * 4]) = make_float4(duv.v[0], duv.v[1], duv.v[2], duv.v[3]);
             }
@@ -259,7 +320,7 @@ __global__ __launch_bounds__(kThreads) void SelectiveScanFwdKernel(SelectiveScan
             for (int k = 0; k < BCPT; ++k) {
                 const int it = tid + k * kThreads;
                 if (it < NBC * per) {
-                    const bool isB = BVAR && it < per;
+                    const bool isB = BVAR && (!CLOAD || it < per);
                     const int r = it % per;
                     float *dst = (isB ? sB : sC) + (r / kQ4) * kRow + (r % kQ4) * 4;
                     *reinterpret_cast<float4 *>(dst) = make_float4(bcreg[k].v[0], bcreg[k].v[1], bcreg[k].v[2], bcreg[k].v[3]);
@@ -287,7 +348,7 @@ __global__ __launch_bounds__(kThreads) void SelectiveScanFwdKernel(SelectiveScan
                     const float4 x = *reinterpret_cast<const float4 *>(sB + (lq * SPL + j) * kRow + q4 * 4);
                     bv[0] = x.x; bv[1] = x.y; bv[2] = x.z; bv[3] = x.w;
                 }
-                if constexpr (CVAR) {
+                if constexpr (CLOAD) {
                     const float4 x = *reinterpret_cast<const float4 *>(sC + (lq * SPL + j) * kRow + q4 * 4);
                     cv[0] = x.x; cv[1] = x.y; cv[2] = x.z; cv[3] = x.w;
                 }
@@ -296,13 +357,15 @@ __global__ __launch_bounds__(kThreads) void SelectiveScanFwdKernel(SelectiveScan
                     const float a = __builtin_amdgcn_exp2f(dlv[e] * A2[j]);
                     const float bt = BVAR ? bv[e] * duv[e] : duv[e];
                     h[j] = fmaf(a, h[j], bt);                 // (a1*a0, a1*b0 + b1)
+                    if constexpr (kState) continue;
                     float cc;
                     if constexpr (CVAR) cc = BVAR ? cv[e] : bco[j] * cv[e];
                     else cc = BVAR ? cco[j] : bco[j];
                     y[e] = fmaf(h[j], cc, y[e]);              // out += h * C
                 }
             }
-            if constexpr (LPC == 8) {
+            if constexpr (kState) {
+            } else if constexpr (LPC == 8) {
                 // lanes c and c + 8 hold the same sum for the same slot: both
                 // write it (no exec-mask region inside the token loop)
                 rY[q4 * 4 + SwapReducedToken(lane)] = SwapReduce8x4(y);
@@ -323,6 +386,7 @@ __global__ __launch_bounds__(kThreads) void SelectiveScanFwdKernel(SelectiveScan
 
     // ---- phase 3: add D*u, store y -------------------------------------------
     auto phase3 = [&](int t0, bool full) __attribute__((always_inline)) {
+        if constexpr (kState) return;
 #pragma unroll
         for (int k = 0; k < IPT; ++k) {
             const int it = tid + k * kThreads;
@@ -343,12 +407,22 @@ __global__ __launch_bounds__(kThreads) void SelectiveScanFwdKernel(SelectiveScan
         // were last read before the previous barrier.
     };
 
-    const int nfull = FAST ? L / kTile : 0;   // tiles taken on the unguarded path
+    const int nfull = FAST ? (te - tb) / kTile : 0;   // tiles taken on the unguarded path
     // a full tile from one register set, prefetching the next tile into the other
-    auto full_tile = [&](int i, F4 (&u)[IPT], F4 (&d)[IPT], F4 (&bc)[BCPT], F4 (&nu)[IPT], F4 (&nd)[IPT],
-                         F4 (&nbc)[BCPT]) __attribute__((always_inline)) {
-        const int t0 = i * kTile;
-        phase1(t0, true, u, d, bc);
+    auto full_tile = [&](int i, const R4 (&u)[IPT], const R4 (&d)[IPT], const R4 (&bc)[BCPT], R4 (&nu)[IPT], R4 (&nd)[IPT],
+                         R4 (&nbc)[BCPT]) __attribute__((always_inline)) {
+        const int t0 = tb + i * kTile;
+        F4 uw[IPT], dw[IPT], bcw[BCPT];
+#pragma unroll
+        for (int k = 0; k < IPT; ++k) {
+            uw[k] = Widen4<IT>(u[k]);
+            dw[k] = Widen4<IT>(d[k]);
+        }
+        if constexpr (NBC > 0) {
+#pragma unroll
+            for (int k = 0; k < BCPT; ++k) bcw[k] = Widen4<IT>(bc[k]);
+        }
+        phase1(t0, true, uw, dw, bcw);
         __syncthreads();
         if (i + 1 < nfull) load_full(t0 + kTile, nu, nd, nbc);   // prefetch; the tail tile loads after the loop
         phase2();
@@ -356,7 +430,7 @@ __global__ __launch_bounds__(kThreads) void SelectiveScanFwdKernel(SelectiveScan
         phase3(t0, true);
     };
     if (nfull > 0) {   // the only path into the full-tile loop
-        load_full(0, uA, dA, bcA);
+        load_full(tb, uA, dA, bcA);
         // A tile is entered with its loads issued before the previous tile's
         // IPT stores (vmcnt counts both).  Dropped stores (beyond the
         // descriptor) after tile 0's loads give the first entry the same
@@ -366,8 +440,10 @@ __global__ __launch_bounds__(kThreads) void SelectiveScanFwdKernel(SelectiveScan
         // 5120 x 2048 0.3407 -> 0.3343 ms, 2 x 4096 x 4096 0.2225 -> 0.2131,
         // 4 x 5120 x 2048 0.2045 -> 0.2016 (an unconditional prefetch on top,
         // the last tile reloaded: 0.3323, 0.2295, 0.2012).
+        if constexpr (!kState) {
 #pragma unroll
-        for (int k = 0; k < IPT; ++k) SsBufStore4<IT>(ryo, kSsDropOffset, 0, F4{});
+            for (int k = 0; k < IPT; ++k) SsBufStore4<IT>(ryo, kSsDropOffset, 0, F4{});
+        }
         for (int i = 0;; i += 2) {
             full_tile(i, uA, dA, bcA, uB, dB, bcB);
             if (i + 1 >= nfull) break;
@@ -375,16 +451,42 @@ __global__ __launch_bounds__(kThreads) void SelectiveScanFwdKernel(SelectiveScan
             if (i + 2 >= nfull) break;
         }
     }
-    for (int t0 = nfull * kTile; t0 < L; t0 += kTile) {   // ragged tail (FAST) or every tile
-        load_guarded(t0, uA, dA, bcA);
-        phase1(t0, false, uA, dA, bcA);
+    for (int t0 = tb + nfull * kTile; t0 < te; t0 += kTile) {   // ragged tail (FAST) or every tile
+        F4 uw[IPT], dw[IPT], bcw[BCPT];
+        load_guarded(t0, uw, dw, bcw);
+        phase1(t0, false, uw, dw, bcw);
         __syncthreads();
         phase2();
         __syncthreads();
         phase3(t0, false);
     }
+    if constexpr (kState) {
+        // the channel's sum of delta' over its kQ4 items, through sDl (last
+        // read before the loop's closing barrier)
+#pragma unroll
+        for (int k = 0; k < IPT; ++k) {
+            const int it = tid + k * kThreads;
+            if (ITEMS % kThreads == 0 || it < ITEMS) sDl[(it / kQ4) * kRow + it % kQ4] = dsum[k];
+        }
+        __syncthreads();
+        if (lane_ok) {
+            float sum = 0.0f;
+#pragma unroll
+            for (int i = 0; i < kQ4; ++i) sum += sDl[lc * kRow + i];
+            for (int s2 = seg + 1; s2 < split.count; ++s2) {
+                float *rec = record(lc, s2, seg);
+                if (lq == 0) rec[0] = sum;
+#pragma unroll
+                for (int j = 0; j < SPL; ++j) {
+                    const int n = lq * SPL + j;
+                    if (n < N) rec[1 + n] = h[j];
+                }
+            }
+        }
+        return;
+    }
     // Scan state after the last token (tokens past the end kept it unchanged).
-    if (p.last_state != nullptr && lane_ok) {
+    if (p.last_state != nullptr && lane_ok && te == L) {
 #pragma unroll
         for (int j = 0; j < SPL; ++j) {
             const int n = lq * SPL + j;
@@ -393,9 +495,25 @@ __global__ __launch_bounds__(kThreads) void SelectiveScanFwdKernel(SelectiveScan
     }
 }
 
+// Lanes per channel and states per lane, with what the forms cost (fp32, one
+// MI355X, interleaved runs of 256 to 4096 tokens at 256 to 20480 channels):
+// the whole pass per token while it has at most one workgroup per CU (ns), the
+// sequence-parallel kernel and the segments per channel and token (ps).
 struct Config {
     int lpc, spl;
+    float whole_ns, seg_ps, split_ps;
 };
+constexpr Config kConfigs[] = {
+    {1, 4, 137.0f, 3.7f, 6.3f},     {2, 4, 105.0f, 5.6f, 5.0f},   {4, 2, 58.0f, 5.6f, 4.6f},
+    {4, 4, 80.0f, 10.0f, 7.5f},     {8, 2, 52.5f, 10.0f, 6.6f},   {16, 1, 45.0f, 10.0f, 9.0f},
+    {8, 4, 81.5f, 18.5f, 11.3f},    {16, 4, 97.0f, 89.0f, 29.0f}, {16, 8, 272.0f, 232.0f, 60.0f},
+    {16, 16, 545.0f, 460.0f, 120.0f},
+};
+Config Layout(int lpc, int spl) {
+    for (const Config &c : kConfigs)
+        if (c.lpc == lpc && c.spl == spl) return c;
+    return kConfigs[0];
+}
 
 // States per lane and lanes per channel by dstate.  The ss_lpc override sets
 // the lanes per channel for dstate <= 16 (1, 2, 4, 8 or 16), for tests and tuning.
@@ -403,73 +521,77 @@ Config ChooseConfig(int N) {
     if (N <= 16) {
         const int forced = static_cast<int>(GetOverride(kOverrideSsLpc));
         switch (forced) {
-            case 4: if (N > 8) return {4, 4}; break;
-            case 8: return {8, 2};
-            case 16: return {16, 1};
-            case 2: if (N <= 8) return {2, 4}; break;
-            case 1: if (N <= 4) return {1, 4}; break;
+            case 4: return N > 8 ? Layout(4, 4) : Layout(4, 2);
+            case 8: return Layout(8, 2);
+            case 16: return Layout(16, 1);
+            case 2: if (N <= 8) return Layout(2, 4); break;
+            case 1: if (N <= 4) return Layout(1, 4); break;
             default: break;
         }
-        if (N <= 4) return {1, 4};
-        if (N <= 8) return {2, 4};
-        return {8, 2};   // measured: 0.445 ms vs 0.454 ms (4 lanes) at 8 x 5120 x 2048 x 16
+        if (N <= 4) return Layout(1, 4);
+        // 8 states: 4 x 2 against 2 x 4 (half the waves, each with twice the
+        // serial work): 8 x 5120 x 2048 0.311 -> 0.256 ms, 4 x 5120 x 2048
+        // 0.214 -> 0.168, 1 x 5120 x 2048 (whole pass) 0.207 -> 0.119
+        if (N <= 8) return Layout(4, 2);
+        return Layout(8, 2);   // measured: 0.445 ms vs 0.454 ms (4 lanes) at 8 x 5120 x 2048 x 16
     }
-    if (N <= 32) return {8, 4};
-    if (N <= 64) return {16, 4};
-    if (N <= 128) return {16, 8};
-    return {16, 16};
+    if (N <= 32) return Layout(8, 4);
+    if (N <= 64) return Layout(16, 4);
+    if (N <= 128) return Layout(16, 8);
+    return Layout(16, 16);
 }
 
 template <typename IT, int LPC, int SPL, bool BVAR, bool CVAR, bool VEC>
-void NoteSs() {
-    XM_NOTE_LAUNCH("SelectiveScanFwdKernel", {TypeTag<IT>()}, LPC, SPL, BVAR, CVAR, VEC);
+void LaunchOne(const SelectiveScanParams &p, const SegSplit &split, unsigned blocks, hipStream_t stream) {
+    if (!(BVAR && CVAR) || split.count <= 1) {   // the split is built for variable B and C
+        XM_NOTE_LAUNCH("SelectiveScanFwdKernel", {TypeTag<IT>()}, LPC, SPL, BVAR, CVAR, VEC, kWhole);
+        hipLaunchKernelGGL((SelectiveScanFwdKernel<IT, LPC, SPL, BVAR, CVAR, VEC, kWhole>), dim3(blocks), dim3(kThreads), 0,
+                           stream, p, split);
+        return;
+    }
+    if constexpr (BVAR && CVAR) {
+        XM_NOTE_LAUNCH("SelectiveScanFwdKernel", {TypeTag<IT>()}, LPC, SPL, BVAR, CVAR, VEC, kSegState);
+        hipLaunchKernelGGL((SelectiveScanFwdKernel<IT, LPC, SPL, BVAR, CVAR, VEC, kSegState>), dim3(blocks * (split.count - 1)),
+                           dim3(kThreads), 0, stream, p, split);
+        XM_NOTE_LAUNCH("SelectiveScanFwdKernel", {TypeTag<IT>()}, LPC, SPL, BVAR, CVAR, VEC, kSegOut);
+        hipLaunchKernelGGL((SelectiveScanFwdKernel<IT, LPC, SPL, BVAR, CVAR, VEC, kSegOut>), dim3(blocks * split.count),
+                           dim3(kThreads), 0, stream, p, split);
+    }
 }
 
 template <typename IT, int LPC, int SPL, bool VEC>
-void LaunchLSV(const SelectiveScanParams &p, dim3 grid, hipStream_t stream) {
-    if (p.b_var && p.c_var) NoteSs<IT, LPC, SPL, true, true, VEC>();
-    else if (p.b_var) NoteSs<IT, LPC, SPL, true, false, VEC>();
-    else if (p.c_var) NoteSs<IT, LPC, SPL, false, true, VEC>();
-    else NoteSs<IT, LPC, SPL, false, false, VEC>();
-    if (p.b_var && p.c_var)
-        hipLaunchKernelGGL((SelectiveScanFwdKernel<IT, LPC, SPL, true, true, VEC>), grid, dim3(kThreads), 0, stream, p);
-    else if (p.b_var)
-        hipLaunchKernelGGL((SelectiveScanFwdKernel<IT, LPC, SPL, true, false, VEC>), grid, dim3(kThreads), 0, stream, p);
-    else if (p.c_var)
-        hipLaunchKernelGGL((SelectiveScanFwdKernel<IT, LPC, SPL, false, true, VEC>), grid, dim3(kThreads), 0, stream, p);
-    else
-        hipLaunchKernelGGL((SelectiveScanFwdKernel<IT, LPC, SPL, false, false, VEC>), grid, dim3(kThreads), 0, stream, p);
+void LaunchLSV(const SelectiveScanParams &p, const SegSplit &split, unsigned blocks, hipStream_t stream) {
+    if (p.b_var && p.c_var) LaunchOne<IT, LPC, SPL, true, true, VEC>(p, split, blocks, stream);
+    else if (p.b_var) LaunchOne<IT, LPC, SPL, true, false, VEC>(p, split, blocks, stream);
+    else if (p.c_var) LaunchOne<IT, LPC, SPL, false, true, VEC>(p, split, blocks, stream);
+    else LaunchOne<IT, LPC, SPL, false, false, VEC>(p, split, blocks, stream);
 }
 
 template <typename IT, int LPC, int SPL>
-void LaunchLS(const SelectiveScanParams &p, int vec, dim3 grid, hipStream_t stream) {
+void LaunchLS(const SelectiveScanParams &p, int vec, const SegSplit &split, unsigned blocks, hipStream_t stream) {
     constexpr int CPW = kThreads / LPC;
     // the fast path's row descriptors span a workgroup's CPW rows: under 2 GiB
     const bool rows_fit = static_cast<long long>(CPW) * p.seqlen * static_cast<long long>(sizeof(IT)) < (1LL << 31);
-    if (vec && rows_fit && p.dim_per_group % CPW == 0) LaunchLSV<IT, LPC, SPL, true>(p, grid, stream);
-    else LaunchLSV<IT, LPC, SPL, false>(p, grid, stream);
-}
-
-// vector accesses are 4 elements: 16 bytes of fp32, 8 of 16-bit data
-bool AlignedVec(const void *ptr, int elem_bytes) {
-    return (reinterpret_cast<uintptr_t>(ptr) & static_cast<uintptr_t>(4 * elem_bytes - 1)) == 0;
+    if (vec && rows_fit && p.dim_per_group % CPW == 0) LaunchLSV<IT, LPC, SPL, true>(p, split, blocks, stream);
+    else LaunchLSV<IT, LPC, SPL, false>(p, split, blocks, stream);
 }
 
 template <typename IT>
-void LaunchTyped(const SelectiveScanParams &p, const Config &cfg, dim3 grid, hipStream_t stream) {
-    const int eb = static_cast<int>(sizeof(IT));
-    const int vec = (p.seqlen % 4 == 0) && AlignedVec(p.u, eb) && AlignedVec(p.delta, eb) && AlignedVec(p.out, eb) &&
-                    (!p.b_var || AlignedVec(p.B, eb)) && (!p.c_var || AlignedVec(p.C, eb));
+void LaunchTyped(const SelectiveScanParams &p, const Config &cfg, const SegSplit &split, unsigned blocks, hipStream_t stream) {
+    const size_t row = static_cast<size_t>(p.seqlen) * sizeof(IT);
+    const int vec = DwordRows(p.u, row) && DwordRows(p.delta, row) && DwordRows(p.out, row) &&
+                    (!p.b_var || DwordRows(p.B, row)) && (!p.c_var || DwordRows(p.C, row));
     switch (cfg.lpc * 100 + cfg.spl) {
-        case 104: LaunchLS<IT, 1, 4>(p, vec, grid, stream); break;
-        case 204: LaunchLS<IT, 2, 4>(p, vec, grid, stream); break;
-        case 404: LaunchLS<IT, 4, 4>(p, vec, grid, stream); break;
-        case 802: LaunchLS<IT, 8, 2>(p, vec, grid, stream); break;
-        case 1601: LaunchLS<IT, 16, 1>(p, vec, grid, stream); break;
-        case 804: LaunchLS<IT, 8, 4>(p, vec, grid, stream); break;
-        case 1604: LaunchLS<IT, 16, 4>(p, vec, grid, stream); break;
-        case 1608: LaunchLS<IT, 16, 8>(p, vec, grid, stream); break;
-        default: LaunchLS<IT, 16, 16>(p, vec, grid, stream); break;
+        case 104: LaunchLS<IT, 1, 4>(p, vec, split, blocks, stream); break;
+        case 204: LaunchLS<IT, 2, 4>(p, vec, split, blocks, stream); break;
+        case 402: LaunchLS<IT, 4, 2>(p, vec, split, blocks, stream); break;
+        case 404: LaunchLS<IT, 4, 4>(p, vec, split, blocks, stream); break;
+        case 802: LaunchLS<IT, 8, 2>(p, vec, split, blocks, stream); break;
+        case 1601: LaunchLS<IT, 16, 1>(p, vec, split, blocks, stream); break;
+        case 804: LaunchLS<IT, 8, 4>(p, vec, split, blocks, stream); break;
+        case 1604: LaunchLS<IT, 16, 4>(p, vec, split, blocks, stream); break;
+        case 1608: LaunchLS<IT, 16, 8>(p, vec, split, blocks, stream); break;
+        default: LaunchLS<IT, 16, 16>(p, vec, split, blocks, stream); break;
     }
 }
 
@@ -496,6 +618,75 @@ void LaunchSkip(const SelectiveScanParams &p, hipStream_t stream) {
     hipLaunchKernelGGL(SelectiveScanSkipKernel<IT>, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, p);
 }
 
+// True when the output shares no byte with an input, so that its rows can hold
+// the sequence split's records while the inputs are still read.
+bool OutputApart(const SelectiveScanParams &p) {
+    const size_t eb = p.in_type == XM_ELEM_FLOAT ? 4 : 2;
+    const size_t rows = static_cast<size_t>(p.batch) * p.dim * p.seqlen;
+    const size_t bc = static_cast<size_t>(p.batch) * p.dstate * p.seqlen, w = static_cast<size_t>(p.dim) * p.dstate;
+    const uintptr_t o = reinterpret_cast<uintptr_t>(p.out);
+    auto apart = [&](const void *x, size_t bytes) {
+        const uintptr_t a = reinterpret_cast<uintptr_t>(x);
+        return x == nullptr || a + bytes <= o || o + rows * eb <= a;
+    };
+    return apart(p.u, rows * eb) && apart(p.delta, rows * eb) && apart(p.A, w * 4) &&
+           apart(p.B, p.b_var ? bc * p.groups_b * eb : w * 4) && apart(p.C, p.c_var ? bc * p.groups_c * eb : w * 4) &&
+           apart(p.D, static_cast<size_t>(p.dim) * 4) && apart(p.delta_bias, static_cast<size_t>(p.dim) * 4) &&
+           apart(p.last_state, static_cast<size_t>(p.batch) * w * 4);
+}
+
+// At most `most` segments whose rows can hold the records; count 1 if none.
+SegSplit FitSegments(const SelectiveScanParams &p, long long most, int min_len) {
+    const long long eb = p.in_type == XM_ELEM_FLOAT ? 4 : 2;
+    for (long long c = std::min<long long>(most, kSplitMax); c >= 2; --c) {
+        const int len = static_cast<int>((p.seqlen + c - 1) / c + 31) / 32 * 32;   // a multiple of the tile (16 or 32)
+        const int n = (p.seqlen + len - 1) / len;
+        const long long last = p.seqlen - static_cast<long long>(n - 1) * len;
+        // the records of n - 1 segments, and the step to a 4-byte boundary, in the shortest segment's rows
+        if (n >= 2 && len >= min_len && 4 + 4LL * (n - 1) * (p.dstate + 1) <= last * eb) return {n, len};
+    }
+    return {1, p.seqlen};
+}
+
+struct SsPlan {
+    bool seq_parallel;   // SelectiveScanSegKernel
+    SegSplit split;
+};
+
+// The form of a call: the whole pass (one chain of seqlen steps per channel
+// block), the sequence-parallel kernel (one workgroup per channel, 1.3 to 1.8
+// times the arithmetic), or segments of the whole pass (1.6 times, two
+// launches).  With fewer blocks than CUs the whole pass takes its chain's
+// time whatever the channels, the other two grow with the channels; the
+// cheapest by the layout's measured costs runs.  Measured us, whole /
+// sequence-parallel / segments: 1 x 5120 x 1999 107 / 114 / 78, 1 x 2048 x
+// 4096 209 / 88 / 72, 1 x 1024 x 2047 107 / 29 / 33, 1 x 7168 x 512 29 / 44 /
+// 33; 64 states, 1 x 2048 x 2048 199 / 375 / 134.  Above one block per CU a
+// CU steps two (1.4 times the chain); there only 16-bit data gains from
+// segments (their reads are half the bytes): 5 x 2048 x 1024 76 -> 69.
+// ss_split override: 1 the whole pass, 2 the sequence-parallel kernel, 3
+// segments wherever the rows hold their records.
+SsPlan ChoosePlan(const SelectiveScanParams &p, const Config &cfg, long long blocks, int64_t forced) {
+    const SegSplit whole{1, p.seqlen};
+    const bool seg_fits = SelectiveScanSegFits(p), splits = p.b_var && p.c_var && OutputApart(p);
+    if (forced == 1) return {false, whole};
+    if (forced == 2) return {seg_fits, whole};
+    if (forced == 3) return {false, splits ? FitSegments(p, kSplitMax, 32) : whole};
+    if (blocks > kSplitMaxChannelBlocks || p.seqlen < kSegMinSeqlen) return {false, whole};
+    const SegSplit split = splits ? FitSegments(p, kSplitTarget / blocks, kSplitMinLen) : whole;
+    const float ct = static_cast<float>(p.batch) * static_cast<float>(p.dim) * 1e-6f;   // us per ps and token
+    const float chain = cfg.whole_ns * 1e-3f;
+    const float t_whole = chain * p.seqlen * (blocks > kSegMaxChannelBlocks ? 1.4f : 1.0f);
+    // the sequence-parallel kernel walks blocks of 512 tokens (1024 to 4 states, 256 above 16)
+    const int walk = p.dstate <= 4 ? 1024 : (p.dstate <= 16 ? 512 : 256);
+    const float t_seg = 3.0f + cfg.seg_ps * ct * (static_cast<float>((p.seqlen + walk - 1) / walk) * walk);
+    const float t_split = 12.0f + std::max(cfg.split_ps * (p.in_type == XM_ELEM_FLOAT ? 1.0f : 0.85f) * ct * p.seqlen,
+                                           1.8f * chain * split.len);
+    const bool seg_ok = seg_fits && blocks < kSegMaxChannelBlocks;
+    if (split.count > 1 && t_split < t_whole && (!seg_ok || t_split < t_seg)) return {false, split};
+    return {seg_ok && t_seg < t_whole, whole};
+}
+
 }  // namespace
 
 void LaunchSelectiveScan(const SelectiveScanParams &p, void *stream_v) {
@@ -511,20 +702,17 @@ void LaunchSelectiveScan(const SelectiveScanParams &p, void *stream_v) {
     const int cpw = kThreads / cfg.lpc;
     const long long ncb = (p.dim_per_group + cpw - 1) / cpw;
     const long long blocks = ncb * p.groups_b * static_cast<long long>(p.batch);
-    // Fewer channel blocks than CUs and a sequence long enough to split: scan
-    // segments of the sequence in parallel, one workgroup per channel
-    // (ss_split override: 1 keeps the channel blocks, 2 always splits).
-    const int64_t split = GetOverride(kOverrideSsSplit);
-    if (SelectiveScanSegFits(p) &&
-        (split == 2 || (split == 0 && blocks < kSegMaxChannelBlocks && p.seqlen >= kSegMinSeqlen))) {
+    const SsPlan plan = ChoosePlan(p, cfg, blocks, GetOverride(kOverrideSsSplit));
+    if (plan.seq_parallel) {
         LaunchSelectiveScanSeg(p, stream);
         return;
     }
-    if (blocks > 2147483647LL) throw Error(XM_ERR_INVALID_ARGUMENT, "SelectiveScanFn launch exceeds the grid limit");
-    const dim3 grid(static_cast<unsigned>(blocks));
-    if (p.in_type == XM_ELEM_FLOAT16) LaunchTyped<_Float16>(p, cfg, grid, stream);
-    else if (p.in_type == XM_ELEM_BFLOAT16) LaunchTyped<Bf16>(p, cfg, grid, stream);
-    else LaunchTyped<float>(p, cfg, grid, stream);
+    const SegSplit &seg = plan.split;
+    if (blocks * seg.count > 2147483647LL) throw Error(XM_ERR_INVALID_ARGUMENT, "SelectiveScanFn launch exceeds the grid limit");
+    const unsigned nblocks = static_cast<unsigned>(blocks);
+    if (p.in_type == XM_ELEM_FLOAT16) LaunchTyped<_Float16>(p, cfg, seg, nblocks, stream);
+    else if (p.in_type == XM_ELEM_BFLOAT16) LaunchTyped<Bf16>(p, cfg, seg, nblocks, stream);
+    else LaunchTyped<float>(p, cfg, seg, nblocks, stream);
     XM_LAUNCH_CHECK("SelectiveScanFn");
 }
 

@@ -57,6 +57,10 @@ struct Bf16 {
     uint16_t bits;
 };
 typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+// four elements of a row that is only dword-aligned
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef _Float16 h4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef unsigned u2u __attribute__((ext_vector_type(2), aligned(4)));
 
 __device__ __forceinline__ float ToF(float x) { return x; }
 __device__ __forceinline__ float ToF(_Float16 x) { return static_cast<float>(x); }
@@ -68,11 +72,16 @@ template <>
 __device__ __forceinline__ float FromF<float>(float x) { return x; }
 template <>
 __device__ __forceinline__ _Float16 FromF<_Float16>(float x) { return static_cast<_Float16>(x); }   // nearest even
+// Two bfloat16 values, nearest even, a NaN staying a (quiet) NaN: the bits of
+// a in the low half (one v_cvt_pk_bf16_f32).
+typedef float f2v __attribute__((ext_vector_type(2)));
+typedef __bf16 b2v __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ unsigned PackBf16(float a, float b) {
+    return __builtin_bit_cast(unsigned, __builtin_convertvector(f2v{a, b}, b2v));
+}
 template <>
-__device__ __forceinline__ Bf16 FromF<Bf16>(float x) {   // nearest even; a NaN stays a (quiet) NaN
-    const uint32_t u = __float_as_uint(x);
-    if ((u & 0x7fffffffu) > 0x7f800000u) return Bf16{static_cast<uint16_t>((u >> 16) | 0x40u)};
-    return Bf16{static_cast<uint16_t>((u + 0x7fffu + ((u >> 16) & 1u)) >> 16)};
+__device__ __forceinline__ Bf16 FromF<Bf16>(float x) {
+    return Bf16{static_cast<uint16_t>(PackBf16(x, x))};
 }
 
 // Four consecutive tokens t..t+3 of a row.  The guarded form clamps every
@@ -80,20 +89,30 @@ __device__ __forceinline__ Bf16 FromF<Bf16>(float x) {   // nearest even; a NaN 
 // has no branches (branches around loads make the compiler wait on each one,
 // which would serialise the one-tile-ahead prefetch).
 // (16 bytes of fp32 or 8 bytes of 16-bit data per vector access)
+// Raw4: four elements as loaded.  Widening 16-bit data at the load would make
+// a prefetch wait for it on the spot; it is widened where it is used.
+template <typename IT>
+using Raw4 = std::conditional_t<sizeof(IT) == 4, f4u, u2u>;
+template <typename IT>
+__device__ __forceinline__ F4 Widen4(Raw4<IT> x) {
+    if constexpr (sizeof(IT) == 4) {
+        return F4{{x[0], x[1], x[2], x[3]}};
+    } else if constexpr (std::is_same_v<IT, _Float16>) {
+        const h4 y = __builtin_bit_cast(h4, x);
+        return F4{{static_cast<float>(y[0]), static_cast<float>(y[1]), static_cast<float>(y[2]),
+                   static_cast<float>(y[3])}};
+    } else {
+        return F4{{__uint_as_float(x[0] << 16), __uint_as_float(x[0] & 0xffff0000u), __uint_as_float(x[1] << 16),
+                   __uint_as_float(x[1] & 0xffff0000u)}};
+    }
+}
+template <typename IT>
+__device__ __forceinline__ Raw4<IT> LoadRaw4(const IT *row, int t) {
+    return *reinterpret_cast<const Raw4<IT> *>(row + t);
+}
 template <typename IT>
 __device__ __forceinline__ F4 LoadRow4Fast(const IT *row, int t) {
-    if constexpr (sizeof(IT) == 4) {
-        const float4 x = *reinterpret_cast<const float4 *>(row + t);
-        return F4{{x.x, x.y, x.z, x.w}};
-    } else if constexpr (std::is_same_v<IT, _Float16>) {
-        const h4 x = *reinterpret_cast<const h4 *>(row + t);
-        return F4{{static_cast<float>(x[0]), static_cast<float>(x[1]), static_cast<float>(x[2]),
-                   static_cast<float>(x[3])}};
-    } else {
-        const uint2 x = *reinterpret_cast<const uint2 *>(row + t);
-        return F4{{__uint_as_float(x.x << 16), __uint_as_float(x.x & 0xffff0000u), __uint_as_float(x.y << 16),
-                   __uint_as_float(x.y & 0xffff0000u)}};
-    }
+    return Widen4<IT>(LoadRaw4(row, t));
 }
 
 template <typename IT>
@@ -108,8 +127,8 @@ __device__ __forceinline__ F4 LoadRow4Guarded(const IT *row, int t, int L, bool 
 }
 
 // Four elements at byte offset voff + soff of a raw buffer (a wave-uniform
-// descriptor, a per-lane offset and a wave-uniform one), converted to fp32 /
-// from fp32 (nearest even).  The offsets are in range by construction.
+// descriptor, a per-lane offset and a wave-uniform one), loaded as they are,
+// stored from fp32 (nearest even).  The offsets are in range by construction.
 typedef __amdgpu_buffer_rsrc_t SsRsrc;
 // A per-lane offset beyond any descriptor size used here: a store there is
 // dropped (the bounds check of a raw buffer).
@@ -120,19 +139,9 @@ __device__ __forceinline__ SsRsrc SsRowsRsrc(const void *base, int bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), static_cast<short>(0), bytes, 0x00020000);
 }
 template <typename IT>
-__device__ __forceinline__ F4 SsBufLoad4(SsRsrc r, int voff, int soff) {
-    if constexpr (sizeof(IT) == 4) {
-        const uint4 x = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
-        return F4{{__uint_as_float(x.x), __uint_as_float(x.y), __uint_as_float(x.z), __uint_as_float(x.w)}};
-    } else if constexpr (std::is_same_v<IT, _Float16>) {
-        const h4 x = __builtin_bit_cast(h4, __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0));
-        return F4{{static_cast<float>(x[0]), static_cast<float>(x[1]), static_cast<float>(x[2]),
-                   static_cast<float>(x[3])}};
-    } else {
-        const uint2 x = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0));
-        return F4{{__uint_as_float(x.x << 16), __uint_as_float(x.x & 0xffff0000u), __uint_as_float(x.y << 16),
-                   __uint_as_float(x.y & 0xffff0000u)}};
-    }
+__device__ __forceinline__ Raw4<IT> SsBufLoad4(SsRsrc r, int voff, int soff) {
+    if constexpr (sizeof(IT) == 4) return __builtin_bit_cast(Raw4<IT>, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
+    else return __builtin_bit_cast(Raw4<IT>, __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0));
 }
 template <typename IT>
 __device__ __forceinline__ void SsBufStore4(SsRsrc r, int voff, int soff, const F4 &x) {
@@ -145,26 +154,21 @@ __device__ __forceinline__ void SsBufStore4(SsRsrc r, int voff, int soff, const 
         for (int e = 0; e < 4; ++e) y[e] = FromF<_Float16>(x.v[e]);
         __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(SsU2, y), r, voff, soff, 0);
     } else {
-        const unsigned lo = static_cast<uint32_t>(FromF<Bf16>(x.v[0]).bits) | (static_cast<uint32_t>(FromF<Bf16>(x.v[1]).bits) << 16);
-        const unsigned hi = static_cast<uint32_t>(FromF<Bf16>(x.v[2]).bits) | (static_cast<uint32_t>(FromF<Bf16>(x.v[3]).bits) << 16);
-        __builtin_amdgcn_raw_buffer_store_b64(SsU2{lo, hi}, r, voff, soff, 0);
+        __builtin_amdgcn_raw_buffer_store_b64(SsU2{PackBf16(x.v[0], x.v[1]), PackBf16(x.v[2], x.v[3])}, r, voff, soff, 0);
     }
 }
 
 template <typename IT>
 __device__ __forceinline__ void StoreRow4Fast(IT *row, int t, const F4 &x) {
     if constexpr (sizeof(IT) == 4) {
-        *reinterpret_cast<float4 *>(row + t) = make_float4(x.v[0], x.v[1], x.v[2], x.v[3]);
+        *reinterpret_cast<f4u *>(row + t) = f4u{x.v[0], x.v[1], x.v[2], x.v[3]};
     } else if constexpr (std::is_same_v<IT, _Float16>) {
-        h4 y;
+        h4u y;
 #pragma unroll
         for (int e = 0; e < 4; ++e) y[e] = FromF<_Float16>(x.v[e]);
-        *reinterpret_cast<h4 *>(row + t) = y;
+        *reinterpret_cast<h4u *>(row + t) = y;
     } else {
-        uint2 y;
-        y.x = static_cast<uint32_t>(FromF<Bf16>(x.v[0]).bits) | (static_cast<uint32_t>(FromF<Bf16>(x.v[1]).bits) << 16);
-        y.y = static_cast<uint32_t>(FromF<Bf16>(x.v[2]).bits) | (static_cast<uint32_t>(FromF<Bf16>(x.v[3]).bits) << 16);
-        *reinterpret_cast<uint2 *>(row + t) = y;
+        *reinterpret_cast<u2u *>(row + t) = u2u{PackBf16(x.v[0], x.v[1]), PackBf16(x.v[2], x.v[3])};
     }
 }
 
@@ -197,6 +201,11 @@ __device__ __forceinline__ float Softplus(float x) {
     return fmaxf(x, 0.0f) + fmaf(__builtin_amdgcn_logf(u), kLn2, -c);
 }
 
+// Rows of row_bytes from ptr on 4-byte boundaries: four-element accesses (16
+// bytes of fp32, 8 of 16-bit data) need no more than dword alignment on gfx950.
+inline bool DwordRows(const void *ptr, size_t row_bytes) {
+    return (reinterpret_cast<uintptr_t>(ptr) & 3) == 0 && row_bytes % 4 == 0;
+}
 
 template <typename IT>
 constexpr const char *TypeTag() {

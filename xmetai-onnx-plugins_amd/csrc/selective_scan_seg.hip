@@ -120,13 +120,16 @@ __device__ __forceinline__ Rsrc RowsRsrc(const void *base, int bytes) {
 }
 
 // Tokens t..t+3 of the B/C row that starts at element `roff` (-1: a padded
-// state), zeros past the sequence end.  VEC: seqlen % 4 == 0 and aligned
-// rows, so a group is entirely inside or outside the sequence.
-template <typename IT, bool VEC>
+// state), zeros past the sequence end.  VEC: rows on 4-byte boundaries, one
+// load for the four; VEC = 1: seqlen % 4 == 0, so a group is entirely inside
+// or outside the sequence; VEC = 2: any seqlen, the tokens of the last group
+// that belong to the next row are replaced by zeros (an infinite or NaN value
+// there must not reach the state through its zero input).
+template <typename IT, int VEC>
 __device__ __forceinline__ F4 BufRow4(Rsrc r, int roff, int t, int L) {
     constexpr int EB = static_cast<int>(sizeof(IT));
     F4 o;
-    if constexpr (VEC) {
+    if constexpr (VEC != 0) {
         const int off = (roff >= 0 && t < L) ? (roff + t) * EB : kOutOfRange;
         if constexpr (EB == 4) {
             const v4f x = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
@@ -141,6 +144,10 @@ __device__ __forceinline__ F4 BufRow4(Rsrc r, int roff, int t, int L) {
                 o = F4{{__uint_as_float(x.x << 16), __uint_as_float(x.x & 0xffff0000u), __uint_as_float(x.y << 16),
                         __uint_as_float(x.y & 0xffff0000u)}};
             }
+        }
+        if constexpr (VEC == 2) {
+#pragma unroll
+            for (int e = 1; e < 4; ++e) o.v[e] = t + e < L ? o.v[e] : 0.0f;
         }
     } else {
 #pragma unroll
@@ -158,7 +165,7 @@ __device__ __forceinline__ F4 BufRow4(Rsrc r, int roff, int t, int L) {
     return o;
 }
 
-template <typename IT, int LPC, int SPL, bool BVAR, bool CVAR, bool VEC>
+template <typename IT, int LPC, int SPL, bool BVAR, bool CVAR, int VEC>
 __global__ __launch_bounds__(64 * kSegWaves) void SelectiveScanSegKernel(SelectiveScanParams p) {
     constexpr int NT = 64 * kSegWaves;
     constexpr int SW = 64 / LPC;             // segments per wave
@@ -234,11 +241,11 @@ __global__ __launch_bounds__(64 * kSegWaves) void SelectiveScanSegKernel(Selecti
                     const float4 yv = *reinterpret_cast<const float4 *>(&sY[li]);
                     const float4 kv = *reinterpret_cast<const float4 *>(&sSk[li]);
                     const F4 o{{kv.x + yv.x, kv.y + yv.y, kv.z + yv.z, kv.w + yv.w}};
-                    if constexpr (VEC) StoreRow4Fast(orow, t - LB, o);
+                    if constexpr (VEC != 0) StoreRow4Fast(orow, t - LB, o);
                     else StoreRow4(orow, t - LB, L, false, o);
                 }
                 F4 uu, dd;
-                if (VEC && t + 3 < L) {
+                if (VEC != 0 && t + 3 < L) {
                     uu = LoadRow4Fast(urow, t);
                     dd = LoadRow4Fast(drow, t);
                 } else {
@@ -399,7 +406,7 @@ __global__ __launch_bounds__(64 * kSegWaves) void SelectiveScanSegKernel(Selecti
                 const float4 yv = *reinterpret_cast<const float4 *>(&sY[li]);
                 const float4 kv = *reinterpret_cast<const float4 *>(&sSk[li]);
                 const F4 o{{kv.x + yv.x, kv.y + yv.y, kv.z + yv.z, kv.w + yv.w}};
-                StoreRow4(orow, t, L, VEC, o);
+                StoreRow4(orow, t, L, VEC != 0, o);
             }
         }
     }
@@ -429,14 +436,14 @@ SegConfig ChooseSegConfig(int N) {
     return {16, 16};
 }
 
-template <typename IT, int LPC, int SPL, bool BVAR, bool CVAR, bool VEC>
+template <typename IT, int LPC, int SPL, bool BVAR, bool CVAR, int VEC>
 void LaunchSeg(const SelectiveScanParams &p, dim3 grid, hipStream_t stream) {
     XM_NOTE_LAUNCH("SelectiveScanSegKernel", {TypeTag<IT>()}, LPC, SPL, BVAR, CVAR, VEC);
     hipLaunchKernelGGL((SelectiveScanSegKernel<IT, LPC, SPL, BVAR, CVAR, VEC>), grid, dim3(64 * kSegWaves), 0, stream,
                        p);
 }
 
-template <typename IT, int LPC, int SPL, bool VEC>
+template <typename IT, int LPC, int SPL, int VEC>
 void LaunchSegLSV(const SelectiveScanParams &p, dim3 grid, hipStream_t stream) {
     if (p.b_var && p.c_var) LaunchSeg<IT, LPC, SPL, true, true, VEC>(p, grid, stream);
     else if (p.b_var) LaunchSeg<IT, LPC, SPL, true, false, VEC>(p, grid, stream);
@@ -445,20 +452,20 @@ void LaunchSegLSV(const SelectiveScanParams &p, dim3 grid, hipStream_t stream) {
 }
 
 template <typename IT, int LPC, int SPL>
-void LaunchSegLS(const SelectiveScanParams &p, bool vec, dim3 grid, hipStream_t stream) {
-    if (vec) LaunchSegLSV<IT, LPC, SPL, true>(p, grid, stream);
-    else LaunchSegLSV<IT, LPC, SPL, false>(p, grid, stream);
-}
-
-bool Aligned4(const void *ptr, int elem_bytes) {
-    return (reinterpret_cast<uintptr_t>(ptr) & static_cast<uintptr_t>(4 * elem_bytes - 1)) == 0;
+void LaunchSegLS(const SelectiveScanParams &p, int vec, dim3 grid, hipStream_t stream) {
+    if (vec == 1) LaunchSegLSV<IT, LPC, SPL, 1>(p, grid, stream);
+    else if (vec == 2) LaunchSegLSV<IT, LPC, SPL, 2>(p, grid, stream);
+    else if constexpr (sizeof(IT) == 2) LaunchSegLSV<IT, LPC, SPL, 0>(p, grid, stream);   // fp32 rows are dword rows
 }
 
 template <typename IT>
 void LaunchSegTyped(const SelectiveScanParams &p, dim3 grid, hipStream_t stream) {
-    const int eb = static_cast<int>(sizeof(IT));
-    const bool vec = (p.seqlen % 4 == 0) && Aligned4(p.u, eb) && Aligned4(p.delta, eb) && Aligned4(p.out, eb) &&
-                     (!p.b_var || Aligned4(p.B, eb)) && (!p.c_var || Aligned4(p.C, eb));
+    // one load per four tokens needs rows on 4-byte boundaries: always so for
+    // fp32, and for 16-bit data of even length at even offsets
+    const size_t row = static_cast<size_t>(p.seqlen) * sizeof(IT);
+    const bool dwords = DwordRows(p.u, row) && DwordRows(p.delta, row) && DwordRows(p.out, row) &&
+                        (!p.b_var || DwordRows(p.B, row)) && (!p.c_var || DwordRows(p.C, row));
+    const int vec = sizeof(IT) == 2 && !dwords ? 0 : (p.seqlen % 4 == 0 ? 1 : 2);
     const SegConfig cfg = ChooseSegConfig(p.dstate);
     switch (cfg.lpc * 100 + cfg.spl) {
         case 401: LaunchSegLS<IT, 4, 1>(p, vec, grid, stream); break;

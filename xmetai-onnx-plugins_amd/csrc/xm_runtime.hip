@@ -152,7 +152,7 @@ constexpr OverrideSpec kOverrides[kOverrideCount] = {
     {"gdn2_rows", {1, 2, 4, 0}},         // rows of 16 lanes per value column (sequential kernel)
     {"m3_path", {1, 0}},                 // 1: the token-by-token kernel
     {"ss_lpc", {1, 2, 4, 8, 16, 0}},     // lanes per channel (dstate <= 16)
-    {"ss_split", {1, 2, 0}},             // 1: one workgroup per channel block; 2: sequence-split
+    {"ss_split", {1, 2, 3, 0}},          // 1: one workgroup per channel block; 2: sequence-parallel; 3: segments
     {"gdn2_kpw4", {1, 0}},               // 1: GDN-2 chunked, 4 key tiles per wave above 128 keys
     {"gdn2_windowed", {1, 0}},           // 1: GDN-2 chunked, windows of 128 chunks only
     {"gdn2_split", {1, 2, 3, 0}},        // GDN-2 chunked: 1 no sequence split, 2 split wherever 2+ chunks,
