@@ -102,7 +102,8 @@ void xm_selective_scan_attrs_default(xm_selective_scan_attrs_t *attrs);
 int xm_selective_scan_check_attrs(const xm_selective_scan_attrs_t *attrs, char *errbuf, size_t errlen);
 /* Run-time shape validation without touching the device (reference:
  * Compute, :58-117).  Writes the output shape and the scratch bytes the call
- * will request from the allocator. */
+ * will request from the allocator (GatedDeltaNet2Fn: at most; a call of up to
+ * 16 tokens requests none). */
 int xm_selective_scan_validate(const xm_tensor_t *inputs, size_t n_inputs,
                                const xm_selective_scan_attrs_t *attrs, int64_t *out_shape,
                                int32_t *out_rank, size_t *scratch_bytes, char *errbuf, size_t errlen);
@@ -259,7 +260,9 @@ int xm_softmax_cpu(const float *in, const int64_t *shape, int32_t rank, int64_t 
  * Process-wide switches that force a kernel variant the dispatchers would not
  * pick by themselves, so that parity tests can run every variant; value 0
  * restores the dispatcher's own choice.  Production callers never need them.
- *   "gdn2_path"      1: GatedDeltaNet2Fn sequential fused kernel (headdim_k <= 512)
+ *   "gdn2_path"      1: GatedDeltaNet2Fn sequential fused kernel (headdim_k <= 512);
+ *                    2: the chunked path also for the few tokens (up to 16) that
+ *                    the single-launch kernel takes by default
  *   "gdn2_pairwise"  1: every chunk of the chunked GDN-2 path forms A and M pairwise
  *   "gdn2_rows"      1, 2, 4: rows of 16 lanes per value column of the fused kernel
  *   "m3_path"        1: Mamba3SisoFn token-by-token kernel

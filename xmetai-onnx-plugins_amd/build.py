@@ -52,6 +52,7 @@ SOURCES = [
     "selective_scan_seg.hip",
     "gated_deltanet2.hip",
     "gated_deltanet2_chunk.hip",
+    "gated_deltanet2_step.hip",
     "gated_deltanet2_noalloc.hip",
     "mamba3_siso.hip",
     "mamba3_siso_chunk.hip",

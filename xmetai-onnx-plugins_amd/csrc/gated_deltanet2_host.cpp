@@ -105,7 +105,9 @@ void Forward(const xm_tensor_t *inputs, size_t n_inputs, const xm_gated_deltanet
              float *final_state, void *stream, const xm_allocator_t *alloc) {
     const GatedDeltaNet2Params p = GatedDeltaNet2Plan(inputs, n_inputs, attrs, out, final_state);
     const bool packed = p.cu_seqlens != nullptr;
-    size_t bytes = GatedDeltaNet2ScratchBytes(p.batch, p.seqlen, p.nheads, p.dk, p.dv, packed);
+    // a few tokens need no scratch (validation still reports the chunked path's)
+    const bool step = GatedDeltaNet2StepFits(p.batch, p.seqlen, p.nheads, p.dk, p.dv, packed);
+    size_t bytes = step ? 0 : GatedDeltaNet2ScratchBytes(p.batch, p.seqlen, p.nheads, p.dk, p.dv, packed);
     Scratch scratch(alloc, stream);
     void *buf = scratch.TryGet(bytes);
     if (buf == nullptr && bytes > 0) {

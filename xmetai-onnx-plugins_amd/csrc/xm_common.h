@@ -139,12 +139,12 @@ int Guard(char *errbuf, size_t errlen, Fn &&fn) {
 // tuning); 0 everywhere means the dispatchers' own choice.  Read with one
 // relaxed atomic load per launch.
 enum Override {
-    kOverrideGdn2Path,       // 1: GatedDeltaNet2Fn sequential fused kernel
+    kOverrideGdn2Path,       // GatedDeltaNet2Fn: 1 sequential fused kernel, 2 chunked also for a few tokens
     kOverrideGdn2Pairwise,   // 1: pairwise A and M in every chunk
     kOverrideGdn2Rows,       // rows of 16 lanes per value column of the fused kernel
     kOverrideM3Path,         // 1: Mamba3SisoFn token-by-token kernel
     kOverrideSsLpc,          // lanes per channel of the selective scan (dstate <= 16)
-    kOverrideSsSplit,        // selective scan: 1 channel blocks only, 2 sequence-split
+    kOverrideSsSplit,        // selective scan: 1 whole pass, 2 sequence-parallel kernel, 3 segments of the whole pass
     kOverrideGdn2Kpw4,       // 1: GDN-2 chunked recurrence above 128 keys with 4 key tiles per wave, ceil(tiles/4) waves
     kOverrideGdn2Windowed,   // 1: GDN-2 chunked path in windows of 128 chunks (not sized to 128 MiB / one packed window)
     kOverrideGdn2Split,      // GDN-2 chunked path: 1 never split the sequence, 2 split it wherever it has 2+ chunks, 3 two unequal segments (the second two tiles per workgroup)

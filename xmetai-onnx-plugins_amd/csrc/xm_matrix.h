@@ -37,6 +37,10 @@ __device__ __forceinline__ float BufF(Rsrc r, int voff, int soff = 0) {
 __device__ __forceinline__ void BufStF(Rsrc r, int voff, float x, int soff = 0) {
     __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, x), r, voff, soff, 0);
 }
+__device__ __forceinline__ void BufStF4(Rsrc r, int voff, v4f x, int soff = 0) {
+    typedef unsigned u4 __attribute__((ext_vector_type(4)));
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, x), r, voff, soff, 0);
+}
 // Orders this wave's LDS accesses before and after (the LDS unit serves one
 // wave's operations in order; this stops the compiler from moving them), so
 // a wave can read back what its other lanes just wrote.

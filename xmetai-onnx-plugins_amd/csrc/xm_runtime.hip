@@ -147,7 +147,7 @@ struct OverrideSpec {
 };
 // Index order of the Override enum.
 constexpr OverrideSpec kOverrides[kOverrideCount] = {
-    {"gdn2_path", {1, 0}},               // 1: the sequential fused kernel
+    {"gdn2_path", {1, 2, 0}},            // 1: the sequential fused kernel; 2: chunked also for a few tokens
     {"gdn2_pairwise", {1, 0}},           // 1: pairwise A and M in every chunk
     {"gdn2_rows", {1, 2, 4, 0}},         // rows of 16 lanes per value column (sequential kernel)
     {"m3_path", {1, 0}},                 // 1: the token-by-token kernel
