@@ -265,7 +265,9 @@ int xm_softmax_cpu(const float *in, const int64_t *shape, int32_t rank, int64_t 
  *                    the single-launch kernel takes by default
  *   "gdn2_pairwise"  1: every chunk of the chunked GDN-2 path forms A and M pairwise
  *   "gdn2_rows"      1, 2, 4: rows of 16 lanes per value column of the fused kernel
- *   "m3_path"        1: Mamba3SisoFn token-by-token kernel
+ *   "m3_path"        1: Mamba3SisoFn token-by-token kernel; 2: the chunked kernel
+ *                    also for the few tokens (up to 16) that the single-launch
+ *                    kernel takes by default
  *   "ss_lpc"         1, 2, 4, 8, 16: SelectiveScanFn lanes per channel (d_state <= 16)
  *   "ss_split"       1: SelectiveScanFn channel-block kernel over the whole
  *                    sequence only; 2: the sequence-parallel kernel wherever it

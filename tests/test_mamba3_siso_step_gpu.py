@@ -1,0 +1,95 @@
+"""Mamba3SisoFn for a few tokens (Mamba3StepKernel: the state through registers
+in one launch) on the GPU vs the fp64 oracle: key counts at the edges of the
+64-key groups and of a four-key group, state rows cut by a row block, the three
+row-block heights, one to sixteen tokens (prepared four at a time), angles of
+some pairs, Q/K heads shared, with and without Z, D, input and final states,
+and agreement with the chunked kernel."""
+
+import numpy as np
+import pytest
+
+import xmetai_onnx_plugins as xp
+from oracle import cref
+from parity import TOL_GPU, TOL_M3, check, to_dev
+from xmetai_onnx_plugins import workloads as W
+
+pytestmark = pytest.mark.gpu
+
+KEYS = ("Q", "K", "V", "ADT", "DT", "Trap", "Q_bias", "K_bias", "Angles", "D", "Z")
+STATES = ("ssm", "angle", "k", "v")
+S = W.Mamba3SisoShape
+
+
+def run(s, seed, start=True):
+    inp = W.mamba3_siso_inputs(s, seed=seed)
+    rng = np.random.default_rng(seed + 1000)
+    states = None
+    if start:
+        states = (rng.standard_normal((s.batch, s.nheads, s.headdim, s.dstate)).astype(np.float32),
+                  rng.uniform(0, 2 * np.pi, (s.batch, s.nheads, s.a)).astype(np.float32),
+                  rng.standard_normal((s.batch, s.nheads, s.dstate)).astype(np.float32),
+                  rng.standard_normal((s.batch, s.nheads, s.headdim)).astype(np.float32))
+    y, f = xp.mamba3_siso_fn(*(to_dev(inp[k]) for k in KEYS), return_final_states=True,
+                             input_states=tuple(to_dev(x) for x in states) if start else None)
+    ref_y, ref_f = cref.mamba3_siso(*(inp[k] for k in KEYS), dtype=np.float64, input_states=states, return_state=True)
+    return (y, *f), (ref_y, *ref_f)
+
+
+def compare(name, got, ref, tol):
+    # an angle next to the wrap may come out one period off: compare on the circle
+    for part, g, r in zip(("y", *STATES), got, ref):
+        g = g.cpu().numpy() if hasattr(g, "cpu") else g
+        r = r.cpu().numpy() if hasattr(r, "cpu") else r
+        if part == "angle":
+            period = 2.0 * float(np.float32(np.pi))
+            d = (g.astype(np.float64) - r + period / 2) % period - period / 2
+            g = r + d
+        check(f"mamba3_siso_step/{name}/{part}", g, r, tol)
+
+
+def step_rows():
+    names = xp.last_launches()
+    if len(names) != 1 or not names[0].startswith("Mamba3StepKernel<"):
+        return 0
+    return 16 * int(names[0][:-1].split(",")[1])
+
+
+@pytest.mark.parametrize("n", [2, 6, 62, 64, 66, 128, 130, 190, 192, 194, 254, 256])
+@pytest.mark.parametrize("tokens", [1, 5])
+def test_step_keys(n, tokens):
+    got, ref = run(S(2, tokens, 4, 20, n, nheads_qk=2, has_z=True), seed=n)
+    assert step_rows() == 16, xp.last_launches()
+    compare(f"n{n}_t{tokens}", got, ref, TOL_M3)
+
+
+@pytest.mark.parametrize("p", [1, 15, 16, 17, 31, 33, 63, 64, 65, 100])
+@pytest.mark.parametrize("heads,rows", [(2, 16), (64, 32), (256, 64)])
+def test_step_rows(p, heads, rows):
+    got, ref = run(S(2, 3, heads, p, 32, angles=5), seed=p)
+    assert step_rows() in (rows, 2 * rows), xp.last_launches()   # more 64-row blocks above 64 rows
+    compare(f"p{p}_h{heads}", got, ref, TOL_M3)
+
+
+@pytest.mark.parametrize("tokens", [1, 2, 4, 7, 8])
+@pytest.mark.parametrize("has_z,has_d,start", [(True, True, True), (False, False, True), (True, False, False)])
+def test_step_tokens(tokens, has_z, has_d, start):
+    got, ref = run(S(2, tokens, 3, 64, 128, angles=40, has_z=has_z, has_d=has_d), seed=tokens, start=start)
+    assert step_rows() == 16
+    compare(f"t{tokens}_{has_z}_{has_d}_{start}", got, ref, TOL_M3)
+
+
+@pytest.mark.parametrize("tokens,heads,step", [(9, 128, True), (16, 128, True), (17, 128, False), (9, 4, False)])
+def test_step_token_limits(tokens, heads, step):
+    got, ref = run(S(2, tokens, heads, 24, 64, has_z=True), seed=tokens)
+    assert (step_rows() > 0) == step, xp.last_launches()
+    compare(f"limit_t{tokens}_h{heads}", got, ref, TOL_M3)
+
+
+def test_step_agrees_with_the_chunked_kernel(override):
+    s = S(3, 6, 4, 64, 128, has_z=True)
+    got, _ = run(s, seed=5)
+    assert step_rows() == 16
+    override("m3_path", 2)
+    chunked, _ = run(s, seed=5)
+    assert xp.last_launches() == ["Mamba3ChunkKernel<2,4,8,0>"], xp.last_launches()
+    compare("vs_chunked", got, [x.cpu().numpy() for x in chunked], TOL_GPU)

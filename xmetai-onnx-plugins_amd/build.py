@@ -56,6 +56,7 @@ SOURCES = [
     "gated_deltanet2_noalloc.hip",
     "mamba3_siso.hip",
     "mamba3_siso_chunk.hip",
+    "mamba3_siso_step.hip",
     "selective_scan_host.cpp",
     "gated_deltanet2_host.cpp",
     "mamba3_siso_host.cpp",

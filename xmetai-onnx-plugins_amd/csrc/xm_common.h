@@ -142,7 +142,7 @@ enum Override {
     kOverrideGdn2Path,       // GatedDeltaNet2Fn: 1 sequential fused kernel, 2 chunked also for a few tokens
     kOverrideGdn2Pairwise,   // 1: pairwise A and M in every chunk
     kOverrideGdn2Rows,       // rows of 16 lanes per value column of the fused kernel
-    kOverrideM3Path,         // 1: Mamba3SisoFn token-by-token kernel
+    kOverrideM3Path,         // Mamba3SisoFn: 1 token-by-token kernel, 2 chunked also for a few tokens
     kOverrideSsLpc,          // lanes per channel of the selective scan (dstate <= 16)
     kOverrideSsSplit,        // selective scan: 1 whole pass, 2 sequence-parallel kernel, 3 segments of the whole pass
     kOverrideGdn2Kpw4,       // 1: GDN-2 chunked recurrence above 128 keys with 4 key tiles per wave, ceil(tiles/4) waves

@@ -126,6 +126,11 @@ size_t GatedDeltaNet2ChunkScratchBytes(int batch, int seqlen, int nheads, int dk
 constexpr int kGdn2ChunkKeyLimit = 512;   // head_k handled by the chunked path
 bool LaunchGatedDeltaNet2Chunked(const GatedDeltaNet2Params &p, void *scratch, size_t scratch_bytes, void *stream);
 void LaunchMamba3Siso(const Mamba3SisoParams &p, void *stream);
+// A few tokens (mamba3_siso_step.hip): unpacked, seqlen up to kM3StepTokens,
+// headdim_qk <= 256.  Returns false, launching nothing, when it does not fit
+// (or the m3_path override asks for another path).
+constexpr int kM3StepTokens = 16;
+bool LaunchMamba3SisoStep(const Mamba3SisoParams &p, void *stream);
 // Chunked fp32-MFMA path (headdim_qk <= 256).  Returns false, launching
 // nothing, when the m3_path override asks for the token-by-token kernel.
 bool LaunchMamba3SisoChunked(const Mamba3SisoParams &p, void *stream);

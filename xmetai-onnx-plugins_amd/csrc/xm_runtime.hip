@@ -150,7 +150,7 @@ constexpr OverrideSpec kOverrides[kOverrideCount] = {
     {"gdn2_path", {1, 2, 0}},            // 1: the sequential fused kernel; 2: chunked also for a few tokens
     {"gdn2_pairwise", {1, 0}},           // 1: pairwise A and M in every chunk
     {"gdn2_rows", {1, 2, 4, 0}},         // rows of 16 lanes per value column (sequential kernel)
-    {"m3_path", {1, 0}},                 // 1: the token-by-token kernel
+    {"m3_path", {1, 2, 0}},              // 1: the token-by-token kernel; 2: chunked also for a few tokens
     {"ss_lpc", {1, 2, 4, 8, 16, 0}},     // lanes per channel (dstate <= 16)
     {"ss_split", {1, 2, 3, 0}},          // 1: one workgroup per channel block; 2: sequence-parallel; 3: segments
     {"gdn2_kpw4", {1, 0}},               // 1: GDN-2 chunked, 4 key tiles per wave above 128 keys
