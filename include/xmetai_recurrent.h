@@ -268,6 +268,9 @@ int xm_softmax_cpu(const float *in, const int64_t *shape, int32_t rank, int64_t 
  *   "m3_path"        1: Mamba3SisoFn token-by-token kernel; 2: the chunked kernel
  *                    also for the few tokens (up to 16) that the single-launch
  *                    kernel takes by default
+ *   "m3_split"       1: the chunked Mamba3SisoFn kernel never splits the sequence;
+ *                    2: it splits wherever the output rows hold the segments'
+ *                    records
  *   "ss_lpc"         1, 2, 4, 8, 16: SelectiveScanFn lanes per channel (d_state <= 16)
  *   "ss_split"       1: SelectiveScanFn channel-block kernel over the whole
  *                    sequence only; 2: the sequence-parallel kernel wherever it

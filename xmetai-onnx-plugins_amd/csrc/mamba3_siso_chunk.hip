@@ -53,7 +53,6 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <cstdlib>
 #include <cstring>
 #include <type_traits>
 
@@ -69,6 +68,7 @@ using namespace m3;
 
 constexpr int kC = 16;          // tokens per chunk
 constexpr int kRows = 32;       // state rows per workgroup (two 16-row tiles)
+constexpr int kStateRows = 64; // state rows per workgroup of the sequence split's state launch
 constexpr int kBufs = 3;        // chunk buffers: preparing j+1, products of j, finishing j-1
 // Row stride (floats) of the [key][token] k^T and [row][token] V^T tiles.
 // LDS bank conflicts of the kernel's access patterns, measured per access on
@@ -134,6 +134,11 @@ struct M3CLayout {
     static constexpr int oBig = 0, oSmall = 2 * kBig, oPart = oSmall + kBufs * kSmall;
     static constexpr size_t kBytes = sizeof(float) * (oPart + 2 * kPart);
     static_assert(kBig % 4 == 0 && kSmall % 4 == 0 && QS % 4 == 0 && kTS % 4 == 0, "16-byte aligned tiles");
+    // the sequence split's state launch keeps only k^T of the tiles and no
+    // partial products, and has more state rows
+    static constexpr int kStateBig = NP * kTS;
+    static constexpr int oStateVT = kSmall, kStateSmall = kSmall + kStateRows * kTS;   // its V^T, behind the fields
+    static constexpr size_t kStateBytes = sizeof(float) * (2 * kStateBig + kBufs * kStateSmall);
     static_assert(kBytes <= 160 * 1024, "LDS budget");
     static_assert(PPW % 8 == 0 && PB * PL == PPW && TPL * TG == kC && VPT * 64 * NPW == kRows * kC, "lane mapping");
     static_assert(VPT * NPW == 8 && kRows == 32 && kC == 16, "V^T: 4 row blocks x 2 token blocks of 8 x 8");
@@ -200,20 +205,97 @@ __device__ __forceinline__ float RowInclusiveScan16(float x) {
     return x;
 }
 
+// ---------------------------------------------------------------------------
+// Sequence split, for calls whose (b,h) row blocks are fewer than the CUs: a
+// workgroup walks its sequence's chunks in order, so such a call takes one
+// walk's time on part of the chip.  The decay is a scalar per token, so a
+// segment maps its start state S to D S + E, with D the exponential of its sum
+// of ADT and E its end state from zero.  The angles are sums over the tokens and
+// a rotation by a sum of angles is the product of the rotations, so E is formed
+// with the angles counted from the segment's start and turned by the start
+// angles afterwards.  Three launches:
+//  1. Mamba3ChunkKernel<kM3State>: E, the angle sums (fp64, in turns) and the
+//     sum of ADT of every fine segment that another follows (segment 0 from
+//     the true start state and angles); k^ alone is rotated, no q, no output.
+//  2. Mamba3SegCombineKernel: start states and start angles of the output
+//     segments, in segment order.
+//  3. Mamba3ChunkKernel<kM3Out>: every output segment from its start state.
+// The records live in the output rows of the segment that starts at the same
+// token (columns of the row block: 4 bytes x W), which only launch 3's
+// workgroup of that segment and row block overwrites, after it has read them:
+// no scratch.  A record is the S^T tiles in lane order, the fine segment's
+// angle sums, its sum of ADT, and the start angles.
+// Packed sequences split likewise, each by its own length.
+// ---------------------------------------------------------------------------
+enum M3Mode { kM3Whole, kM3State, kM3Out };
+struct M3Split {
+    int ls, lf;    // tokens per output segment and per fine segment (multiples of kC; ls a multiple of lf)
+    int need;      // tokens a record takes: the last segment has at least these
+    int maxseg;    // output segments of a sequence of seqlen tokens
+    // output segments of a sequence of T tokens
+    __host__ __device__ int Segments(int T) const { return T < ls + need ? 1 : (T - need) / ls + 1; }
+};
+// Tokens a record needs with NP padded keys at 16 or 32 columns.
+constexpr int M3RecordTokens(int np) { return np + np / 8 + 16; }
+// The record of the segment starting at token tok (in [B*T]): float e of the
+// columns r0 .. r0 + W - 1 of head h.
+struct M3Record {
+    float *base;
+    size_t row;   // floats per token row
+    int w;        // columns, 16 or 32
+    int np;       // padded keys
+    __device__ __forceinline__ float *At(int e) const { return base + static_cast<size_t>(e / w) * row + e % w; }
+    __device__ __forceinline__ float *State(int q) const { return At(4 * q); }              // 4 floats, q < np w / 4
+    __device__ __forceinline__ int AngleSum(int a) const { return np * w + 2 * a; }        // two words of a double
+    __device__ __forceinline__ int DecaySum() const { return np * w + np; }
+    __device__ __forceinline__ int StartAngle(int a) const { return np * w + np + 16 + 2 * a; }
+    __device__ __forceinline__ double GetD(int e) const {
+        const unsigned lo = __float_as_uint(*At(e)), hi = __float_as_uint(*At(e + 1));
+        return __longlong_as_double(static_cast<long long>((static_cast<unsigned long long>(hi) << 32) | lo));
+    }
+    __device__ __forceinline__ void PutD(int e, double x) const {
+        const unsigned long long v = static_cast<unsigned long long>(__double_as_longlong(x));
+        *At(e) = __uint_as_float(static_cast<unsigned>(v));
+        *At(e + 1) = __uint_as_float(static_cast<unsigned>(v >> 32));
+    }
+};
+typedef float v4u __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ M3Record RecordAt(const Mamba3SisoParams &p, size_t tok, int h, int r0, int np) {
+    return {p.out + (tok * p.nheads + h) * p.p + r0, static_cast<size_t>(p.nheads) * p.p, min(kRows, p.p - r0), np};
+}
+// A sequence's tokens: first (in [B*T]) and count.
+struct M3Range {
+    size_t tok0;
+    int T;
+};
+__device__ __forceinline__ M3Range RangeOf(const Mamba3SisoParams &p, int b) {
+    if (p.cu_seqlens == nullptr) return {static_cast<size_t>(b) * p.seqlen, p.seqlen};
+    const long long lo = min(max(p.cu_seqlens[b], 0LL), static_cast<long long>(p.seqlen));
+    const long long hi = min(max(p.cu_seqlens[b + 1], lo), static_cast<long long>(p.seqlen));
+    return {static_cast<size_t>(lo), static_cast<int>(hi - lo)};
+}
+
 // LONG: some tensor's token rows of one sequence span 2 GiB or more, beyond a
 // buffer descriptor's 32-bit range; every chunk then reads and writes through
 // descriptors that start at its own first token.
 // HASZ: a Z input (the SiLU gate); without one the finishing waves issue no Z
 // loads and no gate.
-template <int KBW, int NW, int NPW, bool LONG, bool HASZ>
-__global__ __launch_bounds__(64 * (NW + NPW)) void Mamba3ChunkKernel(Mamba3SisoParams p) {
+// MODE: the whole sequence, or a launch of the sequence split (above).
+template <int KBW, int NW, int NPW, bool LONG, bool HASZ, int MODE>
+__global__ __launch_bounds__(64 * (NW + NPW)) void Mamba3ChunkKernel(Mamba3SisoParams p, M3Split split) {
+    constexpr bool kState = MODE == kM3State;
     using L = M3CLayout<KBW, NW, NPW>;
     static_assert(NW == 4, "product waves 0 and 1 finish, 2 and 3 take shared work off them");
     constexpr int NT = L::NT;
-    constexpr int PPW = L::PPW, PL = L::PL, PB = L::PB, TPL = L::TPL, VPT = L::VPT, QS = L::QS;
+    constexpr int PPW = L::PPW, PL = L::PL, PB = L::PB, TPL = L::TPL, QS = L::QS;
+    constexpr int ROWS = kState ? kStateRows : kRows, PT = ROWS / 16;   // state rows, row tiles
+    constexpr int VPT = ROWS * kC / (64 * NPW);                          // V values per preparation thread
+    constexpr int oVT = kState ? L::oStateVT : L::oVT;
+
+    constexpr int oKT = kState ? 0 : L::oKT, kBig = kState ? L::kStateBig : L::kBig, oSmall = 2 * kBig;
 
     extern __shared__ __attribute__((aligned(16))) float smem[];
-    float *part = smem + L::oPart;
+    float *part = smem + (kState ? 0 : L::oPart);   // unused by kState
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -223,30 +305,53 @@ __global__ __launch_bounds__(64 * (NW + NPW)) void Mamba3ChunkKernel(Mamba3SisoP
     const int i16 = lane & 15, g4 = lane >> 4;
     const int N = p.n, P = p.p, A = p.a, H = p.nheads;
     const int half_n = N / 2;
-    const int nrb = (P + kRows - 1) / kRows;
+    const int nrb = (P + ROWS - 1) / ROWS;
     // the nrb workgroups of one (b,h) prepare the same token vectors: keep them on one XCD
     const int wg = XcdLocalBlock(blockIdx.x, gridDim.x);
     const int rb = wg % nrb;
-    const int bh = wg / nrb;
+    const int nseg_wg = MODE == kM3Whole ? 1 : (kState ? (split.maxseg - 1) * (split.ls / split.lf) : split.maxseg);
+    const int seg = MODE == kM3Whole ? 0 : (wg / nrb) % nseg_wg;   // fine segment (kM3State) or output segment
+    const int bh = wg / nrb / nseg_wg;
     const int b = bh / H, h = bh % H;
     const int gq = h / (H / p.nheads_qk);
-    const int r0 = rb * kRows;
+    const int r0 = rb * ROWS;
     const float dval = p.D ? p.D[h] : 0.0f;
-    int T = p.seqlen;
-    size_t tok0 = static_cast<size_t>(b) * T;    // in [B*T] for Q/K/V/Angles/Z
-    size_t sbase = static_cast<size_t>(bh) * T;  // in [B*H*T] for ADT/DT/Trap
+    // (RangeOf's arithmetic, written out: through the struct the whole pass
+    // measured 1 to 2% slower at 64 keys, the same loops scheduled otherwise)
+    int T_ = p.seqlen;
+    size_t tok0_ = static_cast<size_t>(b) * T_;    // in [B*T] for Q/K/V/Angles/Z
+    size_t sbase_ = static_cast<size_t>(bh) * T_;  // in [B*H*T] for ADT/DT/Trap
     if (p.cu_seqlens != nullptr) {
         const long long lo = min(max(p.cu_seqlens[b], 0LL), static_cast<long long>(p.seqlen));
         const long long hi = min(max(p.cu_seqlens[b + 1], lo), static_cast<long long>(p.seqlen));
-        tok0 = static_cast<size_t>(lo);
-        sbase = static_cast<size_t>(h) * p.seqlen + static_cast<size_t>(lo);
-        T = static_cast<int>(hi - lo);
+        tok0_ = static_cast<size_t>(lo);
+        sbase_ = static_cast<size_t>(h) * p.seqlen + static_cast<size_t>(lo);
+        T_ = static_cast<int>(hi - lo);
     }
     // The offsets come from a vector load: make the sequence's range
     // wave-uniform so the buffer descriptors built from it stay in SGPRs.
-    T = __builtin_amdgcn_readfirstlane(T);
-    tok0 = Uniform64(tok0);
-    sbase = Uniform64(sbase);
+    const int T = __builtin_amdgcn_readfirstlane(T_);
+    const size_t tok0 = Uniform64(tok0_), sbase = Uniform64(sbase_);
+    // this workgroup's tokens [cs, te) of the sequence (cs a multiple of kC;
+    // te too, or the sequence's end)
+    int cs = 0, te = T;
+    bool last_seg = true;
+    if constexpr (MODE != kM3Whole) {
+        const int nseg = split.Segments(T);
+        if constexpr (kState) {
+            cs = seg * split.lf;
+            te = cs + split.lf;
+            if (te > (nseg - 1) * split.ls) return;   // no segment follows (workgroup-uniform)
+        } else {
+            if (seg >= nseg) return;
+            cs = seg * split.ls;
+            last_seg = seg == nseg - 1;
+            te = last_seg ? T : cs + split.ls;
+        }
+    }
+    const bool first_seg = seg == 0;
+    auto record_of = [&](int i) { return RecordAt(p, tok0 + cs, h, r0 + kRows * i, L::NP); };   // its i-th 32 rows'
+    const M3Record rec = record_of(0);
     const float *dtr = p.DT + sbase;
     const float *trr = p.Trap + sbase;
     const float *adr = p.ADT + sbase;
@@ -278,20 +383,25 @@ __global__ __launch_bounds__(64 * (NW + NPW)) void Mamba3ChunkKernel(Mamba3SisoP
         qbias[x] = real ? qb : make_float2(0.0f, 0.0f);
         kbias[x] = real ? kb : make_float2(0.0f, 0.0f);
         carry[x] = (p.in_angle != nullptr && rot) ? static_cast<double>(p.in_angle[static_cast<size_t>(bh) * A + pr[x]]) * kInvTwoPiF : 0.0;
+        if constexpr (kState) {
+            if (!first_seg) carry[x] = 0.0;   // counted from the segment's start
+        } else if constexpr (MODE == kM3Out) {
+            if (!product_wave && rot && !first_seg) carry[x] = rec.GetD(rec.StartAngle(pr[x]));
+        }
 #pragma unroll
         for (int s = 0; s < TPL; ++s) {
             qoff[x][s] = real ? ((TPL * tg + s) * static_cast<int>(q_stride) + 2 * pr[x]) * 4 : kOutOfRange;
             aoff[x][s] = rot ? ((TPL * tg + s) * static_cast<int>(a_stride) + pr[x]) * 4 : kOutOfRange;
         }
     }
-    // V values: block w + NPW u of 8 rows x 8 tokens (row block % 4, token
-    // block / 4), lane l: row l / 8, token l % 8 of the block
+    // V values: block w + NPW u of 8 rows x 8 tokens (row block % (ROWS / 8),
+    // token block / (ROWS / 8)), lane l: row l / 8, token l % 8 of the block
     int vrow[VPT], vtok[VPT], voff[VPT];
 #pragma unroll
     for (int u = 0; u < VPT; ++u) {
         const int blk = w + NPW * u;
-        vrow[u] = 8 * (blk % 4) + (lane >> 3);
-        vtok[u] = 8 * (blk / 4) + (lane & 7);
+        vrow[u] = 8 * (blk % (ROWS / 8)) + (lane >> 3);
+        vtok[u] = 8 * (blk / (ROWS / 8)) + (lane & 7);
         voff[u] = r0 + vrow[u] < P ? (vtok[u] * static_cast<int>(v_stride) + r0 + vrow[u]) * 4 : kOutOfRange;
     }
     // Without LONG (the host keeps T * stride * 4 < 2^31): one descriptor per
@@ -365,7 +475,7 @@ __global__ __launch_bounds__(64 * (NW + NPW)) void Mamba3ChunkKernel(Mamba3SisoP
             dts[s] = ld(d_, (TPL * tg + s) * 4, cd);
 #pragma unroll
             for (int x = 0; x < PB; ++x) {
-                qv[x][s] = ld2(q_, qoff[x][s], cq);
+                if constexpr (!kState) qv[x][s] = ld2(q_, qoff[x][s], cq);
                 kv[x][s] = ld2(k_, qoff[x][s], cq);
                 ang[x][s] = ld(a_, aoff[x][s], ca);
             }
@@ -416,23 +526,25 @@ __global__ __launch_bounds__(64 * (NW + NPW)) void Mamba3ChunkKernel(Mamba3SisoP
                 // a pair without an angle keeps theta = 0: sin 0 = 0, cos 0 = 1
                 const float rev = static_cast<float>(th * kRevPerTurn);
                 const float sn = __builtin_amdgcn_sinf(rev), c = __builtin_amdgcn_cosf(rev);
-                const float2 q = make_float2(qv[x][s].x + qbias[x].x, qv[x][s].y + qbias[x].y);
+                const float2 q = kState ? make_float2(0.0f, 0.0f) : make_float2(qv[x][s].x + qbias[x].x, qv[x][s].y + qbias[x].y);
                 const float2 k = make_float2(kv[x][s].x + kbias[x].x, kv[x][s].y + kbias[x].y);
-                qk[s] = fmaf(q.x, k.x, fmaf(q.y, k.y, qk[s]));   // unrotated q.k (reference :89-106)
-                *reinterpret_cast<float2 *>(bg + L::oQ + (TPL * tg + s) * QS + 2 * pr[x]) =
-                    make_float2(q.x * c - q.y * sn, q.x * sn + q.y * c);
+                if constexpr (!kState) {
+                    qk[s] = fmaf(q.x, k.x, fmaf(q.y, k.y, qk[s]));   // unrotated q.k (reference :89-106)
+                    *reinterpret_cast<float2 *>(bg + L::oQ + (TPL * tg + s) * QS + 2 * pr[x]) =
+                        make_float2(q.x * c - q.y * sn, q.x * sn + q.y * c);
+                }
                 kc0[s] = k.x * c - k.y * sn;
                 kc1[s] = k.x * sn + k.y * c;
-                if constexpr (L::KCOPY)
+                if constexpr (L::KCOPY && !kState)
                     *reinterpret_cast<float2 *>(bg + L::oK + (TPL * tg + s) * QS + 2 * pr[x]) = make_float2(kc0[s], kc1[s]);
             }
             const int r0k = 2 * pr[x], r1k = 2 * pr[x] + 1;   // this lane's tokens stay in one swizzled group
             if constexpr (TPL == 4) {
-                StF4(bg + L::oKT + r0k * kTS + KtCol(r0k, 4 * tg), v4f{kc0[0], kc0[1], kc0[2], kc0[3]});
-                StF4(bg + L::oKT + r1k * kTS + KtCol(r1k, 4 * tg), v4f{kc1[0], kc1[1], kc1[2], kc1[3]});
+                StF4(bg + oKT + r0k * kTS + KtCol(r0k, 4 * tg), v4f{kc0[0], kc0[1], kc0[2], kc0[3]});
+                StF4(bg + oKT + r1k * kTS + KtCol(r1k, 4 * tg), v4f{kc1[0], kc1[1], kc1[2], kc1[3]});
             } else {
-                *reinterpret_cast<float2 *>(bg + L::oKT + r0k * kTS + KtCol(r0k, TPL * tg)) = make_float2(kc0[0], kc0[1]);
-                *reinterpret_cast<float2 *>(bg + L::oKT + r1k * kTS + KtCol(r1k, TPL * tg)) = make_float2(kc1[0], kc1[1]);
+                *reinterpret_cast<float2 *>(bg + oKT + r0k * kTS + KtCol(r0k, TPL * tg)) = make_float2(kc0[0], kc0[1]);
+                *reinterpret_cast<float2 *>(bg + oKT + r1k * kTS + KtCol(r1k, TPL * tg)) = make_float2(kc1[0], kc1[1]);
             }
             // the chunk's last token
             if constexpr (PL == 16) {
@@ -448,7 +560,7 @@ __global__ __launch_bounds__(64 * (NW + NPW)) void Mamba3ChunkKernel(Mamba3SisoP
         }
         // q.k partial over this wave's pairs, per token
 #pragma unroll
-        for (int s = 0; s < TPL; ++s) {
+        for (int s = 0; s < (kState ? 0 : TPL); ++s) {
             float v = qk[s];
             v += DppF<0xB1>(v);    // quad_perm [1,0,3,2]
             v += DppF<0x4E>(v);    // quad_perm [2,3,0,1]
@@ -457,7 +569,7 @@ __global__ __launch_bounds__(64 * (NW + NPW)) void Mamba3ChunkKernel(Mamba3SisoP
             bf[L::oQK + w * kC + TPL * tg + s] = v;   // every lane of the token group holds the sum
         }
 #pragma unroll
-        for (int u = 0; u < VPT; ++u) bf[L::oVT + vrow[u] * kTS + vtok[u]] = vreg[u];
+        for (int u = 0; u < VPT; ++u) bf[oVT + vrow[u] * kTS + vtok[u]] = vreg[u];
         if (w == kScalarWave) {
             const float gam = r.sdt * FastSigmoid(r.strap);
             const float look = r.sdt1 * (1.0f - FastSigmoid(r.strap1));   // zero DT past the end
@@ -475,24 +587,33 @@ __global__ __launch_bounds__(64 * (NW + NPW)) void Mamba3ChunkKernel(Mamba3SisoP
 
     // ---- state: S^T tile (key block kb, row tile pt), lane i16 + 16 g4,
     // register r = S[row r0 + 16 pt + i16][key 16 (KBW w + kb) + 4 g4 + r]
-    v4f S[KBW][2];
+    v4f S[KBW][PT];
     {
         const float look0 = (p.in_ssm != nullptr && T > 0) ? dtr[0] * (1.0f - FastSigmoid(trr[0])) : 0.0f;
 #pragma unroll
         for (int kb = 0; kb < KBW; ++kb)
 #pragma unroll
-            for (int pt = 0; pt < 2; ++pt)
+            for (int pt = 0; pt < PT; ++pt)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int row = r0 + 16 * pt + i16, key = 16 * (KBW * w + kb) + 4 * g4 + r;
                     float v = 0.0f;
-                    if (product_wave && p.in_ssm != nullptr && row < P && key < N) {
+                    if (product_wave && first_seg && p.in_ssm != nullptr && row < P && key < N) {
                         const float vl = p.in_v[static_cast<size_t>(bh) * P + row];
                         const float kl = p.in_k[static_cast<size_t>(bh) * N + key];
                         v = fmaf(vl, kl * look0, p.in_ssm[(static_cast<size_t>(bh) * P + row) * N + key]);
                     }
                     S[kb][pt][r] = v;
                 }
+        if constexpr (MODE == kM3Out) {
+            if (product_wave && !first_seg) {
+#pragma unroll
+                for (int kb = 0; kb < KBW; ++kb)
+#pragma unroll
+                    for (int pt = 0; pt < PT; ++pt)
+                        if (16 * pt < rec.w) S[kb][pt] = *reinterpret_cast<const v4u *>(rec.State(((KBW * w + kb) * (rec.w / 16) + pt) * 64 + lane));
+            }
+        }
     }
 
     // ---- products of one chunk: partial G^T and Y to LDS, then the state update
@@ -514,7 +635,7 @@ __global__ __launch_bounds__(64 * (NW + NPW)) void Mamba3ChunkKernel(Mamba3SisoP
             const int kr = nb0 + 4 * g4 + ks;
             q[ks] = q4[ks];                                       // q^[t = i16][key nb0 + 4 g4 + ks]
             if constexpr (L::KCOPY) k[ks] = k4[ks];               // k^[s = i16][same key]
-            else k[ks] = bg[L::oKT + kr * kTS + KtCol(kr, i16)];
+            else k[ks] = bg[oKT + kr * kTS + KtCol(kr, i16)];
         }
     };
     auto products = [&](const float *bg, const float *bf, float *pp) __attribute__((always_inline)) {
@@ -522,52 +643,54 @@ __global__ __launch_bounds__(64 * (NW + NPW)) void Mamba3ChunkKernel(Mamba3SisoP
 #pragma unroll
         for (int kb = 0; kb < KBW; ++kb) {
             const int nb0 = 16 * (KBW * w + kb);
-            load_qk(bg, nb0, qa[kb], ka[kb]);
-            const v4f t4 = LdsF4(bg + L::oKT + (nb0 + i16) * kTS + KtCol(nb0 + i16, 4 * g4));
+            if constexpr (!kState) load_qk(bg, nb0, qa[kb], ka[kb]);
+            const v4f t4 = LdsF4(bg + oKT + (nb0 + i16) * kTS + KtCol(nb0 + i16, 4 * g4));
 #pragma unroll
             for (int ks = 0; ks < 4; ++ks) kt[kb][ks] = t4[ks];   // k^[s = 4 g4 + ks][key nb0 + i16]
         }
-        if (w >= 2) {
+        if (!kState && w >= 2) {
 #pragma unroll
             for (int x = 0; x < GX; ++x) load_qk(bg, 16 * (KBW * (w - 2) + GK0 + x), qx[x], kx[x]);
         }
         const v4f cs = LdsF4(bf + L::oCs + 4 * g4);
         const float ecum15 = bf[L::oEcum + kC - 1];
-        v4f vt[2];
+        v4f vt[PT];
 #pragma unroll
-        for (int pt = 0; pt < 2; ++pt) vt[pt] = LdsF4(bf + L::oVT + (16 * pt + i16) * kTS + 4 * g4);
+        for (int pt = 0; pt < PT; ++pt) vt[pt] = LdsF4(bf + oVT + (16 * pt + i16) * kTS + 4 * g4);
 
-        v4f gp = {0.0f, 0.0f, 0.0f, 0.0f};
+        if constexpr (!kState) {
+            v4f gp = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int kb = 0; kb < GK0; ++kb)
+            for (int kb = 0; kb < GK0; ++kb)
 #pragma unroll
-            for (int ks = 0; ks < 4; ++ks) gp = Mfma(ka[kb][ks], qa[kb][ks], gp);   // G^T[s][t]
-        if (w >= 2) {
+                for (int ks = 0; ks < 4; ++ks) gp = Mfma(ka[kb][ks], qa[kb][ks], gp);   // G^T[s][t]
+            if (w >= 2) {
 #pragma unroll
-            for (int kb = GK0; kb < KBW; ++kb)
+                for (int kb = GK0; kb < KBW; ++kb)
 #pragma unroll
-                for (int ks = 0; ks < 4; ++ks) gp = Mfma(ka[kb][ks], qa[kb][ks], gp);
+                    for (int ks = 0; ks < 4; ++ks) gp = Mfma(ka[kb][ks], qa[kb][ks], gp);
 #pragma unroll
-            for (int x = 0; x < GX; ++x)
+                for (int x = 0; x < GX; ++x)
 #pragma unroll
-                for (int ks = 0; ks < 4; ++ks) gp = Mfma(kx[x][ks], qx[x][ks], gp);
+                    for (int ks = 0; ks < 4; ++ks) gp = Mfma(kx[x][ks], qx[x][ks], gp);
+            }
+            v4f yp[2];
+#pragma unroll
+            for (int pt = 0; pt < 2; ++pt) {
+                yp[pt] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int kb = 0; kb < KBW; ++kb)
+#pragma unroll
+                    for (int ks = 0; ks < 4; ++ks) yp[pt] = Mfma(qa[kb][ks], S[kb][pt][ks], yp[pt]);   // Y[t][row]
+            }
+            if (GK0 > 0 || w >= 2) StF4(pp + ((w * 3 + 0) * 64 + lane) * 4, gp);
+            StF4(pp + ((w * 3 + 1) * 64 + lane) * 4, yp[0]);
+            StF4(pp + ((w * 3 + 2) * 64 + lane) * 4, yp[1]);
         }
-        v4f yp[2];
-#pragma unroll
-        for (int pt = 0; pt < 2; ++pt) {
-            yp[pt] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int kb = 0; kb < KBW; ++kb)
-#pragma unroll
-                for (int ks = 0; ks < 4; ++ks) yp[pt] = Mfma(qa[kb][ks], S[kb][pt][ks], yp[pt]);   // Y[t][row]
-        }
-        if (GK0 > 0 || w >= 2) StF4(pp + ((w * 3 + 0) * 64 + lane) * 4, gp);
-        StF4(pp + ((w * 3 + 1) * 64 + lane) * 4, yp[0]);
-        StF4(pp + ((w * 3 + 2) * 64 + lane) * 4, yp[1]);
 
         // S^T = e^{cum_15} S^T + K^T V',  V'[s][row] = e^{cum_15 - cum_s} w_s v_s[row]
 #pragma unroll
-        for (int pt = 0; pt < 2; ++pt) {
+        for (int pt = 0; pt < PT; ++pt) {
             float vs[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) vs[r] = vt[pt][r] * cs[r];
@@ -667,12 +790,12 @@ __global__ __launch_bounds__(64 * (NW + NPW)) void Mamba3ChunkKernel(Mamba3SisoP
         }
     };
 
-    const int nch = (T + kC - 1) / kC;
+    const int nch = (te - cs + kC - 1) / kC;
     using P0 = std::integral_constant<int, 0>;
     using P1 = std::integral_constant<int, 1>;
-    auto big = [&](auto P) { return smem + L::oBig + decltype(P)::value * L::kBig; };      // chunk parity P
+    auto big = [&](auto P) { return smem + L::oBig + decltype(P)::value * kBig; };      // chunk parity P
     auto par = [&](auto P) { return part + decltype(P)::value * L::kPart; };
-    auto small = [&](int j) { return smem + L::oSmall + (j % kBufs) * L::kSmall; };
+    auto small = [&](int j) { return smem + oSmall + (j % kBufs) * (kState ? L::kStateSmall : L::kSmall); };
     // Each role runs its own loop (the same barriers, in the same order), so
     // the registers one role carries across chunks (the state S; the
     // prefetched inputs and angle carries) never have to coexist, and no wave
@@ -682,7 +805,61 @@ __global__ __launch_bounds__(64 * (NW + NPW)) void Mamba3ChunkKernel(Mamba3SisoP
     // 0 and 1) or the shared finishing work of chunk j (waves 2 and 3) |
     // prefetch of chunk j+2, preparation of chunk j+1.  Chunk 0's products and
     // the last chunk's finishing are peeled.
-    if (nch > 0 && product_wave && w < 2) {   // workgroup-uniform: an empty sequence passes its states through
+    auto prepare_chunks = [&]() __attribute__((always_inline)) {   // the preparation waves' loop
+        load_prep(cs, raw0);
+        if constexpr (DB) load_prep(cs + min(1, nch - 1) * kC, raw1);
+        prep(big(P0{}), small(0), raw0);
+        if constexpr (!DB) load_prep(cs + min(1, nch - 1) * kC, raw0);
+        __syncthreads();
+        // unrolled by two for the register sets and the parity (P: chunk j + 1's)
+        auto iter = [&](int j, auto P, Raw &ld, const Raw &pr_) __attribute__((always_inline)) {
+            if constexpr (DB) load_prep(cs + min(j + 2, nch - 1) * kC, ld);
+            prep(big(P), small(j + 1), pr_);
+            if constexpr (!DB) load_prep(cs + min(j + 2, nch - 1) * kC, ld);
+            __syncthreads();
+        };
+        if (nch > 1) {
+            for (int j = 0;; j += 2) {
+                iter(j, P1{}, raw0, DB ? raw1 : raw0);
+                if (j + 2 >= nch) break;
+                iter(j + 1, P0{}, DB ? raw1 : raw0, raw0);
+                if (j + 3 >= nch) break;
+            }
+        }
+        __syncthreads();   // the products of the last chunk
+    };
+    if constexpr (kState) {
+        // the same pipeline without products of q and without finishing: the
+        // product waves update the state, the preparation waves run ahead
+        if (product_wave) {
+            float csum = 0.0f;   // the segment's sum of ADT
+            __syncthreads();
+            auto step = [&](int j, auto P) __attribute__((always_inline)) {
+                csum += small(j)[L::oCum + kC - 1];
+                products(big(P), small(j), par(P));
+                __syncthreads();
+            };
+            for (int j = 0; j < nch; j += 2) {
+                step(j, P0{});
+                if (j + 1 >= nch) break;
+                step(j + 1, P1{});
+            }
+#pragma unroll
+            for (int kb = 0; kb < KBW; ++kb)
+#pragma unroll
+                for (int pt = 0; pt < PT; ++pt) {   // two row tiles to each row block's record
+                    if (r0 + 16 * pt >= P) continue;
+                    const M3Record rp = record_of(pt / 2);
+                    *reinterpret_cast<v4u *>(rp.State(((KBW * w + kb) * (rp.w / 16) + pt % 2) * 64 + lane)) = S[kb][pt];
+                }
+            if (tid < PT / 2 && r0 + kRows * tid < P) {
+                const M3Record rp = record_of(tid);
+                *rp.At(rp.DecaySum()) = csum;
+            }
+            return;
+        }
+        prepare_chunks();
+    } else if (nch > 0 && product_wave && w < 2) {   // workgroup-uniform: an empty sequence passes its states through
         __syncthreads();
         // Z of chunk j is loaded in iteration j (before its products) into
         // the register set of j's parity and gated in iteration j + 1, where
@@ -692,7 +869,7 @@ __global__ __launch_bounds__(64 * (NW + NPW)) void Mamba3ChunkKernel(Mamba3SisoP
         // complete.  The sets are written only by the Z loads: a zeroing in
         // every iteration landed on registers the previous stores read.
         float za[4] = {0.0f, 0.0f, 0.0f, 0.0f}, zb[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-        load_z(0, za);
+        load_z(cs, za);
         products(big(P0{}), small(0), par(P0{}));
         __syncthreads();
         // zl: the set for chunk j's Z; zu: chunk j - 1's, finished here.  The
@@ -702,11 +879,11 @@ __global__ __launch_bounds__(64 * (NW + NPW)) void Mamba3ChunkKernel(Mamba3SisoP
         // P: chunk j's parity.
         auto iter = [&](int j, auto P, float (&zl)[4], const float (&zu)[4]) __attribute__((always_inline)) {
             using Q = std::integral_constant<int, 1 - decltype(P)::value>;
-            load_z(j * kC, zl);
+            load_z(cs + j * kC, zl);
             products(big(P), small(j), par(P));
             float y[4];
             finish(small(j - 1), par(Q{}), zu, y);
-            store_y((j - 1) * kC, y);
+            store_y(cs + (j - 1) * kC, y);
             __syncthreads();
         };
         for (int j = 1; j < nch; j += 2) {   // unrolled by two for the sets and the parity
@@ -717,7 +894,7 @@ __global__ __launch_bounds__(64 * (NW + NPW)) void Mamba3ChunkKernel(Mamba3SisoP
         float y[4];
         if ((nch - 1) & 1) finish(small(nch - 1), par(P1{}), zb, y);
         else finish(small(nch - 1), par(P0{}), za, y);
-        store_y((nch - 1) * kC, y);
+        store_y(cs + (nch - 1) * kC, y);
     } else if (nch > 0 && product_wave) {   // waves 2 and 3: products and the shared finishing work
         __syncthreads();
         auto step = [&](int j, auto P) __attribute__((always_inline)) {
@@ -731,30 +908,20 @@ __global__ __launch_bounds__(64 * (NW + NPW)) void Mamba3ChunkKernel(Mamba3SisoP
             step(j + 1, P1{});
         }
     } else if (nch > 0) {
-        load_prep(0, raw0);
-        if constexpr (DB) load_prep(min(1, nch - 1) * kC, raw1);
-        prep(big(P0{}), small(0), raw0);
-        if constexpr (!DB) load_prep(min(1, nch - 1) * kC, raw0);
-        __syncthreads();
-        // unrolled by two for the register sets and the parity (P: chunk j + 1's)
-        auto iter = [&](int j, auto P, Raw &ld, const Raw &pr_) __attribute__((always_inline)) {
-            if constexpr (DB) load_prep(min(j + 2, nch - 1) * kC, ld);
-            prep(big(P), small(j + 1), pr_);
-            if constexpr (!DB) load_prep(min(j + 2, nch - 1) * kC, ld);
-            __syncthreads();
-        };
-        if (nch > 1) {
-            for (int j = 0;; j += 2) {
-                iter(j, P1{}, raw0, DB ? raw1 : raw0);
-                if (j + 2 >= nch) break;
-                iter(j + 1, P0{}, DB ? raw1 : raw0, raw0);
-                if (j + 3 >= nch) break;
-            }
-        }
-        __syncthreads();   // the products of the last chunk
+        prepare_chunks();
     }
 
-    if (p.f_ssm != nullptr) {
+    if constexpr (kState) {   // preparation waves: the angles after the segment's last token
+#pragma unroll
+        for (int x = 0; x < PB; ++x)
+            if (tg == 0 && pr[x] < A) {
+#pragma unroll
+                for (int i = 0; i < ROWS / kRows; ++i)
+                    if (r0 + kRows * i < P) record_of(i).PutD(record_of(i).AngleSum(pr[x]), carry[x]);
+            }
+        return;
+    }
+    if (p.f_ssm != nullptr && last_seg) {
         if (product_wave) {
 #pragma unroll
             for (int kb = 0; kb < KBW; ++kb)
@@ -778,8 +945,8 @@ __global__ __launch_bounds__(64 * (NW + NPW)) void Mamba3ChunkKernel(Mamba3SisoP
         }
         if (rb == 0) {
             // the last chunk's tiles are intact: its k^T column of the last token
-            const int tl = T > 0 ? (T - 1) - (nch - 1) * kC : 0;
-            const float *kt = smem + L::oBig + ((nch > 0 ? nch - 1 : 0) & 1) * L::kBig + L::oKT;
+            const int tl = T > 0 ? (T - 1) - cs - (nch - 1) * kC : 0;
+            const float *kt = smem + L::oBig + ((nch > 0 ? nch - 1 : 0) & 1) * kBig + oKT;
             for (int i = tid; i < N; i += NT) {
                 const size_t o = static_cast<size_t>(bh) * N + i;
                 p.f_k[o] = T > 0 ? kt[i * kTS + KtCol(i, tl)] : (p.in_k != nullptr ? p.in_k[o] : 0.0f);
@@ -788,27 +955,176 @@ __global__ __launch_bounds__(64 * (NW + NPW)) void Mamba3ChunkKernel(Mamba3SisoP
     }
 }
 
-template <int KBW, int NW, int NPW, bool LONG, bool HASZ>
-void LaunchChunkZ(const Mamba3SisoParams &p, hipStream_t stream) {
-    using L = M3CLayout<KBW, NW, NPW>;
-    const long long blocks = static_cast<long long>(p.batch) * p.nheads * ((p.p + kRows - 1) / kRows);
-    if (blocks > 2147483647LL) throw Error(XM_ERR_INVALID_ARGUMENT, "Mamba3SisoFn launch exceeds the grid limit");
-    EnsureDynamicLds(reinterpret_cast<const void *>(&Mamba3ChunkKernel<KBW, NW, NPW, LONG, HASZ>), static_cast<int>(L::kBytes));
-    XM_NOTE_LAUNCH("Mamba3ChunkKernel", {}, KBW, NW, NPW, LONG);
-    hipLaunchKernelGGL((Mamba3ChunkKernel<KBW, NW, NPW, LONG, HASZ>), dim3(static_cast<unsigned>(blocks)), dim3(L::NT),
-                       L::kBytes, stream, p);
+// True when the output shares no byte with an input or a state, so that its
+// rows can hold the sequence split's records while the inputs are still read.
+bool OutputApart(const Mamba3SisoParams &p) {
+    const bool packed = p.cu_seqlens != nullptr;
+    const size_t f = sizeof(float), rows = static_cast<size_t>(packed ? 1 : p.batch) * p.seqlen;
+    const size_t v = rows * p.nheads * p.p * f, q = rows * p.nheads_qk * p.n * f, bh = static_cast<size_t>(p.batch) * p.nheads * f;
+    const uintptr_t o = reinterpret_cast<uintptr_t>(p.out);
+    auto apart = [&](const void *x, size_t bytes) {
+        const uintptr_t a = reinterpret_cast<uintptr_t>(x);
+        return x == nullptr || a + bytes <= o || o + v <= a;
+    };
+    return apart(p.Q, q) && apart(p.K, q) && apart(p.V, v) && apart(p.Z, v) && apart(p.Angles, rows * p.nheads * p.a * f) &&
+           apart(p.ADT, rows * p.nheads * f) && apart(p.DT, rows * p.nheads * f) && apart(p.Trap, rows * p.nheads * f) &&
+           apart(p.Q_bias, static_cast<size_t>(p.nheads) * p.n * f) && apart(p.K_bias, static_cast<size_t>(p.nheads) * p.n * f) &&
+           apart(p.D, static_cast<size_t>(p.nheads) * f) && apart(p.cu_seqlens, (static_cast<size_t>(p.batch) + 1) * 8) &&
+           apart(p.in_ssm, bh * p.p * p.n) && apart(p.in_angle, bh * p.a) && apart(p.in_k, bh * p.n) && apart(p.in_v, bh * p.p) &&
+           apart(p.f_ssm, bh * p.p * p.n) && apart(p.f_angle, bh * p.a) && apart(p.f_k, bh * p.n) && apart(p.f_v, bh * p.p);
 }
 
-template <int KBW, int NW, int NPW, bool LONG>
-void LaunchChunkL(const Mamba3SisoParams &p, hipStream_t stream) {
-    if (p.Z != nullptr) LaunchChunkZ<KBW, NW, NPW, LONG, true>(p, stream);
-    else LaunchChunkZ<KBW, NW, NPW, LONG, false>(p, stream);
+// Split when the row blocks fill at most half the CUs, into as many output
+// segments as fill them (one workgroup per CU: its registers and LDS admit no
+// second), each of as many fine segments as let the state launch fill them too.
+// Measured, 64 x 128 heads (us, whole -> split): 1 x 3001 x 32 heads 285 -> 119
+// (4 output segments of 2 fine ones; of 1: 143, of 3: 134), 2 x 4096 x 32 388 ->
+// 254 (2 of 4; 4 of 1: 295), 1 x 4096 x 8 385 -> 67 (16 of 2), 1 x 1024 x 32 101 ->
+// 63, 1 x 600 x 32 63 -> 58; 128 x 256 heads, 1 x 4096 x 16 728 -> 280.  Packed
+// sequences, whose lengths the host does not know, split where the whole pass
+// fills at most a quarter of the CUs and sequences of even length would gain:
+// 4096 tokens in 2 sequences x 8 heads 299 -> 103, 3 x 8 289 -> 147, 2 x 16 301 ->
+// 167; above that segments sized by the row can lose (5 x 16 heads of 64 keys 179 ->
+// 188).
+constexpr long long kSplitBlocks = 256;   // CUs
+constexpr int kSplitMax = 16, kFineMax = 8;
+M3Split ChooseSplit(const Mamba3SisoParams &p, int np) {
+    const M3Split whole{0, 0, 0, 1};
+    const int forced = static_cast<int>(GetOverride(kOverrideM3Split));
+    if (forced == 1 || p.p % 16 != 0 || !OutputApart(p)) return whole;
+    // a 32-row workgroup of the output launch and a 64-row one of the state
+    // launch per CU: one round of each (packed: of the whole row's segments)
+    const bool packed = p.cu_seqlens != nullptr;
+    const long long bh = static_cast<long long>(packed ? 1 : p.batch) * p.nheads;
+    const long long w32 = bh * ((p.p + kRows - 1) / kRows), w64 = bh * ((p.p + kStateRows - 1) / kStateRows);
+    const long long walks = packed ? w32 * p.batch : w32;   // workgroups of the whole pass
+    if (forced != 2 && walks > (packed ? kSplitBlocks / 4 : kSplitBlocks / 2)) return whole;
+    const long long most = std::max<long long>(2, std::min<long long>(kSplitMax, kSplitBlocks / w32));
+    const float t_whole = static_cast<float>(p.seqlen) / (packed ? std::max(p.batch, 1) : 1) / kC;
+    const int need = M3RecordTokens(np);
+    auto up = [](long long x) { return static_cast<int>((x + kC - 1) / kC * kC); };
+    for (int s = static_cast<int>(most); s >= 2; --s) {
+        const int ls = up((static_cast<long long>(p.seqlen) + s - 1) / s);
+        for (int m = static_cast<int>(std::max<long long>(1, std::min<long long>(kFineMax, kSplitBlocks / (w64 * (s - 1))))); m >= 1; --m) {
+            const int lf = up((ls + m - 1) / m);
+            if (lf < up(need)) continue;
+            M3Split split{lf * m, lf, need, 0};
+            split.maxseg = split.Segments(p.seqlen);
+            if (split.maxseg < 2) continue;
+            // in chunk steps: the longest output segment, the fine segment (0.75
+            // of a step each) and 12 us of launches (8 steps) against the sequence
+            const int out = packed ? split.ls + need : std::max(split.ls, p.seqlen - (split.maxseg - 1) * split.ls);
+            const float t_split = (out + 0.75f * lf) / kC + 8.0f;
+            if (forced == 2 || t_split < 0.9f * t_whole) return split;
+        }
+    }
+    return whole;
+}
+
+// Launch 2 of the sequence split: the start states and start angles of the
+// output segments.  A thread takes four state values, two key pairs of one
+// row; the end states are read before the start states take their places.
+__global__ __launch_bounds__(256) void Mamba3SegCombineKernel(Mamba3SisoParams p, M3Split split, int np, int blocks) {
+    const int H = p.nheads, A = p.a;
+    const int nrb = (p.p + kRows - 1) / kRows;
+    const int blk = blockIdx.x % blocks, rb = blockIdx.x / blocks % nrb, bh = blockIdx.x / blocks / nrb;
+    const int b = bh / H, h = bh % H;
+    const M3Range r = RangeOf(p, b);
+    const int m = split.ls / split.lf, nf = (split.Segments(r.T) - 1) * m;   // fine segments that another follows
+    const int q = blk * 256 + threadIdx.x;
+    auto record = [&](int f) { return RecordAt(p, r.tok0 + static_cast<size_t>(f) * split.lf, h, rb * kRows, np); };
+    const M3Record r0 = record(0);
+    if (nf < 1 || q >= np * r0.w / 4) return;
+    // tile order: key block, row tile, lane; keys 16 block + 4 (lane / 16) .. + 3
+    const int tiles = r0.w / 16, lane = q % 64, key = 16 * (q / 64 / tiles) + 4 * (lane / 16);
+    const bool writes_angles = q / 64 % tiles == 0 && lane % 16 == 0;   // one row's threads write their pairs'
+    double th[2] = {0.0, 0.0};
+    v4f S = {0.0f, 0.0f, 0.0f, 0.0f};   // the state before fine segment f
+    // segment f's end state, angle sums and decay, read one segment ahead
+    struct Rec {
+        v4f end;
+        double dth[2];
+        float decay;
+    };
+    auto load = [&](int f) {
+        Rec x{{0.0f, 0.0f, 0.0f, 0.0f}, {0.0, 0.0}, 0.0f};
+        if (f >= nf) return x;
+        const M3Record rf = record(f);
+        x.end = *reinterpret_cast<const v4u *>(rf.State(q));
+        x.decay = *rf.At(rf.DecaySum());
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+            if (key / 2 + e < A) x.dth[e] = rf.GetD(rf.AngleSum(key / 2 + e));
+        return x;
+    };
+    Rec next = load(0);
+    for (int f = 0; f <= nf; ++f) {
+        Rec cur = next;
+        next = load(f + 1);
+        if (f > 0 && f % m == 0) {
+            const M3Record rf = record(f);
+            *reinterpret_cast<v4u *>(rf.State(q)) = S;
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+                if (writes_angles && key / 2 + e < A) rf.PutD(rf.StartAngle(key / 2 + e), th[e]);
+        }
+        // the end state turned by the segment's start angles (zero for segment
+        // 0, which has the true ones, and for pairs without an angle)
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+            const float rev = static_cast<float>(th[x] * kRevPerTurn);
+            const float sn = __builtin_amdgcn_sinf(rev), c = __builtin_amdgcn_cosf(rev);
+            const float e0 = cur.end[2 * x], e1 = cur.end[2 * x + 1];
+            cur.end[2 * x] = e0 * c - e1 * sn;
+            cur.end[2 * x + 1] = e0 * sn + e1 * c;
+            th[x] = __builtin_amdgcn_fract(th[x] + cur.dth[x]);
+        }
+        // the decay in two halves, which keeps its product with S in range
+        // where the decay alone is not; a zero state stays zero under any growth
+        const float half = __expf(0.5f * cur.decay);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) S[e] = S[e] == 0.0f ? cur.end[e] : fmaf(half * S[e], half, cur.end[e]);
+    }
+}
+
+template <int KBW, int NW, int NPW, bool LONG, bool HASZ, int MODE>
+void LaunchChunkMode(const Mamba3SisoParams &p, const M3Split &split, hipStream_t stream) {
+    using L = M3CLayout<KBW, NW, NPW>;
+    const int nseg = MODE == kM3Whole ? 1 : (MODE == kM3State ? (split.maxseg - 1) * (split.ls / split.lf) : split.maxseg);
+    constexpr int ROWS = MODE == kM3State ? kStateRows : kRows;
+    const long long blocks = static_cast<long long>(p.batch) * p.nheads * ((p.p + ROWS - 1) / ROWS) * nseg;
+    if (blocks > 2147483647LL) throw Error(XM_ERR_INVALID_ARGUMENT, "Mamba3SisoFn launch exceeds the grid limit");
+    constexpr size_t kLds = MODE == kM3State ? L::kStateBytes : L::kBytes;
+    EnsureDynamicLds(reinterpret_cast<const void *>(&Mamba3ChunkKernel<KBW, NW, NPW, LONG, HASZ, MODE>), static_cast<int>(kLds));
+    if constexpr (MODE == kM3Whole) XM_NOTE_LAUNCH("Mamba3ChunkKernel", {}, KBW, NW, NPW, LONG);
+    else XM_NOTE_LAUNCH("Mamba3ChunkKernel", {}, KBW, NW, NPW, LONG, HASZ, MODE);
+    hipLaunchKernelGGL((Mamba3ChunkKernel<KBW, NW, NPW, LONG, HASZ, MODE>), dim3(static_cast<unsigned>(blocks)), dim3(L::NT),
+                       kLds, stream, p, split);
+}
+
+template <int KBW, int NW, int NPW>
+void LaunchSplit(const Mamba3SisoParams &p, const M3Split &split, hipStream_t stream) {
+    constexpr int NP = M3CLayout<KBW, NW, NPW>::NP;
+    const unsigned bh = static_cast<unsigned>(p.batch) * p.nheads;
+    LaunchChunkMode<KBW, NW, NPW, false, false, kM3State>(p, split, stream);
+    const int nrb = (p.p + kRows - 1) / kRows, parts = (NP * std::min(kRows, p.p) / 4 + 255) / 256;
+    XM_NOTE_LAUNCH("Mamba3SegCombineKernel", {}, );
+    hipLaunchKernelGGL(Mamba3SegCombineKernel, dim3(bh * nrb * parts), dim3(256), 0, stream, p, split, NP, parts);
+    if (p.Z != nullptr) LaunchChunkMode<KBW, NW, NPW, false, true, kM3Out>(p, split, stream);
+    else LaunchChunkMode<KBW, NW, NPW, false, false, kM3Out>(p, split, stream);
 }
 
 template <int KBW, int NW, int NPW>
 void LaunchChunk(const Mamba3SisoParams &p, bool long_rows, hipStream_t stream) {
-    if (long_rows) LaunchChunkL<KBW, NW, NPW, true>(p, stream);
-    else LaunchChunkL<KBW, NW, NPW, false>(p, stream);
+    const M3Split none{};
+    if (!long_rows) {
+        const M3Split split = ChooseSplit(p, M3CLayout<KBW, NW, NPW>::NP);
+        if (split.maxseg > 1) return LaunchSplit<KBW, NW, NPW>(p, split, stream);
+    }
+    if (long_rows && p.Z != nullptr) LaunchChunkMode<KBW, NW, NPW, true, true, kM3Whole>(p, none, stream);
+    else if (long_rows) LaunchChunkMode<KBW, NW, NPW, true, false, kM3Whole>(p, none, stream);
+    else if (p.Z != nullptr) LaunchChunkMode<KBW, NW, NPW, false, true, kM3Whole>(p, none, stream);
+    else LaunchChunkMode<KBW, NW, NPW, false, false, kM3Whole>(p, none, stream);
 }
 
 }  // namespace

@@ -149,6 +149,7 @@ enum Override {
     kOverrideGdn2Windowed,   // 1: GDN-2 chunked path in windows of 128 chunks (not sized to 128 MiB / one packed window)
     kOverrideGdn2Split,      // GDN-2 chunked path: 1 never split the sequence, 2 split it wherever it has 2+ chunks, 3 two unequal segments (the second two tiles per workgroup)
     kOverrideGdn2Ct,         // GDN-2 chunked recurrence: value-column tiles per workgroup (1 or 2)
+    kOverrideM3Split,        // Mamba3SisoFn chunked kernel: 1 never split the sequence, 2 split wherever the output rows hold the records
     kOverrideCount
 };
 int64_t GetOverride(Override which);

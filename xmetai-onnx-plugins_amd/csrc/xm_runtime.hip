@@ -158,6 +158,7 @@ constexpr OverrideSpec kOverrides[kOverrideCount] = {
     {"gdn2_split", {1, 2, 3, 0}},        // GDN-2 chunked: 1 no sequence split, 2 split wherever 2+ chunks,
                                          // 3 two unequal segments, the second at two tiles per workgroup
     {"gdn2_ct", {1, 2, 0}},              // GDN-2 chunked: 1 or 2 value-column tiles per recurrence workgroup
+    {"m3_split", {1, 2, 0}},             // Mamba-3 chunked: 1 no sequence split, 2 split wherever possible
 };
 std::atomic<int64_t> g_override[kOverrideCount];
 
