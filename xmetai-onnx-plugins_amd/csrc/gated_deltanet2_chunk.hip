@@ -572,8 +572,8 @@ __device__ __forceinline__ void DecayState(v4f (&S)[KPW], const float (&sc)[NSV]
 // token rows; T: its length; sbase: the row's offset in the [B,H,K,V] states.
 // The state comes from s_in (zeros when null) and goes to s_out (not written
 // when null).  Every wave of the workgroup calls it with the same arguments.
-// Column tiles of a sequence-split run (Gdn2ChunkSplitKernel,
-// Gdn2ChunkSplit2Kernel), in units of the workgroup's CT tiles: with VW =
+// The workgroup's column tiles, and for a sequence-split run
+// (Gdn2ChunkSplitKernel, Gdn2ChunkSplit2Kernel) what they are, in units of the workgroup's CT tiles: with VW =
 // ceil(VT / CT), units below VW are value columns; unit VW + j carries the
 // identity columns 16 (CT j + c)..+15 (keys) in its tile c: WV = 0, initial
 // state I, the output goes to `psi` ([B,T,H,KP] rows, KP = keys padded to
@@ -589,7 +589,7 @@ struct SplitTile {
 template <int KPW, int KS, int CT = 1, bool SPLIT = false>
 __device__ __forceinline__ void Gdn2RecurRun(const GatedDeltaNet2Params &p, float *sXp, int h, size_t tok0, int T,
                                              int cs, int cw0, int nrun, int wn, const float *prep_row, size_t sbase,
-                                             const float *s_in, float *s_out, SplitTile st = {}) {
+                                             const float *s_in, float *s_out, SplitTile st) {
     using L = RecurLayout<KPW, KS, CT>;
     using Ops = ChunkOperands<KPW, KS, CT>;
     constexpr int KQ = L::KQ, FB = L::FB, NSV = L::NSV, NM = L::NM;
@@ -599,7 +599,7 @@ __device__ __forceinline__ void Gdn2RecurRun(const GatedDeltaNet2Params &p, floa
     const int lane = threadIdx.x & 63, ks = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int g4 = lane >> 4;
     const int VT = (dv + 15) / 16, VW = (VT + CT - 1) / CT;   // column tiles; workgroups per (b, h)
-    const int vt = SPLIT ? st.tile : XcdLocalBlock(blockIdx.x, gridDim.x) % VW;
+    const int vt = st.tile;
     const bool ident = SPLIT && st.ident;
     // this lane's value column in each of the workgroup's CT column tiles
     int col[CT];
@@ -972,18 +972,20 @@ __global__ __launch_bounds__(64 * KS) void Gdn2ChunkRecurKernel(GatedDeltaNet2Pa
     __shared__ __attribute__((aligned(16))) float sXp[L::kFloats];
     const int H = p.nheads;
     const int VW = ((p.dv + 15) / 16 + CT - 1) / CT;   // workgroups per (b, h)
-    const int row = XcdLocalBlock(blockIdx.x, gridDim.x) / VW;
     const size_t kv = static_cast<size_t>(p.dk) * p.dv;
     if constexpr (!PACKED) {
+        const int wg = XcdLocalBlock(blockIdx.x, gridDim.x), row = wg / VW;
         const int b = row / H, h = row % H;
         Gdn2RecurRun<KPW, KS, CT>(p, sXp, h, static_cast<size_t>(b) * p.seqlen, p.seqlen, c0, 0, wn, wn,
                                   p.prepared + static_cast<size_t>(row) * wn * L::FB, static_cast<size_t>(row) * kv,
-                                  s_in, s_out);
+                                  s_in, s_out, SplitTile{wg % VW, false, nullptr});
         return;
     } else {
     const int n = p.batch;
-    const int slots = static_cast<int>(gridDim.x) / (H * VW);
-    const int slot = row / H, h = row % H;
+    const int slots = min(n, wn);
+    const XcdUnit u = XcdSpreadUnit(blockIdx.x, VW);
+    const int slot = u.unit / H, h = u.unit % H;
+    if (slot >= slots) return;
     const float *const prep_row = p.prepared + static_cast<size_t>(h) * wn * L::FB;
     for (int b = slot; b < n; b += slots) {   // workgroup-uniform
         const int i0 = p.chunk_off[b], nrun = p.chunk_off[b + 1] - i0;
@@ -995,7 +997,8 @@ __global__ __launch_bounds__(64 * KS) void Gdn2ChunkRecurKernel(GatedDeltaNet2Pa
         const size_t sbase = (static_cast<size_t>(b) * H + h) * kv;
         const float *in = c0 == 0 ? p.initial_state : p.state;
         float *out = c0 + nrun == nch ? p.final_state : p.state;
-        Gdn2RecurRun<KPW, KS, CT>(p, sXp, h, tok0, T, c0, i0, nrun, wn, prep_row, sbase, in, out);
+        Gdn2RecurRun<KPW, KS, CT>(p, sXp, h, tok0, T, c0, i0, nrun, wn, prep_row, sbase, in, out,
+                                  SplitTile{u.part, false, nullptr});
     }
     }
 }
@@ -1547,8 +1550,10 @@ void LaunchRecur(const GatedDeltaNet2Params &p, int c0, int wn, int kq, const fl
     if (blocks == 0) return;   // no packed sequences
     if (blocks > 2147483647LL) throw Error(XM_ERR_INVALID_ARGUMENT, "GatedDeltaNet2Fn launch exceeds the grid limit");
     if (p.chunk_off != nullptr) {
+        const long long spread = XcdSpreadBlocks(rows * p.nheads, vt);
+        if (spread > 2147483647LL) throw Error(XM_ERR_INVALID_ARGUMENT, "GatedDeltaNet2Fn launch exceeds the grid limit");
         XM_NOTE_LAUNCH("Gdn2ChunkRecurKernel", {}, KPW, KS, CT, 1);
-        hipLaunchKernelGGL((Gdn2ChunkRecurKernel<KPW, KS, CT, true>), dim3(static_cast<unsigned>(blocks)),
+        hipLaunchKernelGGL((Gdn2ChunkRecurKernel<KPW, KS, CT, true>), dim3(static_cast<unsigned>(spread)),
                            dim3(64 * KS), 0, stream, p, c0, wn, s_in, s_out);
     } else {
         XM_NOTE_LAUNCH("Gdn2ChunkRecurKernel", {}, KPW, KS, CT, 0);
@@ -1871,9 +1876,9 @@ __global__ __launch_bounds__(256) void Gdn2PackedChunksKernel(GatedDeltaNet2Para
         for (int b = b0; b < b1; ++b) sum += in_window(b);
         part[tid] = sum;
         __syncthreads();
-        if (tid == 0) {   // exclusive prefix of the 256 partial sums
+        if (tid == 0) {   // exclusive prefix of the partial sums in use
             int acc = 0;
-            for (int i = 0; i < 256; ++i) {
+            for (int i = 0; i * per < n; ++i) {
                 const int v = part[i];
                 part[i] = acc;
                 acc += v;

@@ -280,8 +280,12 @@ __device__ __forceinline__ M3Range RangeOf(const Mamba3SisoParams &p, int b) {
 // descriptors that start at its own first token.
 // HASZ: a Z input (the SiLU gate); without one the finishing waves issue no Z
 // loads and no gate.
-// MODE: the whole sequence, or a launch of the sequence split (above).
-template <int KBW, int NW, int NPW, bool LONG, bool HASZ, int MODE>
+// MODE: the whole sequence, or a launch of the sequence split (above).  PACKED:
+// cu_seqlens absent (0), given (1), or seen at run time (2).  A kernel of its own
+// leaves the unpacked pass free of the offsets' code (4 x 4096 x 32 heads 365 ->
+// 360 us), but with a Z the compiler schedules that kernel worse (380 -> 385, 64
+// keys 249 -> 252), so there one kernel serves both.
+template <int KBW, int NW, int NPW, bool LONG, bool HASZ, int MODE, int PACKED>
 __global__ __launch_bounds__(64 * (NW + NPW)) void Mamba3ChunkKernel(Mamba3SisoParams p, M3Split split) {
     constexpr bool kState = MODE == kM3State;
     using L = M3CLayout<KBW, NW, NPW>;
@@ -307,9 +311,17 @@ __global__ __launch_bounds__(64 * (NW + NPW)) void Mamba3ChunkKernel(Mamba3SisoP
     const int half_n = N / 2;
     const int nrb = (P + ROWS - 1) / ROWS;
     // the nrb workgroups of one (b,h) prepare the same token vectors: keep them on one XCD
-    const int wg = XcdLocalBlock(blockIdx.x, gridDim.x);
-    const int rb = wg % nrb;
+    // (packed sequences: a sequence's heads over all XCDs, XcdSpreadUnit)
+    int wg = XcdLocalBlock(blockIdx.x, gridDim.x);
     const int nseg_wg = MODE == kM3Whole ? 1 : (kState ? (split.maxseg - 1) * (split.ls / split.lf) : split.maxseg);
+    const bool packed = PACKED == 1 || (PACKED == 2 && p.cu_seqlens != nullptr);
+    if (packed) {
+        const XcdUnit u = XcdSpreadUnit(blockIdx.x, nrb);   // units: sequence, segment, head
+        const int run = u.unit / H;
+        if (run >= p.batch * nseg_wg) return;
+        wg = ((run / nseg_wg * H + u.unit % H) * nseg_wg + run % nseg_wg) * nrb + u.part;
+    }
+    const int rb = wg % nrb;
     const int seg = MODE == kM3Whole ? 0 : (wg / nrb) % nseg_wg;   // fine segment (kM3State) or output segment
     const int bh = wg / nrb / nseg_wg;
     const int b = bh / H, h = bh % H;
@@ -321,7 +333,7 @@ __global__ __launch_bounds__(64 * (NW + NPW)) void Mamba3ChunkKernel(Mamba3SisoP
     int T_ = p.seqlen;
     size_t tok0_ = static_cast<size_t>(b) * T_;    // in [B*T] for Q/K/V/Angles/Z
     size_t sbase_ = static_cast<size_t>(bh) * T_;  // in [B*H*T] for ADT/DT/Trap
-    if (p.cu_seqlens != nullptr) {
+    if (packed) {
         const long long lo = min(max(p.cu_seqlens[b], 0LL), static_cast<long long>(p.seqlen));
         const long long hi = min(max(p.cu_seqlens[b + 1], lo), static_cast<long long>(p.seqlen));
         tok0_ = static_cast<size_t>(lo);
@@ -1087,19 +1099,28 @@ __global__ __launch_bounds__(256) void Mamba3SegCombineKernel(Mamba3SisoParams p
     }
 }
 
-template <int KBW, int NW, int NPW, bool LONG, bool HASZ, int MODE>
-void LaunchChunkMode(const Mamba3SisoParams &p, const M3Split &split, hipStream_t stream) {
+template <int KBW, int NW, int NPW, bool LONG, bool HASZ, int MODE, int PACKED>
+void LaunchChunkRows(const Mamba3SisoParams &p, const M3Split &split, hipStream_t stream) {
     using L = M3CLayout<KBW, NW, NPW>;
     const int nseg = MODE == kM3Whole ? 1 : (MODE == kM3State ? (split.maxseg - 1) * (split.ls / split.lf) : split.maxseg);
     constexpr int ROWS = MODE == kM3State ? kStateRows : kRows;
-    const long long blocks = static_cast<long long>(p.batch) * p.nheads * ((p.p + ROWS - 1) / ROWS) * nseg;
+    const int nrb = (p.p + ROWS - 1) / ROWS;
+    const long long units = static_cast<long long>(p.batch) * p.nheads * nseg;
+    const long long blocks = p.cu_seqlens != nullptr ? XcdSpreadBlocks(units, nrb) : units * nrb;
     if (blocks > 2147483647LL) throw Error(XM_ERR_INVALID_ARGUMENT, "Mamba3SisoFn launch exceeds the grid limit");
     constexpr size_t kLds = MODE == kM3State ? L::kStateBytes : L::kBytes;
-    EnsureDynamicLds(reinterpret_cast<const void *>(&Mamba3ChunkKernel<KBW, NW, NPW, LONG, HASZ, MODE>), static_cast<int>(kLds));
+    EnsureDynamicLds(reinterpret_cast<const void *>(&Mamba3ChunkKernel<KBW, NW, NPW, LONG, HASZ, MODE, PACKED>), static_cast<int>(kLds));
     if constexpr (MODE == kM3Whole) XM_NOTE_LAUNCH("Mamba3ChunkKernel", {}, KBW, NW, NPW, LONG);
     else XM_NOTE_LAUNCH("Mamba3ChunkKernel", {}, KBW, NW, NPW, LONG, HASZ, MODE);
-    hipLaunchKernelGGL((Mamba3ChunkKernel<KBW, NW, NPW, LONG, HASZ, MODE>), dim3(static_cast<unsigned>(blocks)), dim3(L::NT),
+    hipLaunchKernelGGL((Mamba3ChunkKernel<KBW, NW, NPW, LONG, HASZ, MODE, PACKED>), dim3(static_cast<unsigned>(blocks)), dim3(L::NT),
                        kLds, stream, p, split);
+}
+
+template <int KBW, int NW, int NPW, bool LONG, bool HASZ, int MODE>
+void LaunchChunkMode(const Mamba3SisoParams &p, const M3Split &split, hipStream_t stream) {
+    if constexpr (HASZ && MODE == kM3Whole) LaunchChunkRows<KBW, NW, NPW, LONG, HASZ, MODE, 2>(p, split, stream);
+    else if (p.cu_seqlens != nullptr) LaunchChunkRows<KBW, NW, NPW, LONG, HASZ, MODE, 1>(p, split, stream);
+    else LaunchChunkRows<KBW, NW, NPW, LONG, HASZ, MODE, 0>(p, split, stream);
 }
 
 template <int KBW, int NW, int NPW>

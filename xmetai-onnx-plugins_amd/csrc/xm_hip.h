@@ -106,5 +106,22 @@ __device__ __forceinline__ int XcdLocalBlock(int x, int n) {
     const int xcd = x % kNumXcds, slot = x / kNumXcds;
     return xcd < rem ? xcd * (per + 1) + slot : rem * (per + 1) + (xcd - rem) * per + slot;
 }
+// For packed sequences, whose lengths differ: logical units of `per`
+// workgroups each, unit u on XCD u % 8, so that consecutive units (the heads of
+// one sequence) spread over the XCDs while a unit's workgroups, which read the
+// same data, share an L2.  A contiguous range per XCD (XcdLocalBlock) gives one
+// XCD a long sequence's heads, two workgroups to a CU, and leaves others idle.
+// The launch has XcdSpreadBlocks(units, per) workgroups; those of a unit >=
+// units have nothing to do.
+struct XcdUnit {
+    int unit, part;   // part: the workgroup within the unit
+};
+__device__ __forceinline__ XcdUnit XcdSpreadUnit(int x, int per) {
+    const int xcd = x % kNumXcds, slot = x / kNumXcds;
+    return {slot / per * kNumXcds + xcd, slot % per};
+}
+inline long long XcdSpreadBlocks(long long units, long long per) {
+    return (units + kNumXcds - 1) / kNumXcds * kNumXcds * per;
+}
 
 }  // namespace xm

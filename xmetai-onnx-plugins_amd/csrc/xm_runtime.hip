@@ -100,11 +100,14 @@ __global__ __launch_bounds__(256) void PackedGapsKernel(float *out, size_t row_f
     const long long L = seqlen;
     auto clampt = [&](long long x) { return min(max(x, 0LL), L); };
     const long long first = clampt(cu[0]), last = clampt(max(cu[n], first));
-    for (long long t = blockIdx.x; t < L; t += gridDim.x) {   // workgroup-uniform
+    // non-decreasing offsets leave the rows before first and from last on: the
+    // usual row has none, and the launch ends here (4.5 us with a test of every
+    // row by 1024 workgroups)
+    const long long rows = monotone ? first + (L - last) : L;
+    for (long long i = blockIdx.x; i < rows; i += gridDim.x) {   // workgroup-uniform
+        const long long t = !monotone || i < first ? i : last + (i - first);
         bool covered = false;
-        if (monotone) {
-            covered = t >= first && t < last;
-        } else {
+        if (!monotone) {
             for (int b = 0; b < n && !covered; ++b) {
                 const long long lo = clampt(cu[b]), hi = clampt(max(cu[b + 1], lo));
                 covered = t >= lo && t < hi;
@@ -118,7 +121,7 @@ __global__ __launch_bounds__(256) void PackedGapsKernel(float *out, size_t row_f
 
 void LaunchPackedGaps(float *out, size_t row_floats, const int64_t *cu, int n, int seqlen, void *stream) {
     if (seqlen <= 0 || row_floats == 0) return;
-    const int blocks = std::min(seqlen, 1024);
+    const int blocks = std::min(seqlen, 256);
     XM_NOTE_LAUNCH("PackedGapsKernel", {}, );
     hipLaunchKernelGGL(PackedGapsKernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0,
                        static_cast<hipStream_t>(stream), out, row_floats, cu, n, seqlen);
