@@ -21,6 +21,7 @@ from __future__ import annotations
 import ctypes
 import math
 import os
+import struct
 from typing import Optional, Sequence
 
 from . import _capi
@@ -138,8 +139,7 @@ def _desc_from_tensor(x) -> _capi.XmTensor:
         return _desc_from_shape((0,))
     if not isinstance(x, torch.Tensor):
         raise TypeError("inputs must be torch tensors or None")
-    elem = {torch.float32: _capi.XM_ELEM_FLOAT, torch.int64: _capi.XM_ELEM_INT64,
-            torch.float16: _capi.XM_ELEM_FLOAT16, torch.bfloat16: _capi.XM_ELEM_BFLOAT16}.get(x.dtype, 0)
+    elem = _elem_types().get(x.dtype, 0)
     if x.numel() > 0:
         if not x.is_cuda:
             raise XmError(XM_ERR_INVALID_ARGUMENT, "inputs must be device tensors")
@@ -148,10 +148,66 @@ def _desc_from_tensor(x) -> _capi.XmTensor:
     return _desc_from_shape(tuple(x.shape), x.data_ptr() if x.numel() > 0 else None, elem)
 
 
+_XM_TENSOR = struct.Struct(f"@P{_capi.XM_MAX_RANK}qii")   # xm_tensor_t: data, shape, rank, elem_type
+assert _XM_TENSOR.size == ctypes.sizeof(_capi.XmTensor)
+_PAD = tuple((0,) * (_capi.XM_MAX_RANK - r) for r in range(_capi.XM_MAX_RANK + 1))
+
+
+def _pack_inputs(inputs) -> bytearray:
+    """The xm_tensor_t array of a call's inputs (what _desc_from_tensor says of
+    each), packed in one buffer: a plain call's host time is mostly descriptors."""
+    elems = _elem_types()
+    size = _XM_TENSOR.size
+    buf = bytearray(size * len(inputs))
+    pos = 0
+    for x in inputs:
+        if x is None:
+            _XM_TENSOR.pack_into(buf, pos, 0, 0, *_PAD[1], 1, _capi.XM_ELEM_FLOAT)
+            pos += size
+            continue
+        try:
+            shape, ptr = x.shape, x.data_ptr()
+        except AttributeError:
+            raise TypeError("inputs must be torch tensors or None") from None
+        rank = len(shape)
+        if rank > _capi.XM_MAX_RANK:
+            raise XmError(XM_ERR_INVALID_ARGUMENT, "tensor rank out of range")
+        if x.numel() > 0:
+            if not x.is_cuda:
+                raise XmError(XM_ERR_INVALID_ARGUMENT, "inputs must be device tensors")
+            if not x.is_contiguous():
+                raise XmError(XM_ERR_INVALID_ARGUMENT, "inputs must be contiguous (row-major)")
+        else:
+            ptr = 0
+        _XM_TENSOR.pack_into(buf, pos, ptr, *shape, *_PAD[rank], rank, elems.get(x.dtype, 0))
+        pos += size
+    return buf
+
+
+_elem_map = None
+
+
+def _elem_types():
+    global _elem_map
+    if _elem_map is None:
+        import torch
+        _elem_map = {torch.float32: _capi.XM_ELEM_FLOAT, torch.int64: _capi.XM_ELEM_INT64,
+                     torch.float16: _capi.XM_ELEM_FLOAT16, torch.bfloat16: _capi.XM_ELEM_BFLOAT16}
+    return _elem_map
+
+
+_defaults = {}   # op -> the bytes of its default attribute block
+
+
 def _attrs(op: str, **kw):
     attrs_t, _ = _capi.OPS[op]
     a = attrs_t()
-    getattr(lib(), f"xm_{op}_attrs_default")(ctypes.byref(a))
+    block = _defaults.get(op)
+    if block is None:
+        getattr(lib(), f"xm_{op}_attrs_default")(ctypes.byref(a))
+        _defaults[op] = bytes(a)
+    else:
+        ctypes.memmove(ctypes.byref(a), block, len(block))
     for k, v in kw.items():
         if v is None:
             continue
@@ -286,41 +342,49 @@ def _run(op: str, inputs, out_like_index: int, allocator: Optional[TorchAllocato
     nothing and returns a :class:`PreparedCall` instead."""
     import torch
     n = len(inputs)
-    descs = [_desc_from_tensor(x) for x in inputs]
-    arr = (_capi.XmTensor * n)(*descs)
+    arr = (_capi.XmTensor * n).from_buffer(_pack_inputs(inputs))
     a = _attrs(op, **attrs)
     err = ctypes.create_string_buffer(512)
-    out_shape = (ctypes.c_int64 * _capi.XM_MAX_RANK)()
-    out_rank = ctypes.c_int32()
-    scratch = ctypes.c_size_t()
-    _check(getattr(lib(), f"xm_{op}_validate")(arr, n, ctypes.byref(a), out_shape, ctypes.byref(out_rank),
-                                               ctypes.byref(scratch), err, len(err)), err)
     ref = inputs[out_like_index]
+    if prepare or ref is None or ref.numel() == 0:
+        # the output shape from the C ABI: a prepared call raises for a bad
+        # shape when it is prepared; a plain one below, in the forward call,
+        # which makes the same checks before it enqueues anything
+        out_shape = (ctypes.c_int64 * _capi.XM_MAX_RANK)()
+        out_rank = ctypes.c_int32()
+        scratch = ctypes.c_size_t()
+        _check(getattr(lib(), f"xm_{op}_validate")(arr, n, ctypes.byref(a), out_shape, ctypes.byref(out_rank),
+                                                   ctypes.byref(scratch), err, len(err)), err)
+        shape = tuple(out_shape[i] for i in range(out_rank.value))
+    else:
+        shape = ref.shape   # every operator's output has the shape of u / v / V
+    device = ref.device
     # SelectiveScanFn's y takes u's element type (fp32, or the 16-bit data types)
     out_dtype = ref.dtype if op == "selective_scan" else torch.float32
-    out = torch.empty(tuple(out_shape[i] for i in range(out_rank.value)), dtype=out_dtype, device=ref.device)
+    out = torch.empty(shape, dtype=out_dtype, device=device)
     if stream is None:
-        stream = torch.cuda.current_stream(ref.device)
+        stream = torch.cuda.current_stream(device)
     alloc_ptr = ctypes.byref(allocator.struct) if allocator is not None else None
-    out_ptr = ctypes.c_void_p(out.data_ptr() if out.numel() else None)
-    stream_ptr = ctypes.c_void_p(stream.cuda_stream)
+    out_ptr = out.data_ptr() if out.numel() else None
+    stream_ptr = stream.cuda_stream
     if state_shapes is None:
         fn = getattr(lib(), f"xm_{op}_forward")
         args = (arr, n, ctypes.byref(a), out_ptr, stream_ptr, alloc_ptr, err, len(err))
         states, result = None, out
     else:
-        states = [torch.empty(tuple(int(d) for d in sh), dtype=torch.float32, device=ref.device)
-                  for sh in state_shapes]
+        states = [torch.empty(tuple(int(d) for d in sh), dtype=torch.float32, device=device) for sh in state_shapes]
         fn = getattr(lib(), f"xm_{op}_forward_states")
-        args = (arr, n, ctypes.byref(a), out_ptr,
-                *(ctypes.c_void_p(x.data_ptr() if x.numel() else None) for x in states),
+        args = (arr, n, ctypes.byref(a), out_ptr, *(x.data_ptr() if x.numel() else None for x in states),
                 stream_ptr, alloc_ptr, err, len(err))
         result = (out, states)
     if prepare:
         keep = (inputs, arr, a, allocator, stream)
-        return PreparedCall(fn, args, err, keep, ref.device.index, out, states, result)
-    with torch.cuda.device(ref.device):
+        return PreparedCall(fn, args, err, keep, device.index, out, states, result)
+    if torch.cuda.current_device() == device.index:
         st = fn(*args)
+    else:
+        with torch.cuda.device(device):
+            st = fn(*args)
     _check(st, err)
     return result
 
