@@ -61,3 +61,20 @@ def test_m3_spread(name, heads, p, has_z):
     want = single_runs(lambda lo, hi: xp.mamba3_siso_fn(*(part(k, lo, hi) for k in keys)).cpu().numpy(), off, total,
                        got.shape)
     check(f"packed_spread/m3_{name}_h{heads}_p{p}_{has_z}", got, want, TOL_GPU)
+
+
+@pytest.mark.parametrize("dk,dv", [(64, 40), (128, 128), (128, 65), (192, 48), (256, 80)])
+@pytest.mark.parametrize("offsets", [[0, 1500, 1540, 1600], [k * 100 for k in range(17)]], ids=["one_long", "even"])
+def test_gdn2_tiles_by_length_equal_both_layouts_bitwise(dk, dv, offsets, override):
+    """The packed recurrence picks one or two column tiles per workgroup from the
+    lengths; either choice gives the bits of the fixed layouts."""
+    s = W.GatedDeltaNet2Shape(1, 1600, 32, dk, dv, initial_state=False)
+    inp = W.gated_deltanet2_inputs(s, seed=53)
+    dev = [to_dev(inp[k]) for k in ("q", "k", "v", "g", "beta", "w")]
+    cu = to_dev(np.asarray(offsets, np.int64))
+    got = xp.gated_deltanet2_fn(*dev, scale=s.scale, cu_seqlens=cu)
+    assert any(k.startswith("Gdn2ChunkRecurKernel<") and k.endswith(",0,1>") for k in xp.last_launches()), xp.last_launches()
+    for ct in (1, 2):
+        override("gdn2_ct", ct)
+        fixed = xp.gated_deltanet2_fn(*dev, scale=s.scale, cu_seqlens=cu)
+        assert np.array_equal(got.cpu().numpy(), fixed.cpu().numpy())

@@ -965,25 +965,13 @@ __device__ __forceinline__ void Gdn2RecurRun(const GatedDeltaNet2Params &p, floa
 // (p.state); one that ends it writes final_state (if requested), any other
 // the carry, in place: a workgroup reads and writes only its own rows and
 // columns.
-template <int KPW, int KS, int CT, bool PACKED>
-__global__ __launch_bounds__(64 * KS) void Gdn2ChunkRecurKernel(GatedDeltaNet2Params p, int c0, int wn,
-                                                                const float *s_in, float *s_out) {
+template <int KPW, int KS, int CT>
+__device__ __forceinline__ void Gdn2PackedRecur(const GatedDeltaNet2Params &p, float *sXp, int c0, int wn, int vw) {
     using L = RecurLayout<KPW, KS, CT>;
-    __shared__ __attribute__((aligned(16))) float sXp[L::kFloats];
-    const int H = p.nheads;
-    const int VW = ((p.dv + 15) / 16 + CT - 1) / CT;   // workgroups per (b, h)
+    const int H = p.nheads, n = p.batch;
     const size_t kv = static_cast<size_t>(p.dk) * p.dv;
-    if constexpr (!PACKED) {
-        const int wg = XcdLocalBlock(blockIdx.x, gridDim.x), row = wg / VW;
-        const int b = row / H, h = row % H;
-        Gdn2RecurRun<KPW, KS, CT>(p, sXp, h, static_cast<size_t>(b) * p.seqlen, p.seqlen, c0, 0, wn, wn,
-                                  p.prepared + static_cast<size_t>(row) * wn * L::FB, static_cast<size_t>(row) * kv,
-                                  s_in, s_out, SplitTile{wg % VW, false, nullptr});
-        return;
-    } else {
-    const int n = p.batch;
     const int slots = min(n, wn);
-    const XcdUnit u = XcdSpreadUnit(blockIdx.x, VW);
+    const XcdUnit u = XcdSpreadUnit(blockIdx.x, vw);
     const int slot = u.unit / H, h = u.unit % H;
     if (slot >= slots) return;
     const float *const prep_row = p.prepared + static_cast<size_t>(h) * wn * L::FB;
@@ -1000,6 +988,50 @@ __global__ __launch_bounds__(64 * KS) void Gdn2ChunkRecurKernel(GatedDeltaNet2Pa
         Gdn2RecurRun<KPW, KS, CT>(p, sXp, h, tok0, T, c0, i0, nrun, wn, prep_row, sbase, in, out,
                                   SplitTile{u.part, false, nullptr});
     }
+}
+
+// One column tile per workgroup (half the work on a long sequence's chain) or
+// two (less work in all), from the window's sequence lengths, which only the
+// device knows; the results are the same bits.  In steps of 0.01 us: a
+// workgroup alone steps one tile in 0.72 and two in 1.2, a full CU one tile in
+// 0.70 and, two at a time, in 0.60 each.  Measured (us, one / two tiles),
+// 128 x 128: 5000 tokens x 16 heads, longest of 7 sequences 1636 188 / 234, even
+// 195 / 178; 4000 x 8 heads in 5 114 / 164; 16384 x 16 in 16, ragged 587 / 573;
+// 64 x 64, 4000 x 16 in 5 104 / 159; 256 x 256, 4000 x 8 in 6 221 / 310.
+constexpr int kCus = 256;
+__device__ __forceinline__ bool PackedTwoTiles(const GatedDeltaNet2Params &p, int vt) {
+    int longest = 0;
+    for (int b = threadIdx.x & 63; b < p.batch; b += 64) longest = max(longest, p.chunk_off[b + 1] - p.chunk_off[b]);
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) longest = max(longest, __shfl_xor(longest, o));
+    const float chain = static_cast<float>(__builtin_amdgcn_readfirstlane(longest));
+    const float work = static_cast<float>(p.chunk_off[p.batch]) * p.nheads * vt / kCus;
+    return fmaxf(120.0f * chain, 60.0f * work) < fmaxf(72.0f * chain, 70.0f * work);
+}
+
+// CT: value-column tiles per workgroup; 0 (packed): one or two, by the lengths
+// (the launch has the one-tile workgroups; two tiles leave the last ones idle).
+template <int KPW, int KS, int CT, bool PACKED>
+__global__ __launch_bounds__(64 * KS) void Gdn2ChunkRecurKernel(GatedDeltaNet2Params p, int c0, int wn,
+                                                                const float *s_in, float *s_out) {
+    using L = RecurLayout<KPW, KS, CT == 0 ? 2 : CT>;
+    __shared__ __attribute__((aligned(16))) float sXp[L::kFloats];
+    const int VT = (p.dv + 15) / 16;
+    if constexpr (!PACKED) {
+        const int H = p.nheads;
+        const int VW = (VT + CT - 1) / CT;   // workgroups per (b, h)
+        const size_t kv = static_cast<size_t>(p.dk) * p.dv;
+        const int wg = XcdLocalBlock(blockIdx.x, gridDim.x), row = wg / VW;
+        const int b = row / H, h = row % H;
+        Gdn2RecurRun<KPW, KS, CT>(p, sXp, h, static_cast<size_t>(b) * p.seqlen, p.seqlen, c0, 0, wn, wn,
+                                  p.prepared + static_cast<size_t>(row) * wn * L::FB, static_cast<size_t>(row) * kv,
+                                  s_in, s_out, SplitTile{wg % VW, false, nullptr});
+    } else if constexpr (CT != 0) {
+        Gdn2PackedRecur<KPW, KS, CT>(p, sXp, c0, wn, (VT + CT - 1) / CT);
+    } else if (PackedTwoTiles(p, VT)) {
+        Gdn2PackedRecur<KPW, KS, 2>(p, sXp, c0, wn, (VT + 1) / 2);
+    } else {
+        Gdn2PackedRecur<KPW, KS, 1>(p, sXp, c0, wn, VT);
     }
 }
 
@@ -1542,7 +1574,10 @@ template <int KPW, int KS, int CT>
 void LaunchRecur(const GatedDeltaNet2Params &p, int c0, int wn, int kq, const float *s_in, float *s_out,
                  hipStream_t stream) {
     if (kq != RecurLayout<KPW, KS, CT>::KQ) throw Error(XM_ERR_DEVICE, "GatedDeltaNet2Fn chunk configuration mismatch");
-    const int vt = ((p.dv + 15) / 16 + CT - 1) / CT;   // workgroups per (b, h)
+    // packed, two tiles by the dispatcher's choice: the kernel looks at the lengths
+    constexpr int PCT = CT == 2 ? 0 : CT;
+    const bool by_length = p.chunk_off != nullptr && CT == 2 && GetOverride(kOverrideGdn2Ct) == 0;
+    const int vt = by_length ? (p.dv + 15) / 16 : ((p.dv + 15) / 16 + CT - 1) / CT;   // workgroups per (b, h)
     // packed: min(sequences, chunks) slots per (h, column tile); a slot's
     // workgroup takes every slots-th sequence that meets the window
     const long long rows = p.chunk_off != nullptr ? std::min(p.batch, wn) : p.batch;
@@ -1552,9 +1587,15 @@ void LaunchRecur(const GatedDeltaNet2Params &p, int c0, int wn, int kq, const fl
     if (p.chunk_off != nullptr) {
         const long long spread = XcdSpreadBlocks(rows * p.nheads, vt);
         if (spread > 2147483647LL) throw Error(XM_ERR_INVALID_ARGUMENT, "GatedDeltaNet2Fn launch exceeds the grid limit");
-        XM_NOTE_LAUNCH("Gdn2ChunkRecurKernel", {}, KPW, KS, CT, 1);
-        hipLaunchKernelGGL((Gdn2ChunkRecurKernel<KPW, KS, CT, true>), dim3(static_cast<unsigned>(spread)),
-                           dim3(64 * KS), 0, stream, p, c0, wn, s_in, s_out);
+        if (by_length) {
+            XM_NOTE_LAUNCH("Gdn2ChunkRecurKernel", {}, KPW, KS, PCT, 1);
+            hipLaunchKernelGGL((Gdn2ChunkRecurKernel<KPW, KS, PCT, true>), dim3(static_cast<unsigned>(spread)),
+                               dim3(64 * KS), 0, stream, p, c0, wn, s_in, s_out);
+        } else {
+            XM_NOTE_LAUNCH("Gdn2ChunkRecurKernel", {}, KPW, KS, CT, 1);
+            hipLaunchKernelGGL((Gdn2ChunkRecurKernel<KPW, KS, CT, true>), dim3(static_cast<unsigned>(spread)),
+                               dim3(64 * KS), 0, stream, p, c0, wn, s_in, s_out);
+        }
     } else {
         XM_NOTE_LAUNCH("Gdn2ChunkRecurKernel", {}, KPW, KS, CT, 0);
         hipLaunchKernelGGL((Gdn2ChunkRecurKernel<KPW, KS, CT, false>), dim3(static_cast<unsigned>(blocks)),
