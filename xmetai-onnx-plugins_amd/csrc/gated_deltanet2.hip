@@ -673,13 +673,14 @@ size_t GatedDeltaNet2ScratchBytes(int batch, int seqlen, int nheads, int dk, int
 }
 
 void LaunchGatedDeltaNet2(GatedDeltaNet2Params p, void *scratch, size_t scratch_bytes, void *stream_v) {
-    // packed: token rows outside every sequence are zeros, not left unwritten
-    if (p.cu_seqlens != nullptr)
-        LaunchPackedGaps(p.out, static_cast<size_t>(p.nheads) * p.dv, p.cu_seqlens, p.batch, p.seqlen, stream_v);
     // a few tokens: gated_deltanet2_step.hip
     if (LaunchGatedDeltaNet2Step(p, stream_v)) return;
     // dk <= 512: gated_deltanet2_chunk.hip (the fused kernel under the gdn2_path override)
     if (LaunchGatedDeltaNet2Chunked(p, scratch, scratch_bytes, stream_v)) return;
+    // packed: token rows outside every sequence are zeros, not left unwritten
+    // (the chunked path's own launches see to that)
+    if (p.cu_seqlens != nullptr)
+        LaunchPackedGaps(p.out, static_cast<size_t>(p.nheads) * p.dv, p.cu_seqlens, p.batch, p.seqlen, stream_v);
     hipStream_t stream = static_cast<hipStream_t>(stream_v);
     if (p.cu_seqlens != nullptr && p.dk > kFusedKeyLimit)
         throw Error(XM_ERR_UNSUPPORTED, "GatedDeltaNet2Fn with cu_seqlens supports headdim_k up to 512");

@@ -94,6 +94,41 @@ __device__ __forceinline__ void LoadKeys(const float *src, float (&x)[KT]) {
     }
 }
 
+// Packed sequences: zeros the token rows of `out` ([seqlen][row_floats]) that
+// no sequence covers, the part of workgroup wg of nwg (every thread of the
+// workgroup calls it).  Sequence b covers [lo_b, hi_b), lo_b = clamp(cu[b]),
+// hi_b = clamp(max(cu[b + 1], lo_b)), the ranges the operator kernels use;
+// non-decreasing offsets cover exactly [lo_0, hi_{n-1}), so only the rows before
+// and after are visited (the usual row has none); other offsets are checked
+// sequence by sequence (malformed input: time linear in n per row).
+__device__ __forceinline__ void ZeroPackedGaps(float *out, size_t row_floats, const int64_t *cu, int n, int seqlen,
+                                               int wg, int nwg) {
+    __shared__ int s_monotone;
+    if (threadIdx.x == 0) s_monotone = 1;
+    __syncthreads();
+    bool mono = true;
+    for (int b = threadIdx.x; b < n; b += blockDim.x) mono = mono && cu[b] <= cu[b + 1];
+    if (!mono) s_monotone = 0;
+    __syncthreads();
+    const bool monotone = s_monotone != 0;
+    const long long L = seqlen;
+    auto clampt = [&](long long x) { return min(max(x, 0LL), L); };
+    const long long first = clampt(cu[0]), last = clampt(max(cu[n], first));
+    const long long rows = monotone ? first + (L - last) : L;
+    for (long long i = wg; i < rows; i += nwg) {   // workgroup-uniform
+        const long long t = !monotone || i < first ? i : last + (i - first);
+        bool covered = false;
+        if (!monotone) {
+            for (int b = 0; b < n && !covered; ++b) {
+                const long long lo = clampt(cu[b]), hi = clampt(max(cu[b + 1], lo));
+                covered = t >= lo && t < hi;
+            }
+        }
+        if (!covered)
+            for (size_t f = threadIdx.x; f < row_floats; f += blockDim.x) out[static_cast<size_t>(t) * row_floats + f] = 0.0f;
+    }
+}
+
 // MI355X deals the workgroups of a launch round-robin to its 8 XCDs
 // (workgroup x runs on XCD x % 8), and each XCD has its own L2.  This maps
 // the hardware index to a logical one under which XCD j owns one contiguous
