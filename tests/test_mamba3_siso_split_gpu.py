@@ -80,9 +80,11 @@ def test_split_parity(name, start, override):
     compare(f"{name}/vs_whole", (y, *f), [x.cpu().numpy() for x in (y1, *f1)], TOL_GPU)
 
 
-@pytest.mark.parametrize("offsets", [[0, 700, 1400], [0, 40, 41, 1400], [0, 0, 600, 600, 1400], [3, 500, 1390]])
+@pytest.mark.parametrize("offsets", [[0, 700, 1400], [0, 40, 41, 1400], [0, 0, 600, 600, 1400], [3, 500, 1390], [0, 600, 20, 20]])
 @pytest.mark.parametrize("start", [True, False])
 def test_split_packed(offsets, start, override):
+    """Also offsets that fall: [0, 600), nothing, nothing (the device sees that
+    they do not rise and keeps the sequences whole)."""
     s = S(1, 1400, 2, 64, 128, has_z=True)
     inp = W.mamba3_siso_inputs(s, seed=43)
     n = len(offsets) - 1
@@ -149,3 +151,18 @@ def test_output_over_an_input_is_not_split(override):
     assert not split_launched()
     torch.cuda.synchronize()
     check("mamba3_siso_split/in_place", dev[2].cpu().numpy(), want.cpu().numpy(), TOL_GPU)
+
+
+def test_overlapping_packed_sequences_keep_their_states(override):
+    """Falling offsets may give two sequences the same rows ([0, 900) and [300,
+    1400) here); their final states are those of the whole pass."""
+    s = S(1, 1400, 2, 64, 128)
+    inp = W.mamba3_siso_inputs(s, seed=48)
+    cu = to_dev(np.asarray([0, 900, 300, 1400], np.int64))
+    out = []
+    for mode in (2, 1):
+        override("m3_split", mode)
+        y, f = xp.mamba3_siso_fn(*(to_dev(inp[k]) for k in KEYS), return_final_states=True, cu_seqlens=cu)
+        out.append([x.cpu().numpy() for x in f])
+    for part, a, b in zip(PARTS[1:], *out):
+        np.testing.assert_array_equal(a, b, err_msg=part)

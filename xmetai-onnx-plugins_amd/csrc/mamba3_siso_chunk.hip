@@ -275,6 +275,18 @@ __device__ __forceinline__ M3Range RangeOf(const Mamba3SisoParams &p, int b) {
     return {static_cast<size_t>(lo), static_cast<int>(hi - lo)};
 }
 
+// Output segments of a sequence of T tokens in this call.  Packed offsets that
+// do not rise can give two sequences the same output rows, and so the same
+// records: such a call is not split.  (Every lane of the wave calls it.)
+__device__ __forceinline__ int SegmentsOf(const Mamba3SisoParams &p, const M3Split &split, int T) {
+    if (p.cu_seqlens != nullptr) {
+        bool rises = true;
+        for (int b = threadIdx.x & 63; b < p.batch; b += 64) rises = rises && p.cu_seqlens[b] <= p.cu_seqlens[b + 1];
+        if (__ballot(!rises) != 0) return 1;
+    }
+    return split.Segments(T);
+}
+
 // LONG: some tensor's token rows of one sequence span 2 GiB or more, beyond a
 // buffer descriptor's 32-bit range; every chunk then reads and writes through
 // descriptors that start at its own first token.
@@ -349,7 +361,7 @@ __global__ __launch_bounds__(64 * (NW + NPW)) void Mamba3ChunkKernel(Mamba3SisoP
     int cs = 0, te = T;
     bool last_seg = true;
     if constexpr (MODE != kM3Whole) {
-        const int nseg = split.Segments(T);
+        const int nseg = SegmentsOf(p, split, T);
         if constexpr (kState) {
             cs = seg * split.lf;
             te = cs + split.lf;
@@ -1042,7 +1054,7 @@ __global__ __launch_bounds__(256) void Mamba3SegCombineKernel(Mamba3SisoParams p
     const int blk = blockIdx.x % blocks, rb = blockIdx.x / blocks % nrb, bh = blockIdx.x / blocks / nrb;
     const int b = bh / H, h = bh % H;
     const M3Range r = RangeOf(p, b);
-    const int m = split.ls / split.lf, nf = (split.Segments(r.T) - 1) * m;   // fine segments that another follows
+    const int m = split.ls / split.lf, nf = (SegmentsOf(p, split, r.T) - 1) * m;   // fine segments that another follows
     const int q = blk * 256 + threadIdx.x;
     auto record = [&](int f) { return RecordAt(p, r.tok0 + static_cast<size_t>(f) * split.lf, h, rb * kRows, np); };
     const M3Record r0 = record(0);
