@@ -103,7 +103,8 @@ int xm_selective_scan_check_attrs(const xm_selective_scan_attrs_t *attrs, char *
 /* Run-time shape validation without touching the device (reference:
  * Compute, :58-117).  Writes the output shape and the scratch bytes the call
  * will request from the allocator (GatedDeltaNet2Fn: at most; a call of up to
- * 16 tokens requests none). */
+ * 16 tokens requests none, unless an output shares memory with q, k, g or beta
+ * or overlaps v or w out of place). */
 int xm_selective_scan_validate(const xm_tensor_t *inputs, size_t n_inputs,
                                const xm_selective_scan_attrs_t *attrs, int64_t *out_shape,
                                int32_t *out_rank, size_t *scratch_bytes, char *errbuf, size_t errlen);

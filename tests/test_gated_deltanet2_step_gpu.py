@@ -2,7 +2,8 @@
 registers in one launch) on the GPU vs the fp64 oracle: every key tiling at its
 edges, value columns cut by a group of four or by a column block, both column
 block widths, one to sixteen tokens (prepared four at a time), with and without
-states, the L2 norm and an in-place state; 17 tokens take the chunked path."""
+states, the L2 norm and an in-place state; 17 tokens and outputs over an input
+that several column blocks read take the chunked path."""
 
 import numpy as np
 import pytest
@@ -73,20 +74,72 @@ def test_step_agrees_with_the_chunked_path(override):
     check("gated_deltanet2_step/vs_chunked/s", f, fc, TOL_GPU)
 
 
-def test_step_state_in_place():
-    """A decode loop may keep one state buffer: final_state over initial_state."""
+def call_states(dev, s, out_ptr, state_ptr):
+    """xm_gated_deltanet2_forward_states on device tensors, outputs at the given addresses."""
     import ctypes
     import torch
     from xmetai_onnx_plugins import _capi
+    arr = (_capi.XmTensor * 7)(*[xp._desc_from_tensor(x) for x in dev])
+    attrs = xp._attrs("gated_deltanet2", scale=s.scale, output_final_state=1)
+    err = ctypes.create_string_buffer(256)
+    st = xp.lib().xm_gated_deltanet2_forward_states(arr, 7, ctypes.byref(attrs), out_ptr, state_ptr,
+                                                    torch.cuda.current_stream().cuda_stream, None, err, len(err))
+    assert st == xp.XM_OK, err.value
+    torch.cuda.synchronize()
+
+
+def test_step_state_in_place():
+    """A decode loop may keep one state buffer: final_state over initial_state."""
+    import torch
     s = S(2, 2, 4, 128, 64)
     inp = W.gated_deltanet2_inputs(s, seed=4)
     dev = [to_dev(inp[k]) for k in KEYS]
     o, f = xp.gated_deltanet2_fn(*dev, scale=s.scale, output_final_state=True)
-    arr = (_capi.XmTensor * 7)(*[xp._desc_from_tensor(x) for x in dev])
-    attrs = xp._attrs("gated_deltanet2", scale=s.scale, output_final_state=1)
-    err, out = ctypes.create_string_buffer(256), torch.empty_like(o)
-    st = xp.lib().xm_gated_deltanet2_forward_states(arr, 7, ctypes.byref(attrs), out.data_ptr(), dev[6].data_ptr(),
-                                                    torch.cuda.current_stream().cuda_stream, None, err, len(err))
-    assert st == xp.XM_OK, err.value
-    torch.cuda.synchronize()
+    out = torch.empty_like(o)
+    call_states(dev, s, out.data_ptr(), dev[6].data_ptr())
     assert torch.equal(out, o) and torch.equal(dev[6], f)
+
+
+@pytest.mark.parametrize("tokens", [1, 6])
+@pytest.mark.parametrize("key", KEYS[:6])
+def test_outputs_over_an_input(key, tokens):
+    """out over q, k, g or beta, which every column block of a head reads whole:
+    the chunked path, which has read them before it writes; over v or w, which a
+    block reads only in its own columns: still one launch."""
+    import torch
+    s = S(3, tokens, 8, 128, 128)
+    inp = W.gated_deltanet2_inputs(s, seed=6)
+    dev = [to_dev(inp[k]) for k in KEYS]
+    o, f = xp.gated_deltanet2_fn(*dev, scale=s.scale, output_final_state=True)
+    assert step_launched(32)
+    state, at = torch.empty_like(f), KEYS.index(key)
+    call_states(dev, s, dev[at].data_ptr(), state.data_ptr())
+    assert step_launched(32) == (key in ("v", "w")), xp.last_launches()
+    assert xp.last_launches()[-1].startswith(("Gdn2StepKernel<", "Gdn2ChunkRecurKernel<")), xp.last_launches()
+    check(f"gated_deltanet2_step/over_{key}_t{tokens}/o", dev[at].cpu().numpy(), o.cpu().numpy(), TOL_GPU)
+    check(f"gated_deltanet2_step/over_{key}_t{tokens}/s", state.cpu().numpy(), f.cpu().numpy(), TOL_GPU)
+
+
+def test_outputs_over_a_part_of_an_input():
+    """out one token row behind v; final_state over the end of g."""
+    import torch
+    s = S(1, 5, 4, 64, 64)
+    inp = W.gated_deltanet2_inputs(s, seed=7)
+    dev = [to_dev(inp[k]) for k in KEYS]
+    o, f = xp.gated_deltanet2_fn(*dev, scale=s.scale, output_final_state=True)
+    row = s.nheads * s.dv
+    buf = torch.empty(o.numel() + row, device="cuda")
+    v = buf[row:].view(o.shape)
+    v.copy_(dev[2])
+    state = torch.empty_like(f)
+    call_states([*dev[:2], v, *dev[3:]], s, buf.data_ptr(), state.data_ptr())
+    assert not step_launched(32), xp.last_launches()
+    check("gated_deltanet2_step/behind_v/o", buf[:-row].view(o.shape).cpu().numpy(), o.cpu().numpy(), TOL_GPU)
+    check("gated_deltanet2_step/behind_v/s", state.cpu().numpy(), f.cpu().numpy(), TOL_GPU)
+    n = dev[3].numel()
+    buf = torch.empty(n + f.numel() - 64, device="cuda")
+    g = buf[:n].view(dev[3].shape)
+    g.copy_(dev[3])
+    call_states([*dev[:3], g, *dev[4:]], s, torch.empty_like(o).data_ptr(), buf[n - 64:].data_ptr())
+    assert not step_launched(32), xp.last_launches()
+    check("gated_deltanet2_step/over_g/s", buf[n - 64:].view(f.shape).cpu().numpy(), f.cpu().numpy(), TOL_GPU)

@@ -106,7 +106,7 @@ void Forward(const xm_tensor_t *inputs, size_t n_inputs, const xm_gated_deltanet
     const GatedDeltaNet2Params p = GatedDeltaNet2Plan(inputs, n_inputs, attrs, out, final_state);
     const bool packed = p.cu_seqlens != nullptr;
     // a few tokens need no scratch (validation still reports the chunked path's)
-    const bool step = GatedDeltaNet2StepFits(p.batch, p.seqlen, p.nheads, p.dk, p.dv, packed);
+    const bool step = GatedDeltaNet2StepFits(p);
     size_t bytes = step ? 0 : GatedDeltaNet2ScratchBytes(p.batch, p.seqlen, p.nheads, p.dk, p.dv, packed);
     Scratch scratch(alloc, stream);
     void *buf = scratch.TryGet(bytes);

@@ -87,8 +87,7 @@ extern "C" int xm_gated_deltanet2_forward_noalloc(const xm_tensor_t *inputs, siz
                             "GatedDeltaNet2Fn (xm_gated_deltanet2_forward_noalloc): the call needs more than the " +
                                 std::to_string(xm::kNoAllocScratchBytes >> 20) +
                                 " MiB of device scratch this entry point holds; use xm_gated_deltanet2_forward");
-        if (need == 0 || xm::GatedDeltaNet2StepFits(p.batch, p.seqlen, p.nheads, p.dk, p.dv,
-                                                    p.cu_seqlens != nullptr)) {   // nothing touches the array
+        if (need == 0 || xm::GatedDeltaNet2StepFits(p)) {   // nothing touches the array
             xm::LaunchGatedDeltaNet2(p, nullptr, 0, stream);
             return;
         }

@@ -234,10 +234,21 @@ void LaunchStepKeys(const GatedDeltaNet2Params &p, hipStream_t stream) {
 
 }  // namespace
 
-bool GatedDeltaNet2StepFits(int batch, int seqlen, int nheads, int dk, int dv, bool packed) {
-    if (packed || batch < 1 || seqlen < 1 || seqlen > kGdn2StepTokens || nheads < 1 || dk < 1 ||
-        dk > kGdn2ChunkKeyLimit || dv < 1 || static_cast<long long>(dk) * dv * 4 >= (1LL << 31))
+bool GatedDeltaNet2StepFits(const GatedDeltaNet2Params &p) {
+    if (p.cu_seqlens != nullptr || p.batch < 1 || p.seqlen < 1 || p.seqlen > kGdn2StepTokens || p.nheads < 1 || p.dk < 1 ||
+        p.dk > kGdn2ChunkKeyLimit || p.dv < 1 || static_cast<long long>(p.dk) * p.dv * 4 >= (1LL << 31))
         return false;
+    // Every column block of a (b,h) reads the tokens' whole q, k, g and beta
+    // rows: an output over them may change what another block has yet to read.
+    // The chunked path has read them all before it writes anything.  A block
+    // reads v and w of its own columns token by token, so the output may be v or
+    // w itself, but not a shifted part of them.
+    const size_t rows = static_cast<size_t>(p.batch) * p.seqlen * p.nheads * sizeof(float);
+    const size_t keys = rows * p.dk, cols = rows * p.dv, state = static_cast<size_t>(p.batch) * p.nheads * p.dk * p.dv * sizeof(float);
+    if (AnyOverlap({{p.out, cols}, {p.final_state, state}}, {{p.q, keys}, {p.k, keys}, {p.g, keys}, {p.beta, keys}}))
+        return false;
+    for (const float *x : {p.v, p.w})
+        if (p.out != x && Overlap({p.out, cols}, {x, cols})) return false;
     for (Override o : {kOverrideGdn2Path, kOverrideGdn2Pairwise, kOverrideGdn2Kpw4, kOverrideGdn2Windowed,
                        kOverrideGdn2Split, kOverrideGdn2Ct})
         if (GetOverride(o) != 0) return false;   // a variant of another path is asked for
@@ -245,7 +256,7 @@ bool GatedDeltaNet2StepFits(int batch, int seqlen, int nheads, int dk, int dv, b
 }
 
 bool LaunchGatedDeltaNet2Step(const GatedDeltaNet2Params &p, void *stream_v) {
-    if (!GatedDeltaNet2StepFits(p.batch, p.seqlen, p.nheads, p.dk, p.dv, p.cu_seqlens != nullptr)) return false;
+    if (!GatedDeltaNet2StepFits(p)) return false;
     hipStream_t stream = static_cast<hipStream_t>(stream_v);
     const long long wide = static_cast<long long>(p.batch) * p.nheads * ((p.dv + 63) / 64);
     if (wide >= kStepWideBlocks) LaunchStepKeys<16>(p, stream);

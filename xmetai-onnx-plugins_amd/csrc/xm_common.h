@@ -135,6 +135,24 @@ int Guard(char *errbuf, size_t errlen, Fn &&fn) {
     }
 }
 
+// The bytes of a tensor (nullptr: none), to see where an output shares memory
+// with an input: C callers may compute in place, so a kernel whose workgroups
+// read what another one of the same launch writes must not be given such a call.
+struct MemRange {
+    const void *ptr;
+    size_t bytes;
+};
+inline bool Overlap(const MemRange &x, const MemRange &y) {
+    const uintptr_t a = reinterpret_cast<uintptr_t>(x.ptr), b = reinterpret_cast<uintptr_t>(y.ptr);
+    return x.ptr != nullptr && y.ptr != nullptr && a < b + y.bytes && b < a + x.bytes;
+}
+inline bool AnyOverlap(std::initializer_list<MemRange> xs, std::initializer_list<MemRange> ys) {
+    for (const MemRange &x : xs)
+        for (const MemRange &y : ys)
+            if (Overlap(x, y)) return true;
+    return false;
+}
+
 // Kernel-selection overrides, set through xm_set_kernel_override (tests and
 // tuning); 0 everywhere means the dispatchers' own choice.  Read with one
 // relaxed atomic load per launch.

@@ -103,8 +103,8 @@ size_t GatedDeltaNet2ScratchBytes(int batch, int seqlen, int nheads, int dk, int
 // GatedDeltaNet2ScratchBytes chose for cap = scratch_bytes.
 void LaunchGatedDeltaNet2(GatedDeltaNet2Params p, void *scratch, size_t scratch_bytes, void *stream);
 // A few tokens (gated_deltanet2_step.hip): unpacked, seqlen up to
-// kGdn2StepTokens, dk <= kGdn2ChunkKeyLimit, no override that asks for a
-// variant of another path.  No scratch.  Launch: false, launching nothing,
+// kGdn2StepTokens, dk <= kGdn2ChunkKeyLimit, no output over q, k, g or beta, no
+// override that asks for a variant of another path.  No scratch.  Launch: false, launching nothing,
 // when it does not fit.  The limit is one chunk of the chunked path, whose
 // time does not depend on how full the chunk is; at 16 tokens the step kernel
 // is still ahead everywhere measured (us, chunked / step: 32 x 16 heads at
@@ -112,7 +112,7 @@ void LaunchGatedDeltaNet2(GatedDeltaNet2Params p, void *scratch, size_t scratch_
 // 29.0 / 19.1, 64 x 16 heads at 64 x 64 33.8 / 27.3), and grows by 1 to 1.5 us
 // a token where a second chunk costs the chunked path about 1.
 constexpr int kGdn2StepTokens = 16;
-bool GatedDeltaNet2StepFits(int batch, int seqlen, int nheads, int dk, int dv, bool packed);
+bool GatedDeltaNet2StepFits(const GatedDeltaNet2Params &p);
 bool LaunchGatedDeltaNet2Step(const GatedDeltaNet2Params &p, void *stream);
 // Chunked fp32-MFMA path (dk <= kGdn2ChunkKeyLimit).  Returns false, launching nothing, when
 // the shape is not one it takes (or the gdn2_path override asks for the sequential kernel).  `scratch` holds
