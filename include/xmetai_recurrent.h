@@ -172,6 +172,11 @@ int xm_mamba3_siso_forward(const xm_tensor_t *inputs, size_t n_inputs,
  * after the last token to device buffers ssm_state [B,H,P,N], angle_state
  * [B,H,A], k_state [B,H,N] and v_state [B,H,P] (the layouts inputs 11-14
  * take).  The buffers are ignored (may be NULL) when return_final_states == 0.
+ * With N up to 256 each may be the input state's own buffer (a decode loop that
+ * keeps one) where one workgroup owns a head: P up to 32, and P up to 64 for
+ * calls of up to 16 tokens without cu_seqlens.  With a larger P ssm_state and
+ * v_state still may, but angle_state and k_state need buffers apart from inputs
+ * 12 and 13, which every workgroup of a head reads.
  * A widening with no counterpart in the reference (mamba3_siso_fn_ort.cpp:50-52). */
 int xm_mamba3_siso_forward_states(const xm_tensor_t *inputs, size_t n_inputs,
                                   const xm_mamba3_siso_attrs_t *attrs, float *out, float *ssm_state,

@@ -3,7 +3,8 @@ in one launch) on the GPU vs the fp64 oracle: key counts at the edges of the
 64-key groups and of a four-key group, state rows cut by a row block, the three
 row-block heights, one to sixteen tokens (prepared four at a time), angles of
 some pairs, Q/K heads shared, with and without Z, D, input and final states,
-and agreement with the chunked kernel."""
+agreement with the chunked kernel, and outputs over inputs: final states over the
+input states (one row block a head), y over V, Z, Q and a part of V."""
 
 import numpy as np
 import pytest
@@ -93,3 +94,73 @@ def test_step_agrees_with_the_chunked_kernel(override):
     chunked, _ = run(s, seed=5)
     assert xp.last_launches() == ["Mamba3ChunkKernel<2,4,8,0>"], xp.last_launches()
     compare("vs_chunked", got, [x.cpu().numpy() for x in chunked], TOL_GPU)
+
+
+def call_states(dev, states, outs):
+    """xm_mamba3_siso_forward_states on device tensors; outs: y and the four states."""
+    import ctypes
+    import torch
+    from xmetai_onnx_plugins import _capi
+    ins = [*dev, *states]
+    arr = (_capi.XmTensor * len(ins))(*[xp._desc_from_tensor(x) for x in ins])
+    attrs = xp._attrs("mamba3_siso", has_d=1, has_z=int(dev[10] is not None), return_final_states=1, has_input_states=1)
+    err = ctypes.create_string_buffer(256)
+    st = xp.lib().xm_mamba3_siso_forward_states(arr, len(ins), ctypes.byref(attrs), *(x.data_ptr() for x in outs),
+                                                torch.cuda.current_stream().cuda_stream, None, err, len(err))
+    assert st == xp.XM_OK, err.value
+    torch.cuda.synchronize()
+
+
+def sharing_case(s, seed):
+    """Inputs and input states on the device, and the call's results in buffers of their own."""
+    import torch
+    inp = W.mamba3_siso_inputs(s, seed=seed)
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    states = [torch.randn((s.batch, s.nheads, *d), generator=g, device="cuda")
+              for d in ((s.headdim, s.dstate), (s.a,), (s.dstate,), (s.headdim,))]
+    states[1] = states[1].abs()
+    dev = [to_dev(inp[k]) for k in KEYS]
+    y, f = xp.mamba3_siso_fn(*dev, return_final_states=True, input_states=tuple(states))
+    return dev, states, [y, *f]
+
+
+@pytest.mark.parametrize("tokens", [1, 6, 16])
+@pytest.mark.parametrize("p,heads,rows", [(8, 4, 16), (32, 4, 32), (33, 4, 64), (64, 4, 64), (64, 80, 64), (96, 4, 0)])
+def test_step_states_in_place(p, heads, rows, tokens):
+    """A decode loop may keep one set of state buffers.  Row block 0 writes the k
+    and angle states that every row block of a head reads, so a head is one block
+    up to 64 rows, and the call the chunked kernel's above (there only ssm and v in place)."""
+    import torch
+    dev, states, want = sharing_case(S(2, tokens, heads, p, 128, angles=40, has_z=True), seed=p + tokens)
+    if p <= 64:
+        outs = [torch.empty_like(want[0]), *states]
+        call_states(dev, states, outs)
+        # 16 tokens of few blocks are the chunked kernel's, whose workgroups of 32 rows own a head of up to 32
+        chunked = tokens > 8 and p <= 32
+        assert step_rows() == (0 if chunked else rows), xp.last_launches()
+    else:
+        outs = [torch.empty_like(want[0]), states[0], want[2].clone(), want[3].clone(), states[3]]
+        call_states(dev, states, outs)
+        assert (step_rows() == 16) == (tokens <= 8), xp.last_launches()
+    compare(f"in_place_p{p}_h{heads}_t{tokens}", outs, [x.cpu().numpy() for x in want], TOL_GPU)
+
+
+@pytest.mark.parametrize("tokens", [1, 4, 6])
+@pytest.mark.parametrize("over", ["V", "Z", "Q", "behind_V"])
+def test_y_over_an_input(over, tokens):
+    """y over V or Z, which a block reads only in its own rows and tokens: as ever;
+    over Q, or a part of V: only while a call's tokens are read at once (four)."""
+    import torch
+    dev, states, want = sharing_case(S(2, tokens, 3, 32, 32, has_z=True), seed=tokens)
+    n, row = want[0].numel(), want[0][0, 0].numel()
+    if over == "behind_V":   # y one token row before V
+        buf = torch.empty(n + row, device="cuda")
+        y, v = buf[:n].view(want[0].shape), buf[row:].view(want[0].shape)
+        v.copy_(dev[2])
+        dev[2] = v
+    else:
+        y = dev[KEYS.index(over)]
+    outs = [y, *(torch.empty_like(x) for x in want[1:])]
+    call_states(dev, states, outs)
+    assert step_rows() == (0 if over in ("Q", "behind_V") and tokens > 4 else 32 if over == "Q" else 16), xp.last_launches()
+    compare(f"y_over_{over}_t{tokens}", outs, [x.cpu().numpy() for x in want], TOL_GPU)

@@ -1,0 +1,70 @@
+"""Which kernel a call takes where an output shares memory with an input, read
+from xm_last_launches without a GPU: the addresses are made up and nothing runs
+(so the file skips itself where a GPU is visible).  The runs on the GPU, for
+the cases whose result does not depend on the order of the workgroups, are in the
+operators' GPU tests."""
+
+import ctypes
+
+import pytest
+
+import xmetai_onnx_plugins as xp
+from xmetai_onnx_plugins import _capi
+
+
+@pytest.fixture(autouse=True)
+def _no_gpu():
+    import torch
+    if torch.cuda.is_available():
+        pytest.skip("made-up addresses: only where no kernel can run")
+
+
+def launches(op, shapes, outs, at=(), **attrs):
+    """Kernels that xm_<op>_forward_states enqueues for inputs of these shapes
+    (None: absent) at 1 GiB steps, in order, and then the outputs; `at`: output
+    index -> (input index, byte offset) for an output placed over an input."""
+    addr = [(i + 1) << 30 for i in range(len(shapes) + outs)]
+    ins = (_capi.XmTensor * len(shapes))(*[xp._desc_from_shape(sh, a) if sh is not None else xp._desc_from_tensor(None)
+                                           for sh, a in zip(shapes, addr)])
+    out = addr[len(shapes):]
+    for o, (i, off) in dict(at).items():
+        out[o] = addr[i] + off
+    a, err = xp._attrs(op, **attrs), ctypes.create_string_buffer(512)
+    getattr(xp.lib(), f"xm_{op}_forward_states")(ins, len(shapes), ctypes.byref(a), *out, None, None, err, len(err))
+    return [k.split("<")[0] for k in xp.last_launches()]
+
+
+def m3_launches(b, t, h, p, n, a, at=()):
+    qk, th, hn = (b, t, h, n), (b, h, t), (h, n)
+    shapes = [qk, qk, (b, t, h, p), th, th, th, hn, hn, (b, t, h, a), (h,), None, (b, h, p, n), (b, h, a), (b, h, n),
+              (b, h, p)]
+    return launches("mamba3_siso", shapes, 5, at, has_d=1, has_z=0, return_final_states=1, has_input_states=1)
+
+
+STEP = ["Mamba3StepKernel"]
+
+
+@pytest.mark.parametrize("t", [1, 4])
+@pytest.mark.parametrize("at,one_block", [
+    ({}, False),
+    ({1: (11, 0)}, False), ({4: (14, 0)}, False),   # ssm and v in place: a row block's own
+    ({2: (12, 0)}, True), ({3: (13, 0)}, True),     # angle and k in place
+    ({3: (13, 508)}, True), ({3: (13, 512)}, False),   # k over the last value of k, and just behind
+    ({3: (1, 0)}, True), ({2: (8, 4)}, True), ({0: (0, 0)}, True), ({1: (9, 0)}, True), ({4: (6, 0)}, True),
+], ids=str)
+def test_m3_step_with_outputs_over_inputs(at, one_block, t):
+    """An output over what all row blocks of a head read: one row block, or (above 64 rows) not this kernel."""
+    for p in (16, 32, 64):
+        got = m3_launches(1, t, 1, p, 128, 40, at)
+        assert got == STEP
+        rows = 16 * int(xp.last_launches()[0][:-1].split(",")[1])
+        assert rows >= p if one_block else rows == 16
+    assert (m3_launches(1, t, 1, 65, 128, 40, at) == STEP) == (not one_block)
+
+
+def test_m3_step_reads_its_tokens_four_at_a_time():
+    row = 32 * 4
+    for t, ok in ((4, True), (5, False)):
+        assert (m3_launches(1, t, 1, 32, 32, 16, {0: (2, row)}) == STEP) == ok    # y one token behind V
+        assert (m3_launches(1, t, 1, 32, 32, 16, {0: (0, 0)}) == STEP) == ok      # y over Q
+        assert m3_launches(1, t, 1, 32, 32, 16, {0: (2, 0)}) == STEP              # y over V

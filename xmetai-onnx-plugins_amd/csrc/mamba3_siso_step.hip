@@ -290,6 +290,25 @@ void LaunchStepKeys(const Mamba3SisoParams &p, hipStream_t stream) {
     else LaunchStep<4, RP>(p, stream);
 }
 
+// Where an output shares memory with an input.
+struct OutputSharing {
+    bool with_head;   // with an input that every row block of a head reads
+    bool out_moves;   // the y rows with those, or with another place of V or Z
+};
+OutputSharing SharesOf(const Mamba3SisoParams &p) {
+    const size_t f = sizeof(float), rows = static_cast<size_t>(p.batch) * p.seqlen;
+    const size_t bh = static_cast<size_t>(p.batch) * p.nheads * f, th = rows * p.nheads * f, h = static_cast<size_t>(p.nheads) * f;
+    const size_t qk = rows * p.nheads_qk * p.n * f;
+    const MemRange out{p.out, th * p.p};
+    const std::initializer_list<MemRange> head = {
+        {p.Q, qk}, {p.K, qk}, {p.Angles, th * p.a}, {p.ADT, th}, {p.DT, th}, {p.Trap, th}, {p.Q_bias, h * p.n},
+        {p.K_bias, h * p.n}, {p.D, h}, {p.in_angle, bh * p.a}, {p.in_k, bh * p.n}};
+    OutputSharing s{AnyOverlap({out, {p.f_ssm, bh * p.p * p.n}, {p.f_angle, bh * p.a}, {p.f_k, bh * p.n}, {p.f_v, bh * p.p}}, head),
+                    AnyOverlap({out}, head)};
+    for (const float *x : {p.V, p.Z}) s.out_moves = s.out_moves || (p.out != x && Overlap(out, {x, th * p.p}));
+    return s;
+}
+
 }  // namespace
 
 bool LaunchMamba3SisoStep(const Mamba3SisoParams &p, void *stream_v) {
@@ -299,11 +318,19 @@ bool LaunchMamba3SisoStep(const Mamba3SisoParams &p, void *stream_v) {
                   static_cast<long long>(p.nheads) * p.p}) * 4 * (p.seqlen + kTB) >= (1LL << 31) ||
         GetOverride(kOverrideM3Path) != 0)
         return false;
+    const OutputSharing shares = SharesOf(p);
+    // A block takes its tokens kTB at a time: what it writes of the first ones
+    // must not be an input of later ones.
+    if (shares.out_moves && p.seqlen > kTB) return false;
+    // Above 64 rows a head has several row blocks: none may write what another
+    // has yet to read (final states over the input states, for instance).
+    if (shares.with_head && p.p > 64) return false;
+    const int one_block = shares.with_head ? p.p : 0;   // rows that must be one block's
     const long long tall = static_cast<long long>(p.batch) * p.nheads * ((p.p + 63) / 64);
-    if (p.seqlen > kM3StepTokens / 2 && tall < kBlocksAllTokens) return false;
+    if (p.seqlen > kM3StepTokens / 2 && tall < kBlocksAllTokens && one_block <= 32) return false;
     hipStream_t stream = static_cast<hipStream_t>(stream_v);
-    if (tall >= kBlocks64) LaunchStepKeys<4>(p, stream);
-    else if (tall >= kBlocks32) LaunchStepKeys<2>(p, stream);
+    if (tall >= kBlocks64 || one_block > 32) LaunchStepKeys<4>(p, stream);
+    else if (tall >= kBlocks32 || one_block > 16) LaunchStepKeys<2>(p, stream);
     else LaunchStepKeys<1>(p, stream);
     XM_LAUNCH_CHECK("Mamba3SisoFn (step)");
     return true;
