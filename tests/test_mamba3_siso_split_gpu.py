@@ -4,7 +4,7 @@ tiling, row blocks of 16 and 32 rows and several of them, ragged last segments,
 partial angles, shared Q/K heads, with and without Z, D, input and final states,
 packed sequences shorter and longer than a segment and empty ones, growth that
 overflows a plain decay, the automatic choice, and outputs that share memory
-with an input (no split)."""
+with an input, final states over the input states among them (no split)."""
 
 import numpy as np
 import pytest
@@ -166,3 +166,30 @@ def test_overlapping_packed_sequences_keep_their_states(override):
         out.append([x.cpu().numpy() for x in f])
     for part, a, b in zip(PARTS[1:], *out):
         np.testing.assert_array_equal(a, b, err_msg=part)
+
+
+@pytest.mark.parametrize("p,parts", [(32, (0, 1, 2, 3)), (64, (0, 3)), (64, (0,)), (32, (1,)), (32, (2,)), (64, (3,)), (64, ())])
+def test_final_states_over_the_input_states_are_not_split(p, parts):
+    """One workgroup walks the whole sequence of its rows and may keep the states
+    in one buffer (angle and k up to 32 rows, one workgroup a head); the segments'
+    workgroups of one launch may not.  y and the other states apart."""
+    import ctypes
+    import torch
+    from xmetai_onnx_plugins import _capi
+    s = S(1, 1001, 4, p, 128, has_z=True)
+    inp = W.mamba3_siso_inputs(s, seed=49)
+    dev = [to_dev(inp[k]) for k in KEYS]
+    states = [to_dev(x) for x in start_states(s, 1, 50)]
+    y, f = xp.mamba3_siso_fn(*dev, return_final_states=True, input_states=tuple(states))
+    assert split_launched(), xp.last_launches()
+    outs = [torch.empty_like(y), *(states[i] if i in parts else torch.empty_like(f[i]) for i in range(4))]
+    ins = [*dev, *states]
+    arr = (_capi.XmTensor * len(ins))(*[xp._desc_from_tensor(x) for x in ins])
+    attrs = xp._attrs("mamba3_siso", has_d=1, has_z=1, return_final_states=1, has_input_states=1)
+    err = ctypes.create_string_buffer(256)
+    st = xp.lib().xm_mamba3_siso_forward_states(arr, len(ins), ctypes.byref(attrs), *(x.data_ptr() for x in outs),
+                                                torch.cuda.current_stream().cuda_stream, None, err, len(err))
+    assert st == xp.XM_OK, err.value
+    assert split_launched() == (not parts), xp.last_launches()
+    torch.cuda.synchronize()
+    compare(f"states_in_place_p{p}_{parts}", outs, [x.cpu().numpy() for x in (y, *f)], TOL_GPU)

@@ -979,23 +979,22 @@ __global__ __launch_bounds__(64 * (NW + NPW)) void Mamba3ChunkKernel(Mamba3SisoP
     }
 }
 
-// True when the output shares no byte with an input or a state, so that its
-// rows can hold the sequence split's records while the inputs are still read.
-bool OutputApart(const Mamba3SisoParams &p) {
-    const bool packed = p.cu_seqlens != nullptr;
-    const size_t f = sizeof(float), rows = static_cast<size_t>(packed ? 1 : p.batch) * p.seqlen;
-    const size_t v = rows * p.nheads * p.p * f, q = rows * p.nheads_qk * p.n * f, bh = static_cast<size_t>(p.batch) * p.nheads * f;
-    const uintptr_t o = reinterpret_cast<uintptr_t>(p.out);
-    auto apart = [&](const void *x, size_t bytes) {
-        const uintptr_t a = reinterpret_cast<uintptr_t>(x);
-        return x == nullptr || a + bytes <= o || o + v <= a;
-    };
-    return apart(p.Q, q) && apart(p.K, q) && apart(p.V, v) && apart(p.Z, v) && apart(p.Angles, rows * p.nheads * p.a * f) &&
-           apart(p.ADT, rows * p.nheads * f) && apart(p.DT, rows * p.nheads * f) && apart(p.Trap, rows * p.nheads * f) &&
-           apart(p.Q_bias, static_cast<size_t>(p.nheads) * p.n * f) && apart(p.K_bias, static_cast<size_t>(p.nheads) * p.n * f) &&
-           apart(p.D, static_cast<size_t>(p.nheads) * f) && apart(p.cu_seqlens, (static_cast<size_t>(p.batch) + 1) * 8) &&
-           apart(p.in_ssm, bh * p.p * p.n) && apart(p.in_angle, bh * p.a) && apart(p.in_k, bh * p.n) && apart(p.in_v, bh * p.p) &&
-           apart(p.f_ssm, bh * p.p * p.n) && apart(p.f_angle, bh * p.a) && apart(p.f_k, bh * p.n) && apart(p.f_v, bh * p.p);
+// True when no output shares memory with an input, and y none with a final
+// state: the rows of y can then hold the sequence split's records, and the last
+// segment's workgroup may write the final states while the first segments' read
+// the inputs and the input states (a caller may keep both in one buffer).
+bool OutputsApart(const Mamba3SisoParams &p) {
+    const size_t f = sizeof(float), rows = static_cast<size_t>(p.cu_seqlens != nullptr ? 1 : p.batch) * p.seqlen;
+    const size_t bh = static_cast<size_t>(p.batch) * p.nheads * f, th = rows * p.nheads * f, h = static_cast<size_t>(p.nheads) * f;
+    const size_t qk = rows * p.nheads_qk * p.n * f;
+    const MemRange y{p.out, th * p.p}, ssm{p.f_ssm, bh * p.p * p.n}, angle{p.f_angle, bh * p.a}, k{p.f_k, bh * p.n},
+        v{p.f_v, bh * p.p};
+    return !AnyOverlap({y}, {ssm, angle, k, v}) &&
+           !AnyOverlap({y, ssm, angle, k, v},
+                       {{p.Q, qk}, {p.K, qk}, {p.V, th * p.p}, {p.Z, th * p.p}, {p.Angles, th * p.a}, {p.ADT, th}, {p.DT, th},
+                        {p.Trap, th}, {p.Q_bias, h * p.n}, {p.K_bias, h * p.n}, {p.D, h},
+                        {p.cu_seqlens, (static_cast<size_t>(p.batch) + 1) * sizeof(int64_t)}, {p.in_ssm, bh * p.p * p.n},
+                        {p.in_angle, bh * p.a}, {p.in_k, bh * p.n}, {p.in_v, bh * p.p}});
 }
 
 // Split when the row blocks fill at most half the CUs, into as many output
@@ -1015,7 +1014,7 @@ constexpr int kSplitMax = 16, kFineMax = 8;
 M3Split ChooseSplit(const Mamba3SisoParams &p, int np) {
     const M3Split whole{0, 0, 0, 1};
     const int forced = static_cast<int>(GetOverride(kOverrideM3Split));
-    if (forced == 1 || p.p % 16 != 0 || !OutputApart(p)) return whole;
+    if (forced == 1 || p.p % 16 != 0 || !OutputsApart(p)) return whole;
     // a 32-row workgroup of the output launch and a 64-row one of the state
     // launch per CU: one round of each (packed: of the whole row's segments)
     const bool packed = p.cu_seqlens != nullptr;
