@@ -68,3 +68,13 @@ def test_m3_step_reads_its_tokens_four_at_a_time():
         assert (m3_launches(1, t, 1, 32, 32, 16, {0: (2, row)}) == STEP) == ok    # y one token behind V
         assert (m3_launches(1, t, 1, 32, 32, 16, {0: (0, 0)}) == STEP) == ok      # y over Q
         assert m3_launches(1, t, 1, 32, 32, 16, {0: (2, 0)}) == STEP              # y over V
+
+
+def test_ss_segments_with_outputs_over_inputs():
+    """y or the last state over an input, or over each other: one launch of the whole pass, not two of segments."""
+    u, w, bc = (1, 5120, 2048), (5120, 16), (1, 1, 16, 2048)
+    shapes = [u, u, w, bc, bc, (5120,), None, (5120,)]
+    for at, two in (({}, True), ({0: (0, 0)}, False), ({1: (2, 0)}, False), ({1: (5, 0)}, False), ({0: (4, 64)}, False),
+                    ({1: (7, 5120 * 4 - 4)}, False), ({1: (7, 5120 * 4)}, True)):
+        got = launches("selective_scan", shapes, 2, at, return_last_state=1)
+        assert got == ["SelectiveScanFwdKernel"] * (2 if two else 1), (at, xp.last_launches())

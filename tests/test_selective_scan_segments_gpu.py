@@ -3,7 +3,8 @@ the segments' states handed over through the output rows) on the GPU vs the
 fp64 oracle, through the C ABI: ragged last tiles and segments, rows on every
 4-byte offset, groups, the state layouts, 16-bit rows of even and odd length,
 the last state, the automatic choice, growth that overflows a plain decay
-product, and outputs that share memory with an input (the whole pass)."""
+product, and outputs that share memory with an input (the whole pass), the last
+state over A among them."""
 
 import numpy as np
 import pytest
@@ -139,3 +140,27 @@ def test_output_over_an_input_takes_the_whole_pass(override):
     assert not segments_launched()
     torch.cuda.synchronize()
     check("selective_scan_segments/in_place", dev[0].cpu().numpy(), run_ref(inp, state=False), TOL_SS)
+
+
+def test_last_state_over_the_weights_takes_the_whole_pass(override):
+    """The last state of one sequence has A's size: over A, whose channel one
+    workgroup of the whole pass reads before it writes."""
+    import ctypes
+    import torch
+    import xmetai_onnx_plugins as xp
+    from xmetai_onnx_plugins import _capi
+    inp = W.selective_scan_inputs(S(1, 64, 512, 16), seed=36)
+    override("ss_split", 3)
+    dev = [to_dev(inp[k]) for k in KEYS]
+    y = torch.empty_like(dev[0])
+    arr = (_capi.XmTensor * len(dev))(*[xp._desc_from_tensor(x) for x in dev])
+    attrs = xp._attrs("selective_scan", delta_softplus=1, return_last_state=1)
+    err = ctypes.create_string_buffer(256)
+    st = xp.lib().xm_selective_scan_forward_states(arr, len(dev), ctypes.byref(attrs), y.data_ptr(), dev[2].data_ptr(),
+                                                   torch.cuda.current_stream().cuda_stream, None, err, len(err))
+    assert st == xp.XM_OK, err.value
+    assert not segments_launched(), last_launches()
+    torch.cuda.synchronize()
+    ref_y, ref_h = run_ref(inp)
+    check("selective_scan_segments/last_state_over_A/y", y.cpu().numpy(), ref_y, TOL_SS)
+    check("selective_scan_segments/last_state_over_A/h", dev[2].cpu().numpy()[None], ref_h, TOL_SS)

@@ -618,21 +618,17 @@ void LaunchSkip(const SelectiveScanParams &p, hipStream_t stream) {
     hipLaunchKernelGGL(SelectiveScanSkipKernel<IT>, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, p);
 }
 
-// True when the output shares no byte with an input, so that its rows can hold
-// the sequence split's records while the inputs are still read.
-bool OutputApart(const SelectiveScanParams &p) {
-    const size_t eb = p.in_type == XM_ELEM_FLOAT ? 4 : 2;
-    const size_t rows = static_cast<size_t>(p.batch) * p.dim * p.seqlen;
-    const size_t bc = static_cast<size_t>(p.batch) * p.dstate * p.seqlen, w = static_cast<size_t>(p.dim) * p.dstate;
-    const uintptr_t o = reinterpret_cast<uintptr_t>(p.out);
-    auto apart = [&](const void *x, size_t bytes) {
-        const uintptr_t a = reinterpret_cast<uintptr_t>(x);
-        return x == nullptr || a + bytes <= o || o + rows * eb <= a;
-    };
-    return apart(p.u, rows * eb) && apart(p.delta, rows * eb) && apart(p.A, w * 4) &&
-           apart(p.B, p.b_var ? bc * p.groups_b * eb : w * 4) && apart(p.C, p.c_var ? bc * p.groups_c * eb : w * 4) &&
-           apart(p.D, static_cast<size_t>(p.dim) * 4) && apart(p.delta_bias, static_cast<size_t>(p.dim) * 4) &&
-           apart(p.last_state, static_cast<size_t>(p.batch) * w * 4);
+// True when neither y nor the last state shares memory with an input (B and C
+// variable), or with the other: the rows of y can then hold the sequence split's
+// records, and the last segment's workgroup may write the last state while other
+// segments' still read the channel's inputs (A, of the same size, among them).
+bool OutputsApart(const SelectiveScanParams &p) {
+    const size_t eb = p.in_type == XM_ELEM_FLOAT ? 4 : 2, f = sizeof(float), dim = static_cast<size_t>(p.dim);
+    const size_t rows = p.batch * dim * p.seqlen * eb, bc = static_cast<size_t>(p.batch) * p.dstate * p.seqlen * eb;
+    const MemRange y{p.out, rows}, last{p.last_state, p.batch * dim * p.dstate * f};
+    return !Overlap(y, last) &&
+           !AnyOverlap({y, last}, {{p.u, rows}, {p.delta, rows}, {p.A, dim * p.dstate * f}, {p.B, bc * p.groups_b},
+                                   {p.C, bc * p.groups_c}, {p.D, dim * f}, {p.delta_bias, dim * f}});
 }
 
 // At most `most` segments whose rows can hold the records; count 1 if none.
@@ -668,7 +664,7 @@ struct SsPlan {
 // segments wherever the rows hold their records.
 SsPlan ChoosePlan(const SelectiveScanParams &p, const Config &cfg, long long blocks, int64_t forced) {
     const SegSplit whole{1, p.seqlen};
-    const bool seg_fits = SelectiveScanSegFits(p), splits = p.b_var && p.c_var && OutputApart(p);
+    const bool seg_fits = SelectiveScanSegFits(p), splits = p.b_var && p.c_var && OutputsApart(p);
     if (forced == 1) return {false, whole};
     if (forced == 2) return {seg_fits, whole};
     if (forced == 3) return {false, splits ? FitSegments(p, kSplitMax, 32) : whole};
