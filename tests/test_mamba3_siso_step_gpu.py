@@ -3,7 +3,8 @@ in one launch) on the GPU vs the fp64 oracle: key counts at the edges of the
 64-key groups and of a four-key group, state rows cut by a row block, the three
 row-block heights, one to sixteen tokens (prepared four at a time), angles of
 some pairs, Q/K heads shared, with and without Z, D, input and final states,
-agreement with the chunked kernel, and outputs over inputs: final states over the
+agreement with the chunked kernel, what lies behind a sequence's tokens, and
+outputs over inputs: final states over the
 input states (one row block a head), y over V, Z, Q and a part of V."""
 
 import numpy as np
@@ -164,3 +165,32 @@ def test_y_over_an_input(over, tokens):
     call_states(dev, states, outs)
     assert step_rows() == (0 if over in ("Q", "behind_V") and tokens > 4 else 32 if over == "Q" else 16), xp.last_launches()
     compare(f"y_over_{over}_t{tokens}", outs, [x.cpu().numpy() for x in want], TOL_GPU)
+
+
+@pytest.mark.parametrize("has_z", [True, False])
+@pytest.mark.parametrize("tokens", [1, 2, 3, 5, 6, 7])
+def test_step_reads_nothing_behind_its_tokens(tokens, has_z):
+    """A block takes four tokens: those past the end read as zeros, whatever
+    follows a sequence's rows (here NaN, in the same allocation)."""
+    import torch
+    s = S(3, tokens, 4, 24, 64, angles=20, has_z=has_z)
+    dev, states, want = sharing_case(s, seed=tokens)
+
+    def guarded(x):
+        buf = torch.full((x.numel() + 16 * s.nheads * 64,), float("nan"), device="cuda")
+        t = buf[:x.numel()].view(x.shape)
+        t.copy_(x)
+        return t
+    outs = [torch.empty_like(x) for x in want]
+    call_states([x if x is None else guarded(x) for x in dev], states, outs)
+    assert step_rows() == 16
+    for g, w in zip(outs, want):
+        assert torch.isfinite(g).all() and torch.equal(g, w)
+    for b in (1, 2):   # the sequence behind one whose results must not change
+        part = [x if x is None else x.clone() for x in dev]
+        for i in (0, 1, 2, 3, 4, 5, 8, 10):
+            if part[i] is not None:
+                part[i][b] = float("nan")
+        call_states(part, states, outs)
+        for g, w in zip(outs, want):
+            assert torch.equal(g[:b], w[:b])

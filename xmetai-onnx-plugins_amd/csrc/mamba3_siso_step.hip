@@ -69,7 +69,9 @@ __global__ __launch_bounds__(kThreads) void Mamba3StepKernel(Mamba3SisoParams p)
     // Every input through a raw-buffer descriptor: tokens past T, pairs past the
     // end and absent tensors (size 0) read zeros with no branch, so all of a
     // block's loads go out at once (a kernel this short is a few dependent
-    // memory latencies long).
+    // memory latencies long).  The scalar offset is that of a block's first token,
+    // which is below the size; what a wave or slot adds to it, and all of an
+    // offset into a tensor that may be absent, is per lane.
     const size_t tok0 = static_cast<size_t>(b) * T, sb = static_cast<size_t>(bh) * T;
     auto rows_of = [&](const float *x, size_t first, int stride) {   // token rows of `stride` floats from x + first
         return MakeRsrc(x != nullptr ? x + first : p.DT, x != nullptr ? T * stride * 4 : 0);
@@ -99,10 +101,10 @@ __global__ __launch_bounds__(kThreads) void Mamba3StepKernel(Mamba3SisoParams p)
         const int t = t0 + wave;
 #pragma unroll
         for (int x = 0; x < PB; ++x) {
-            qv[x] = BufF2(rq, poff[x], t * qs * 4);
-            kv[x] = BufF2(rk, poff[x], t * qs * 4);
+            qv[x] = BufF2(rq, poff[x] + wave * qs * 4, t0 * qs * 4);
+            kv[x] = BufF2(rk, poff[x] + wave * qs * 4, t0 * qs * 4);
 #pragma unroll
-            for (int s = 0; s < kTB; ++s) ang[x][s] = BufF(ra, aoff[x], (t0 + s) * as * 4);
+            for (int s = 0; s < kTB; ++s) ang[x][s] = BufF(ra, aoff[x] + s * as * 4, t0 * as * 4);
         }
 #pragma unroll
         for (int s = 0; s < kTB; ++s) dts[s] = BufF(rdt, (t0 + s) * 4);
@@ -115,9 +117,9 @@ __global__ __launch_bounds__(kThreads) void Mamba3StepKernel(Mamba3SisoParams p)
         ad = BufF(rad, t * 4);
         dt1 = BufF(rdt, (t + 1) * 4);   // zero past the last token: no look-ahead
         tr1 = BufF(rtr, (t + 1) * 4);
-        const int o = vlane ? vtok * vs * 4 + vrow * 4 : kOutOfRange;
-        vreg = BufF(rv, o, t0 * vs * 4);
-        zreg = BufF(rz, o, t0 * vs * 4);
+        const int o = vlane ? ((t0 + vtok) * vs + vrow) * 4 : kOutOfRange;
+        vreg = BufF(rv, o);
+        zreg = BufF(rz, o);
     };
     auto prepare = [&](int t0) __attribute__((always_inline)) {
         float qk = 0.0f;

@@ -22,6 +22,8 @@ __device__ __forceinline__ void StF4(float *p, v4f v) { *reinterpret_cast<v4f *>
 // stores there are dropped (the range check covers the sum: measured on
 // gfx950, size 256 with scalar offset 128 drops per-lane offsets from 128 on),
 // which masks tokens past the sequence end and columns past dv with no branch.
+// The scalar offset alone stays below the size: a check that subtracts it from
+// the size would wrap.
 typedef __amdgpu_buffer_rsrc_t Rsrc;
 constexpr int kRawBufferWord3 = 0x00020000;                       // untyped 32-bit data format
 constexpr int kOutOfRange = static_cast<int>(0x80000000u);        // beyond any descriptor size used here
