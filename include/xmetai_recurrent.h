@@ -238,7 +238,8 @@ int xm_gated_deltanet2_forward_states(const xm_tensor_t *inputs, size_t n_inputs
  * library runs on holds until the process ends; the chunked path's windows
  * and the preparation chunks of head_k > 512 shrink to fit it, and a call that
  * cannot fit (e.g. a carried state of 64 MiB or more) fails with
- * XM_ERR_UNSUPPORTED before anything is enqueued.  It calls no hipMalloc or
+ * XM_ERR_UNSUPPORTED before anything is enqueued.  A call of up to 16 tokens
+ * that needs no scratch (above) never fails so.  It calls no hipMalloc or
  * hipFree.  Every call on a GPU shares that GPU's array: calls that overlap on
  * one GPU (concurrent streams) race and must be serialised by the caller.
  * Results equal xm_gated_deltanet2_forward's, except where that call splits

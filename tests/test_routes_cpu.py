@@ -78,3 +78,15 @@ def test_ss_segments_with_outputs_over_inputs():
                     ({1: (7, 5120 * 4 - 4)}, False), ({1: (7, 5120 * 4)}, True)):
         got = launches("selective_scan", shapes, 2, at, return_last_state=1)
         assert got == ["SelectiveScanFwdKernel"] * (2 if two else 1), (at, xp.last_launches())
+
+
+@pytest.mark.parametrize("at,refused", [(7, False), (0, True), (3, True)])
+def test_noalloc_decode_of_many_heads(at, refused):
+    """A call of a few tokens needs none of the fixed array, so its heads are not
+    limited by it; the chunked path, which an output over q or g takes, is."""
+    k, state = (4096, 1, 16, 128), (4096, 16, 128, 128)
+    ins = (_capi.XmTensor * 7)(*[xp._desc_from_shape(sh, (i + 1) << 34) for i, sh in enumerate([k] * 6 + [state])])
+    a, err = xp._attrs("gated_deltanet2", scale=1.0), ctypes.create_string_buffer(512)
+    st = xp.lib().xm_gated_deltanet2_forward_noalloc(ins, 7, ctypes.byref(a), (at + 1) << 34, None, err, len(err))
+    assert (st == xp.XM_ERR_UNSUPPORTED) == refused, err.value
+    assert xp.last_launches() == ([] if refused else ["Gdn2StepKernel<16,8>"])

@@ -147,6 +147,15 @@ def test_noalloc_calls_on_two_streams_are_ordered():
         np.testing.assert_array_equal(out.cpu().numpy(), ref.cpu().numpy())
 
 
+@pytest.mark.gpu
+def test_noalloc_decode_of_many_heads():
+    # one token of 192 sequences x 16 heads at 128 x 128: the chunked path would
+    # need more than the array for one chunk, the single launch needs nothing
+    got, want, launched = run_both(S(192, 1, 16, 128, 128), seed=8)
+    np.testing.assert_array_equal(got, want)
+    assert launched == ["Gdn2StepKernel<16,8>"], launched
+
+
 def test_noalloc_rejects_calls_beyond_the_array():
     # The carried state alone (64 heads x 512 x 512 fp32 = 64 MiB) leaves no
     # room for a window: rejected before anything is enqueued (no device use).

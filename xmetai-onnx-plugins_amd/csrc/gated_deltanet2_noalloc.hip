@@ -80,6 +80,10 @@ extern "C" int xm_gated_deltanet2_forward_noalloc(const xm_tensor_t *inputs, siz
             xm::Invalid("GatedDeltaNet2Fn with output_final_state=1 needs a final_state output "
                         "(xm_gated_deltanet2_forward_states)");
         const xm::GatedDeltaNet2Params p = xm::GatedDeltaNet2Plan(inputs, n_inputs, *attrs, out, nullptr);
+        if (xm::GatedDeltaNet2StepFits(p)) {   // a few tokens: no scratch, however many the heads
+            xm::LaunchGatedDeltaNet2(p, nullptr, 0, stream);
+            return;
+        }
         const size_t need = xm::GatedDeltaNet2ScratchBytes(p.batch, p.seqlen, p.nheads, p.dk, p.dv,
                                                            p.cu_seqlens != nullptr, xm::kNoAllocScratchBytes);
         if (need == SIZE_MAX)
@@ -87,7 +91,7 @@ extern "C" int xm_gated_deltanet2_forward_noalloc(const xm_tensor_t *inputs, siz
                             "GatedDeltaNet2Fn (xm_gated_deltanet2_forward_noalloc): the call needs more than the " +
                                 std::to_string(xm::kNoAllocScratchBytes >> 20) +
                                 " MiB of device scratch this entry point holds; use xm_gated_deltanet2_forward");
-        if (need == 0 || xm::GatedDeltaNet2StepFits(p)) {   // nothing touches the array
+        if (need == 0) {   // nothing touches the array
             xm::LaunchGatedDeltaNet2(p, nullptr, 0, stream);
             return;
         }
