@@ -3,7 +3,7 @@ handed over through the output rows) on the GPU vs the fp64 oracle: every key
 tiling, row blocks of 16 and 32 rows and several of them, ragged last segments,
 partial angles, shared Q/K heads, with and without Z, D, input and final states,
 packed sequences shorter and longer than a segment and empty ones, growth that
-overflows a plain decay, the automatic choice, and outputs that share memory
+overflows a plain decay, infinite and NaN inputs, the automatic choice, and outputs that share memory
 with an input, final states over the input states among them (no split)."""
 
 import numpy as np
@@ -121,6 +121,44 @@ def test_split_growth_beyond_one_decay(override):
     # measure's floor of 1e-3 of the largest: 1e3 times the bound)
     check("mamba3_siso_split/growth/y", y.cpu().numpy(), ref_y, Gate(1e-4, 1e-1))
     check("mamba3_siso_split/growth/ssm", f[0].cpu().numpy(), ref_f[0], 1e-4)
+
+
+NOT_FINITE = {   # input, place, value
+    "v_inf": ("V", (0, 300, 1, 5), np.inf),
+    "v_minus_inf_first": ("V", (0, 0, 1, 5), -np.inf),
+    "v_nan": ("V", (0, 300, 1, 5), np.nan),
+    "k_inf": ("K", (0, 300, 0, 4), np.inf),
+    "k_inf_last_of_a_segment": ("K", (0, 223, 0, 7), -np.inf),
+    "adt_inf": ("ADT", (0, 1, 300), np.inf),
+    "adt_minus_inf": ("ADT", (0, 1, 300), -np.inf),
+    "dt_inf": ("DT", (0, 1, 300), np.inf),
+    "angle_nan": ("Angles", (0, 300, 1, 2), np.nan),
+    "q_inf": ("Q", (0, 300, 0, 4), np.inf),
+}
+
+
+@pytest.mark.parametrize("name", sorted(NOT_FINITE))
+@pytest.mark.parametrize("shape,cu", [(S(1, 1000, 2, 64, 64, has_z=True), None), (S(1, 1000, 2, 48, 128, angles=40), None),
+                                      (S(1, 1100, 2, 32, 256), [0, 1000, 1100])], ids=["n64", "n128", "n256_packed"])
+def test_split_of_infinite_and_nan_inputs(name, shape, cu, override):
+    """An infinite or NaN input makes every later state of its rows or heads so, at
+    the same places and with the same signs as the whole pass (turning a segment's
+    end state would mix infinities of two keys); all else stays as it was."""
+    inp = W.mamba3_siso_inputs(shape, seed=51)
+    key, at, value = NOT_FINITE[name]
+    inp[key][at] = value
+    out = []
+    for mode in (2, 1):
+        override("m3_split", mode)
+        y, f = xp.mamba3_siso_fn(*(to_dev(inp[k]) for k in KEYS), return_final_states=True,
+                                 cu_seqlens=None if cu is None else to_dev(np.asarray(cu, np.int64)))
+        assert split_launched() == (mode == 2), xp.last_launches()
+        out.append([x.cpu().numpy() for x in (y, *f)])
+    finite = []
+    for part, a, b in zip(PARTS, *out):
+        np.testing.assert_array_equal(np.where(np.isfinite(a), 0.0, a), np.where(np.isfinite(b), 0.0, b), err_msg=part)
+        finite.append((np.where(np.isfinite(a), a, 0.0), np.where(np.isfinite(b), b, 0.0)))
+    compare(f"{name}_n{shape.dstate}", *zip(*finite), TOL_GPU)
 
 
 def test_split_chosen_for_one_prompt():

@@ -224,7 +224,10 @@ __device__ __forceinline__ float RowInclusiveScan16(float x) {
 // token (columns of the row block: 4 bytes x W), which only launch 3's
 // workgroup of that segment and row block overwrites, after it has read them:
 // no scratch.  A record is the S^T tiles in lane order, the fine segment's
-// angle sums, its sum of ADT, and the start angles.
+// angle sums, its sum of ADT, the start angles, and a flag per 64 quads of the
+// start state: one of them is not finite.  A turn would mix an infinity of one
+// key into the key beside it, so a segment whose start state is not finite walks
+// the sequence from its first token instead and stores only its own rows.
 // Packed sequences split likewise, each by its own length.
 // ---------------------------------------------------------------------------
 enum M3Mode { kM3Whole, kM3State, kM3Out };
@@ -249,6 +252,8 @@ struct M3Record {
     __device__ __forceinline__ int AngleSum(int a) const { return np * w + 2 * a; }        // two words of a double
     __device__ __forceinline__ int DecaySum() const { return np * w + np; }
     __device__ __forceinline__ int StartAngle(int a) const { return np * w + np + 16 + 2 * a; }
+    __device__ __forceinline__ int Flags() const { return np * w / 256; }                   // at most 32
+    __device__ __forceinline__ float *Flag(int i) const { return At(np * w + 2 * np + 16 + i); }
     __device__ __forceinline__ double GetD(int e) const {
         const unsigned lo = __float_as_uint(*At(e)), hi = __float_as_uint(*At(e + 1));
         return __longlong_as_double(static_cast<long long>((static_cast<unsigned long long>(hi) << 32) | lo));
@@ -373,9 +378,20 @@ __global__ __launch_bounds__(64 * (NW + NPW)) void Mamba3ChunkKernel(Mamba3SisoP
             te = last_seg ? T : cs + split.ls;
         }
     }
-    const bool first_seg = seg == 0;
     auto record_of = [&](int i) { return RecordAt(p, tok0 + cs, h, r0 + kRows * i, L::NP); };   // its i-th 32 rows'
     const M3Record rec = record_of(0);
+    const int y_from = cs;      // first token whose y this workgroup stores
+    bool at_start = seg == 0;   // the walk starts with the sequence, from the input states
+    float flag = 0.0f;          // kM3Out: a lane's part of the record's
+    auto see_flags = [&]() __attribute__((always_inline)) {
+        if (__ballot(flag != 0.0f) == 0) return;
+        at_start = true;
+        cs = 0;
+    };
+    if constexpr (MODE == kM3Out) {
+        if (!at_start && lane < rec.Flags()) flag = *rec.Flag(lane);
+        if (product_wave) see_flags();   // the others have loads of their own to send first
+    }
     const float *dtr = p.DT + sbase;
     const float *trr = p.Trap + sbase;
     const float *adr = p.ADT + sbase;
@@ -396,6 +412,7 @@ __global__ __launch_bounds__(64 * (NW + NPW)) void Mamba3ChunkKernel(Mamba3SisoP
     const int pq = lane % PL, tg = lane / PL;
     int pr[PB], qoff[PB][TPL], aoff[PB][TPL];
     float2 qbias[PB], kbias[PB];
+    double carry_rec[PB];   // kM3Out: from the record
     double carry[PB];   // wrapped angle after the last prepared token, in turns of the wrap period
 #pragma unroll
     for (int x = 0; x < PB; ++x) {
@@ -408,9 +425,9 @@ __global__ __launch_bounds__(64 * (NW + NPW)) void Mamba3ChunkKernel(Mamba3SisoP
         kbias[x] = real ? kb : make_float2(0.0f, 0.0f);
         carry[x] = (p.in_angle != nullptr && rot) ? static_cast<double>(p.in_angle[static_cast<size_t>(bh) * A + pr[x]]) * kInvTwoPiF : 0.0;
         if constexpr (kState) {
-            if (!first_seg) carry[x] = 0.0;   // counted from the segment's start
+            if (!at_start) carry[x] = 0.0;   // counted from the segment's start
         } else if constexpr (MODE == kM3Out) {
-            if (!product_wave && rot && !first_seg) carry[x] = rec.GetD(rec.StartAngle(pr[x]));
+            carry_rec[x] = !product_wave && rot && !at_start ? rec.GetD(rec.StartAngle(pr[x])) : carry[x];
         }
 #pragma unroll
         for (int s = 0; s < TPL; ++s) {
@@ -622,7 +639,7 @@ __global__ __launch_bounds__(64 * (NW + NPW)) void Mamba3ChunkKernel(Mamba3SisoP
                 for (int r = 0; r < 4; ++r) {
                     const int row = r0 + 16 * pt + i16, key = 16 * (KBW * w + kb) + 4 * g4 + r;
                     float v = 0.0f;
-                    if (product_wave && first_seg && p.in_ssm != nullptr && row < P && key < N) {
+                    if (product_wave && at_start && p.in_ssm != nullptr && row < P && key < N) {
                         const float vl = p.in_v[static_cast<size_t>(bh) * P + row];
                         const float kl = p.in_k[static_cast<size_t>(bh) * N + key];
                         v = fmaf(vl, kl * look0, p.in_ssm[(static_cast<size_t>(bh) * P + row) * N + key]);
@@ -630,7 +647,7 @@ __global__ __launch_bounds__(64 * (NW + NPW)) void Mamba3ChunkKernel(Mamba3SisoP
                     S[kb][pt][r] = v;
                 }
         if constexpr (MODE == kM3Out) {
-            if (product_wave && !first_seg) {
+            if (product_wave && !at_start) {
 #pragma unroll
                 for (int kb = 0; kb < KBW; ++kb)
 #pragma unroll
@@ -751,6 +768,7 @@ __global__ __launch_bounds__(64 * (NW + NPW)) void Mamba3ChunkKernel(Mamba3SisoP
     // store's data register rewritten behind it waits for the store to
     // complete (stores count in vmcnt on gfx950).
     auto store_y = [&](int c0, const float (&y)[4]) __attribute__((always_inline)) {
+        if (MODE == kM3Out && c0 < y_from) return;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             if constexpr (LONG) BufStF(chunk_rsrc(p.out + vbase, v_stride, c0), ooff[r], y[r]);
@@ -814,7 +832,7 @@ __global__ __launch_bounds__(64 * (NW + NPW)) void Mamba3ChunkKernel(Mamba3SisoP
         }
     };
 
-    const int nch = (te - cs + kC - 1) / kC;
+    int nch = (te - cs + kC - 1) / kC;
     using P0 = std::integral_constant<int, 0>;
     using P1 = std::integral_constant<int, 1>;
     auto big = [&](auto P) { return smem + L::oBig + decltype(P)::value * kBig; };      // chunk parity P
@@ -832,6 +850,17 @@ __global__ __launch_bounds__(64 * (NW + NPW)) void Mamba3ChunkKernel(Mamba3SisoP
     auto prepare_chunks = [&]() __attribute__((always_inline)) {   // the preparation waves' loop
         load_prep(cs, raw0);
         if constexpr (DB) load_prep(cs + min(1, nch - 1) * kC, raw1);
+        if constexpr (MODE == kM3Out) {
+            see_flags();
+            if (cs != y_from) {
+                nch = (te + kC - 1) / kC;
+                load_prep(0, raw0);
+                if constexpr (DB) load_prep(min(1, nch - 1) * kC, raw1);
+            } else {
+#pragma unroll
+                for (int x = 0; x < PB; ++x) carry[x] = carry_rec[x];
+            }
+        }
         prep(big(P0{}), small(0), raw0);
         if constexpr (!DB) load_prep(cs + min(1, nch - 1) * kC, raw0);
         __syncthreads();
@@ -1087,6 +1116,9 @@ __global__ __launch_bounds__(256) void Mamba3SegCombineKernel(Mamba3SisoParams p
         if (f > 0 && f % m == 0) {
             const M3Record rf = record(f);
             *reinterpret_cast<v4u *>(rf.State(q)) = S;
+            const bool inf = !(isfinite(S[0]) && isfinite(S[1]) && isfinite(S[2]) && isfinite(S[3]));
+            const bool any = __ballot(inf) != 0;   // whole waves: np w / 4 is a multiple of 64
+            if (lane == 0) *rf.Flag(q / 64) = any ? 1.0f : 0.0f;
 #pragma unroll
             for (int e = 0; e < 2; ++e)
                 if (writes_angles && key / 2 + e < A) rf.PutD(rf.StartAngle(key / 2 + e), th[e]);
