@@ -3,14 +3,14 @@ the segments' states handed over through the output rows) on the GPU vs the
 fp64 oracle, through the C ABI: ragged last tiles and segments, rows on every
 4-byte offset, groups, the state layouts, 16-bit rows of even and odd length,
 the last state, the automatic choice, growth that overflows a plain decay
-product, and outputs that share memory with an input (the whole pass), the last
+product, infinite and NaN inputs, and outputs that share memory with an input (the whole pass), the last
 state over A among them."""
 
 import numpy as np
 import pytest
 
 from oracle import cref
-from parity import TOL_SS, check, to_dev
+from parity import TOL_GPU, TOL_SS, check, to_dev
 from xmetai_onnx_plugins import last_launches, selective_scan_fn, workloads as W
 
 pytestmark = pytest.mark.gpu
@@ -120,6 +120,41 @@ def test_growth_beyond_one_decay_product(u0, override):
     want = u0 * 1e-30 * N * np.exp(128.0)
     got = y[0, :, -1].double().cpu().numpy()
     assert np.all(np.abs(got - want) <= 1e-4 * abs(want))   # 64 factors exp2(2 log2 e), each within 4 x 2^-23
+
+
+NOT_FINITE = {   # input, place, value
+    "u_inf": ("u", (0, 3, 300), np.inf),
+    "u_nan": ("u", (0, 3, 300), np.nan),
+    "u_minus_inf_first": ("u", (0, 3, 0), -np.inf),
+    "delta_inf": ("delta", (0, 3, 300), np.inf),
+    "b_inf": ("B", (0, 0, 2, 300), np.inf),
+    "c_inf": ("C", (0, 0, 2, 300), np.inf),
+    "a_inf": ("A", (3, 0), np.inf),
+    "a_minus_inf": ("A", (3, 0), -np.inf),
+}
+
+
+@pytest.mark.parametrize("name", sorted(NOT_FINITE))
+@pytest.mark.parametrize("shape", [S(1, 64, 1000, 16), S(1, 40, 999, 3), S(2, 64, 1021, 8), S(1, 32, 1100, 64)],
+                         ids=["n16", "n3_ragged", "n8", "n64"])
+@pytest.mark.parametrize("softplus", [True, False])
+def test_infinite_and_nan_inputs(name, shape, softplus, override):
+    """Infinite and NaN states (without softplus the states of this input overflow
+    by themselves) come out where and as they do in the whole pass."""
+    inp = W.selective_scan_inputs(shape, seed=37)
+    key, at, value = NOT_FINITE[name]
+    inp[key].reshape((shape.batch, 1, shape.dstate, shape.seqlen) if key in "BC" else inp[key].shape)[at] = value
+    out = []
+    for split in (3, 1):
+        override("ss_split", split)
+        y, h = selective_scan_fn(*(to_dev(inp[k]) for k in KEYS), delta_softplus=softplus, return_last_state=True)
+        assert segments_launched() == (split == 3), last_launches()
+        out.append((y.cpu().numpy(), h.cpu().numpy()))
+    for part, a, b in zip("yh", *out):
+        np.testing.assert_array_equal(np.where(np.isfinite(a), 0.0, a), np.where(np.isfinite(b), 0.0, b), err_msg=part)
+        if softplus:   # states of one size: held to the tolerance between two device paths
+            check(f"selective_scan_segments/{name}_n{shape.dstate}/{part}", np.where(np.isfinite(a), a, 0.0),
+                  np.where(np.isfinite(b), b, 0.0), TOL_GPU)
 
 
 def test_output_over_an_input_takes_the_whole_pass(override):

@@ -96,7 +96,10 @@ __device__ __forceinline__ float LaneGroupSum(float x) {
 //    C, no y): 5.4 of the 8.2 issue slots per state and token of a whole
 //    pass.  Writes each channel's sum of delta' and end state.
 //  * kSegOut: every segment from its true start state, the composition of the
-//    records of the segments before it (h <- exp2(A sum delta') h + h_end).
+//    records of the segments before it (h <- exp2(A sum delta') h + h_end).  An
+//    infinite state, whose decay over a segment may be 0 where no token's is,
+//    would not be the whole pass's: the workgroup then walks the sequence from
+//    its first token and stores only the segment's y.
 // The records live in the output rows that the later segments will write:
 // segment s's go into slot s of every later segment's rows, so a workgroup of
 // the second launch reads only rows that it alone overwrites, before its
@@ -135,6 +138,7 @@ __global__ __launch_bounds__(kThreads) void SelectiveScanFwdKernel(SelectiveScan
         tb = seg * split.len;
         te = min(L, tb + split.len);
     }
+    const int y_from = tb;                   // first token whose y this workgroup stores
     const int cb = wg % ncb;
     wg /= ncb;
     const int g = wg % p.groups_b;
@@ -387,6 +391,7 @@ __global__ __launch_bounds__(kThreads) void SelectiveScanFwdKernel(SelectiveScan
     // ---- phase 3: add D*u, store y -------------------------------------------
     auto phase3 = [&](int t0, bool full) __attribute__((always_inline)) {
         if constexpr (kState) return;
+        if (MODE == kSegOut && t0 < y_from) return;
 #pragma unroll
         for (int k = 0; k < IPT; ++k) {
             const int it = tid + k * kThreads;
@@ -407,7 +412,7 @@ __global__ __launch_bounds__(kThreads) void SelectiveScanFwdKernel(SelectiveScan
         // were last read before the previous barrier.
     };
 
-    const int nfull = FAST ? (te - tb) / kTile : 0;   // tiles taken on the unguarded path
+    int nfull = FAST ? (te - tb) / kTile : 0;   // tiles taken on the unguarded path
     // a full tile from one register set, prefetching the next tile into the other
     auto full_tile = [&](int i, const R4 (&u)[IPT], const R4 (&d)[IPT], const R4 (&bc)[BCPT], R4 (&nu)[IPT], R4 (&nd)[IPT],
                          R4 (&nbc)[BCPT]) __attribute__((always_inline)) {
@@ -429,8 +434,27 @@ __global__ __launch_bounds__(kThreads) void SelectiveScanFwdKernel(SelectiveScan
         __syncthreads();
         phase3(t0, true);
     };
+    if constexpr (MODE == kSegOut) {
+        if (nfull > 0) load_full(tb, uA, dA, bcA);   // before the wait for the records
+        bool finite = true;
+#pragma unroll
+        for (int j = 0; j < SPL; ++j) finite = finite && isfinite(h[j]);
+        const bool wave_finite = __ballot(!finite) == 0;
+        if (lane == 0) sY[tid / 64] = wave_finite ? 0.0f : 1.0f;   // next written behind phase 1's barrier
+        __syncthreads();
+        bool walk = false;
+#pragma unroll
+        for (int i = 0; i < kThreads / 64; ++i) walk = walk || sY[i] != 0.0f;
+        if (__builtin_amdgcn_readfirstlane(walk)) {
+            tb = 0;
+            nfull = FAST ? te / kTile : 0;
+#pragma unroll
+            for (int j = 0; j < SPL; ++j) h[j] = 0.0f;
+            if (nfull > 0) load_full(0, uA, dA, bcA);
+        }
+    }
     if (nfull > 0) {   // the only path into the full-tile loop
-        load_full(tb, uA, dA, bcA);
+        if constexpr (MODE != kSegOut) load_full(tb, uA, dA, bcA);
         // A tile is entered with its loads issued before the previous tile's
         // IPT stores (vmcnt counts both).  Dropped stores (beyond the
         // descriptor) after tile 0's loads give the first entry the same
