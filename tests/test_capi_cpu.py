@@ -277,6 +277,35 @@ def test_wrong_input_count():
         validate("selective_scan", ss_shapes()[:7])
 
 
+class _LooksLikeATensor:
+    """Not a tensor, but with what the descriptors are made from."""
+    shape = (2, 8, 16)
+    is_cuda = True
+    dtype = None
+
+    def data_ptr(self):
+        return 16
+
+    def numel(self):
+        return 256
+
+    def is_contiguous(self):
+        return True
+
+
+def test_front_end_refuses_what_is_no_device_tensor():
+    import torch
+    import xmetai_onnx_plugins as xp
+    t = torch.zeros(2, 8, 16)
+    with pytest.raises(TypeError, match="inputs must be torch tensors or None"):
+        xp.selective_scan_fn(_LooksLikeATensor(), t, t, t, t)
+    with pytest.raises(TypeError, match="inputs must be torch tensors or None"):
+        xp.selective_scan_fn(t.numpy(), t, t, t, t)
+    for x in (t, t.to_sparse(), t.transpose(1, 2)):   # a sparse tensor has no address to ask for
+        with pytest.raises(XmError, match="inputs must be device tensors"):
+            xp.selective_scan_fn(x, t, t, t, t)
+
+
 # ---------------------------------------------------------------------------
 # GatedDeltaNet2Fn shapes
 # ---------------------------------------------------------------------------

@@ -165,32 +165,33 @@ def _pack_inputs(inputs) -> bytearray:
             _XM_TENSOR.pack_into(buf, pos, 0, 0, *_PAD[1], 1, _capi.XM_ELEM_FLOAT)
             pos += size
             continue
-        try:
-            shape, ptr = x.shape, x.data_ptr()
-        except AttributeError:
-            raise TypeError("inputs must be torch tensors or None") from None
-        rank = len(shape)
-        if rank > _capi.XM_MAX_RANK:
-            raise XmError(XM_ERR_INVALID_ARGUMENT, "tensor rank out of range")
+        if not isinstance(x, _tensor_type):
+            raise TypeError("inputs must be torch tensors or None")
+        ptr = 0
         if x.numel() > 0:
             if not x.is_cuda:
                 raise XmError(XM_ERR_INVALID_ARGUMENT, "inputs must be device tensors")
             if not x.is_contiguous():
                 raise XmError(XM_ERR_INVALID_ARGUMENT, "inputs must be contiguous (row-major)")
-        else:
-            ptr = 0
+            ptr = x.data_ptr()
+        shape = x.shape
+        rank = len(shape)
+        if rank > _capi.XM_MAX_RANK:
+            raise XmError(XM_ERR_INVALID_ARGUMENT, "tensor rank out of range")
         _XM_TENSOR.pack_into(buf, pos, ptr, *shape, *_PAD[rank], rank, elems.get(x.dtype, 0))
         pos += size
     return buf
 
 
 _elem_map = None
+_tensor_type = None   # torch.Tensor, set with the map (torch is imported on first use)
 
 
 def _elem_types():
-    global _elem_map
+    global _elem_map, _tensor_type
     if _elem_map is None:
         import torch
+        _tensor_type = torch.Tensor
         _elem_map = {torch.float32: _capi.XM_ELEM_FLOAT, torch.int64: _capi.XM_ELEM_INT64,
                      torch.float16: _capi.XM_ELEM_FLOAT16, torch.bfloat16: _capi.XM_ELEM_BFLOAT16}
     return _elem_map
