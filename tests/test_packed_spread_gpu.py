@@ -78,3 +78,36 @@ def test_gdn2_tiles_by_length_equal_both_layouts_bitwise(dk, dv, offsets, overri
         override("gdn2_ct", ct)
         fixed = xp.gated_deltanet2_fn(*dev, scale=s.scale, cu_seqlens=cu)
         assert np.array_equal(got.cpu().numpy(), fixed.cpu().numpy())
+
+
+def many_lengths(kind):
+    rng = np.random.default_rng(7)
+    ln = rng.integers(0, 40, 150)
+    if kind != "short":
+        ln[{"long_first": 0, "long_middle": 70, "long_last": 149}[kind]] = 3000
+    return ln
+
+
+@pytest.mark.parametrize("kind", ["short", "long_first", "long_middle", "long_last"])
+@pytest.mark.parametrize("heads,dk,dv,windowed", [(16, 64, 64, False), (23, 128, 40, False), (16, 64, 64, True)])
+def test_gdn2_many_sequences_equal_both_layouts_bitwise(kind, heads, dk, dv, windowed, override):
+    """150 sequences, some empty: the launch has the two-tile workgroups only, and
+    with one long sequence among them, which is stepped a tile at a time, each
+    takes two sequences.  Outputs and final states are the fixed layouts'."""
+    off = np.concatenate([[0], np.cumsum(many_lengths(kind))]).astype(np.int64)
+    s = W.GatedDeltaNet2Shape(1, int(off[-1]) + 3, heads, dk, dv, initial_state=False)
+    inp = W.gated_deltanet2_inputs(s, seed=54)
+    dev = [to_dev(inp[k]) for k in ("q", "k", "v", "g", "beta", "w")]
+    start = to_dev(np.random.default_rng(8).standard_normal((150, heads, dk, dv)).astype(np.float32))
+    override("gdn2_windowed", int(windowed))
+    out = {}
+    for ct in (0, 1, 2):
+        override("gdn2_ct", ct)
+        y, f = xp.gated_deltanet2_fn(*dev, start, scale=s.scale, cu_seqlens=to_dev(off), output_final_state=True)
+        out[ct] = (y.cpu().numpy(), f.cpu().numpy())
+        tag = [k for k in xp.last_launches() if k.startswith("Gdn2ChunkRecurKernel<")]
+        assert tag and all(f",{ct},1>" in k for k in tag), xp.last_launches()
+    for ct in (1, 2):
+        for a, b in zip(out[0], out[ct]):
+            np.testing.assert_array_equal(a, b)
+    assert not out[0][0][0, off[-1]:].any()

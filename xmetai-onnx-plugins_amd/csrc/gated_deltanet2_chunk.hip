@@ -240,8 +240,12 @@ __device__ __forceinline__ void PairwiseAM(const GatedDeltaNet2Params &p, size_t
     }
 }
 
-// Largest b with off[b] <= g (off non-decreasing over [0, n], off[0] = 0 <= g
-// < off[n]): the packed sequence that holds global chunk g.
+// The first block of packed sequence b in the window's table, whose first entry
+// is 0 or, for two column tiles per workgroup, kTwoTilesBit.
+constexpr int kTwoTilesBit = static_cast<int>(0x80000000u);
+__device__ __forceinline__ int ChunkStart(const GatedDeltaNet2Params &p, int b) { return p.chunk_off[b] & ~kTwoTilesBit; }
+// Largest b with off[b] <= g (off non-decreasing over [1, n], off[0] counting
+// as 0 <= g < off[n]): the packed sequence that holds global chunk g.
 __device__ __forceinline__ int SequenceOfChunk(const int *off, int n, int g) {
     int lo = 0, hi = n;
     while (hi - lo > 1) {
@@ -300,7 +304,7 @@ __global__ __launch_bounds__(64 * PW) void Gdn2ChunkPrepKernel(GatedDeltaNet2Par
         if (cw >= p.chunk_off[p.batch]) return;   // past the window's blocks: never read
         const int b = SequenceOfChunk(p.chunk_off, p.batch, cw);
         PackedRange(p, b, tok0, T);
-        t0 = (c0 + cw - p.chunk_off[b]) * kC;
+        t0 = (c0 + cw - ChunkStart(p, b)) * kC;
     }
     const bool live = t0 + m16 < T;
     const size_t rowbase = ((tok0 + min(t0 + m16, T - 1)) * H + h) * p.dk;
@@ -970,13 +974,14 @@ __device__ __forceinline__ void Gdn2PackedRecur(const GatedDeltaNet2Params &p, f
     using L = RecurLayout<KPW, KS, CT>;
     const int H = p.nheads, n = p.batch;
     const size_t kv = static_cast<size_t>(p.dk) * p.dv;
-    const int slots = min(n, wn);
+    // as many as the launch has workgroups for (LaunchRecur)
+    const int slots = min(min(n, wn), static_cast<int>(gridDim.x) / kNumXcds / vw * kNumXcds / H);
     const XcdUnit u = XcdSpreadUnit(blockIdx.x, vw);
     const int slot = u.unit / H, h = u.unit % H;
     if (slot >= slots) return;
     const float *const prep_row = p.prepared + static_cast<size_t>(h) * wn * L::FB;
     for (int b = slot; b < n; b += slots) {   // workgroup-uniform
-        const int i0 = p.chunk_off[b], nrun = p.chunk_off[b + 1] - i0;
+        const int i0 = ChunkStart(p, b), nrun = p.chunk_off[b + 1] - i0;
         if (nrun <= 0) continue;   // no chunks in this window
         size_t tok0;
         int T;
@@ -998,19 +1003,16 @@ __device__ __forceinline__ void Gdn2PackedRecur(const GatedDeltaNet2Params &p, f
 // 128 x 128: 5000 tokens x 16 heads, longest of 7 sequences 1636 188 / 234, even
 // 195 / 178; 4000 x 8 heads in 5 114 / 164; 16384 x 16 in 16, ragged 587 / 573;
 // 64 x 64, 4000 x 16 in 5 104 / 159; 256 x 256, 4000 x 8 in 6 221 / 310.
+// Gdn2PackedChunksKernel decides, once a window: every workgroup here looking
+// through all lengths made 4096 sequences of 8 tokens x 8 heads 1.36 -> 4.26 ms.
 constexpr int kCus = 256;
-__device__ __forceinline__ bool PackedTwoTiles(const GatedDeltaNet2Params &p, int vt) {
-    int longest = 0;
-    for (int b = threadIdx.x & 63; b < p.batch; b += 64) longest = max(longest, p.chunk_off[b + 1] - p.chunk_off[b]);
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) longest = max(longest, __shfl_xor(longest, o));
-    const float chain = static_cast<float>(__builtin_amdgcn_readfirstlane(longest));
-    const float work = static_cast<float>(p.chunk_off[p.batch]) * p.nheads * vt / kCus;
+__device__ __forceinline__ bool PackedTwoTiles(int longest, int total, int nheads, int vt) {   // in chunks
+    const float chain = static_cast<float>(longest);
+    const float work = static_cast<float>(total) * nheads * vt / kCus;
     return fmaxf(120.0f * chain, 60.0f * work) < fmaxf(72.0f * chain, 70.0f * work);
 }
 
-// CT: value-column tiles per workgroup; 0 (packed): one or two, by the lengths
-// (the launch has the one-tile workgroups; two tiles leave the last ones idle).
+// CT: value-column tiles per workgroup; 0 (packed): one or two, by the lengths.
 template <int KPW, int KS, int CT, bool PACKED>
 __global__ __launch_bounds__(64 * KS) void Gdn2ChunkRecurKernel(GatedDeltaNet2Params p, int c0, int wn,
                                                                 const float *s_in, float *s_out) {
@@ -1028,7 +1030,7 @@ __global__ __launch_bounds__(64 * KS) void Gdn2ChunkRecurKernel(GatedDeltaNet2Pa
                                   s_in, s_out, SplitTile{wg % VW, false, nullptr});
     } else if constexpr (CT != 0) {
         Gdn2PackedRecur<KPW, KS, CT>(p, sXp, c0, wn, (VT + CT - 1) / CT);
-    } else if (PackedTwoTiles(p, VT)) {
+    } else if (p.chunk_off[0] != 0) {   // kTwoTilesBit
         Gdn2PackedRecur<KPW, KS, 2>(p, sXp, c0, wn, (VT + 1) / 2);
     } else {
         Gdn2PackedRecur<KPW, KS, 1>(p, sXp, c0, wn, VT);
@@ -1570,6 +1572,12 @@ void LaunchPrep(const ChunkConfig &c, const GatedDeltaNet2Params &p, int c0, int
     }
 }
 
+// Packed by length, at least 64 sequences: from this many two-tile workgroups
+// (16 per CU) the launch has only those.  Idle ones cost more than the coarser
+// one-tile slots lose there: 128 x 128, 1024 sequences of 16 tokens x 16 heads 809 ->
+// 764 us (two tiles always: 770), one of 8192 tokens among 1023 of 8 x 8 heads
+// 584 (one tile always 591, two 768); 64 of 256 x 16 heads 474 -> 477.
+constexpr long long kManyBlocks = 16 * 256;
 template <int KPW, int KS, int CT>
 void LaunchRecur(const GatedDeltaNet2Params &p, int c0, int wn, int kq, const float *s_in, float *s_out,
                  hipStream_t stream) {
@@ -1577,10 +1585,15 @@ void LaunchRecur(const GatedDeltaNet2Params &p, int c0, int wn, int kq, const fl
     // packed, two tiles by the dispatcher's choice: the kernel looks at the lengths
     constexpr int PCT = CT == 2 ? 0 : CT;
     const bool by_length = p.chunk_off != nullptr && CT == 2 && GetOverride(kOverrideGdn2Ct) == 0;
-    const int vt = by_length ? (p.dv + 15) / 16 : ((p.dv + 15) / 16 + CT - 1) / CT;   // workgroups per (b, h)
     // packed: min(sequences, chunks) slots per (h, column tile); a slot's
     // workgroup takes every slots-th sequence that meets the window
     const long long rows = p.chunk_off != nullptr ? std::min(p.batch, wn) : p.batch;
+    // By length: the one-tile workgroups, of which two tiles leave half idle; with
+    // many sequences the two-tile ones (kManyBlocks), and one tile takes two
+    // sequences per slot.
+    const int tiles = (p.dv + 15) / 16;
+    const bool many = rows >= 64 && rows * p.nheads * ((tiles + 1) / 2) >= kManyBlocks;
+    const int vt = by_length && !many ? tiles : (tiles + CT - 1) / CT;   // workgroups per (b, h)
     const long long blocks = rows * p.nheads * vt;
     if (blocks == 0) return;   // no packed sequences
     if (blocks > 2147483647LL) throw Error(XM_ERR_INVALID_ARGUMENT, "GatedDeltaNet2Fn launch exceeds the grid limit");
@@ -1896,7 +1909,9 @@ WindowPlan PlanWindows(int batch, int seqlen, int nheads, int dk, int dv, bool p
 
 // Packed sequences: for every window w, offs[w][b] = the chunks in [w win,
 // (w + 1) win) of sequences 0..b-1 (b = 0..n): where sequence b's blocks of
-// window w start.  An empty sequence, which no recurrence workgroup visits,
+// window w start; the sign of offs[w][0], which is 0 otherwise, is set where the
+// recurrence takes two column tiles per workgroup (PackedTwoTiles).  An empty
+// sequence, which no recurrence workgroup visits,
 // passes its initial state (zeros without one) to final_state here.  All of
 // that is workgroup 0; the others zero the output rows that no sequence covers
 // (a launch of its own took 4.7 us of a 215 us call).
@@ -1906,8 +1921,8 @@ __global__ __launch_bounds__(256) void Gdn2PackedChunksKernel(GatedDeltaNet2Para
                        gridDim.x - 1);
         return;
     }
-    __shared__ int part[256];
-    const int n = p.batch, tid = threadIdx.x;
+    __shared__ int part[256], most[256];
+    const int n = p.batch, tid = threadIdx.x, vt = (p.dv + 15) / 16;
     const int per = (n + 255) / 256;
     const int b0 = min(n, tid * per), b1 = min(n, b0 + per);
     auto chunks = [&](int b) {
@@ -1919,9 +1934,15 @@ __global__ __launch_bounds__(256) void Gdn2PackedChunksKernel(GatedDeltaNet2Para
     for (int w = 0; w < nwin; ++w) {   // workgroup-uniform
         int *const off = offs + static_cast<size_t>(w) * (n + 1);
         auto in_window = [&](int b) { return min(max(chunks(b) - w * win, 0), win); };
-        int sum = 0;
-        for (int b = b0; b < b1; ++b) sum += in_window(b);
+        int sum = 0, longest = 0;
+        bool two = false;   // thread 0, which writes offs[w][0]
+        for (int b = b0; b < b1; ++b) {
+            const int c = in_window(b);
+            sum += c;
+            longest = max(longest, c);
+        }
         part[tid] = sum;
+        most[tid] = longest;
         __syncthreads();
         if (tid == 0) {   // exclusive prefix of the partial sums in use
             int acc = 0;
@@ -1929,13 +1950,15 @@ __global__ __launch_bounds__(256) void Gdn2PackedChunksKernel(GatedDeltaNet2Para
                 const int v = part[i];
                 part[i] = acc;
                 acc += v;
+                longest = max(longest, most[i]);
             }
             off[n] = acc;
+            two = PackedTwoTiles(longest, acc, p.nheads, vt);
         }
         __syncthreads();
         int acc = part[tid];
         for (int b = b0; b < b1; ++b) {
-            off[b] = acc;
+            off[b] = two && b == 0 ? kTwoTilesBit : acc;
             acc += in_window(b);
         }
         __syncthreads();   // part is rewritten by the next window

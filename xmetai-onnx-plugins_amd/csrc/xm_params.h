@@ -54,7 +54,8 @@ struct GatedDeltaNet2Params {
     // seqlen tokens (the tensors' batch dimension is 1), or nullptr.
     const int64_t *cu_seqlens;
     // Chunked path with packed sequences: [batch + 1] prefix sums of the
-    // sequences' 16-token chunk counts (device scratch), or nullptr.
+    // sequences' 16-token chunk counts (device scratch; the first carries
+    // kTwoTilesBit), or nullptr.
     const int *chunk_off;
 };
 
