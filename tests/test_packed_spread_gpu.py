@@ -111,3 +111,27 @@ def test_gdn2_many_sequences_equal_both_layouts_bitwise(kind, heads, dk, dv, win
         for a, b in zip(out[0], out[ct]):
             np.testing.assert_array_equal(a, b)
     assert not out[0][0][0, off[-1]:].any()
+
+
+@pytest.mark.parametrize("windowed", [False, True])
+def test_gdn2_table_of_many_sequences(windowed, override):
+    """700 sequences (three to a thread of the launch that builds the chunk table),
+    empty ones among them, in one call and in two."""
+    ln = np.random.default_rng(9).integers(0, 6, 700)
+    ln[[0, 255, 256, 699]] = [0, 90, 0, 2100]
+    off = np.concatenate([[0], np.cumsum(ln)]).astype(np.int64)
+    s = W.GatedDeltaNet2Shape(1, int(off[-1]), 4, 64, 48, initial_state=False)
+    inp = W.gated_deltanet2_inputs(s, seed=55)
+    dev = [to_dev(inp[k]) for k in ("q", "k", "v", "g", "beta", "w")]
+    start = to_dev(np.random.default_rng(10).standard_normal((700, 4, 64, 48)).astype(np.float32))
+    override("gdn2_windowed", int(windowed))
+
+    def call(a, b):
+        y, f = xp.gated_deltanet2_fn(*(x[:, off[a]:off[b]].contiguous() for x in dev), start[a:b].contiguous(),
+                                     scale=s.scale, cu_seqlens=to_dev(off[a:b + 1] - off[a]), output_final_state=True)
+        return y.cpu().numpy(), f.cpu().numpy()
+    y, f = call(0, 700)
+    parts = [call(0, 301), call(301, 700)]
+    np.testing.assert_array_equal(y, np.concatenate([x[0] for x in parts], axis=1))
+    np.testing.assert_array_equal(f, np.concatenate([x[1] for x in parts]))
+    np.testing.assert_array_equal(f[ln == 0], start.cpu().numpy()[ln == 0])

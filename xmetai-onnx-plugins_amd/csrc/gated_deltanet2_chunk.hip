@@ -1910,67 +1910,73 @@ WindowPlan PlanWindows(int batch, int seqlen, int nheads, int dk, int dv, bool p
 // Packed sequences: for every window w, offs[w][b] = the chunks in [w win,
 // (w + 1) win) of sequences 0..b-1 (b = 0..n): where sequence b's blocks of
 // window w start; the sign of offs[w][0], which is 0 otherwise, is set where the
-// recurrence takes two column tiles per workgroup (PackedTwoTiles).  An empty
-// sequence, which no recurrence workgroup visits,
-// passes its initial state (zeros without one) to final_state here.  All of
-// that is workgroup 0; the others zero the output rows that no sequence covers
-// (a launch of its own took 4.7 us of a 215 us call).
+// recurrence takes two column tiles per workgroup (PackedTwoTiles).  All of that
+// is workgroup 0; the others zero the output rows that no sequence covers (a
+// launch of its own took 4.7 us of a 215 us call) and pass the initial state
+// (zeros without one) of an empty sequence, which no recurrence workgroup
+// visits, to final_state.  Scans by lane exchange: one thread adding 256 partial
+// sums, and one workgroup looking at the sequences one by one for empty ones,
+// took 65 us for 252 sequences (4 now).
 __global__ __launch_bounds__(256) void Gdn2PackedChunksKernel(GatedDeltaNet2Params p, int *offs, int win, int nwin) {
-    if (blockIdx.x > 0) {
-        ZeroPackedGaps(p.out, static_cast<size_t>(p.nheads) * p.dv, p.cu_seqlens, p.batch, p.seqlen, blockIdx.x - 1,
-                       gridDim.x - 1);
-        return;
-    }
-    __shared__ int part[256], most[256];
-    const int n = p.batch, tid = threadIdx.x, vt = (p.dv + 15) / 16;
-    const int per = (n + 255) / 256;
-    const int b0 = min(n, tid * per), b1 = min(n, b0 + per);
+    const int n = p.batch, tid = threadIdx.x;
     auto chunks = [&](int b) {
         size_t tok0;
         int T;
         PackedRange(p, b, tok0, T);
         return (T + kC - 1) / kC;
     };
-    for (int w = 0; w < nwin; ++w) {   // workgroup-uniform
-        int *const off = offs + static_cast<size_t>(w) * (n + 1);
-        auto in_window = [&](int b) { return min(max(chunks(b) - w * win, 0), win); };
-        int sum = 0, longest = 0;
-        bool two = false;   // thread 0, which writes offs[w][0]
-        for (int b = b0; b < b1; ++b) {
-            const int c = in_window(b);
-            sum += c;
-            longest = max(longest, c);
-        }
-        part[tid] = sum;
-        most[tid] = longest;
-        __syncthreads();
-        if (tid == 0) {   // exclusive prefix of the partial sums in use
-            int acc = 0;
-            for (int i = 0; i * per < n; ++i) {
-                const int v = part[i];
-                part[i] = acc;
-                acc += v;
-                longest = max(longest, most[i]);
-            }
-            off[n] = acc;
-            two = PackedTwoTiles(longest, acc, p.nheads, vt);
-        }
-        __syncthreads();
-        int acc = part[tid];
-        for (int b = b0; b < b1; ++b) {
-            off[b] = two && b == 0 ? kTwoTilesBit : acc;
-            acc += in_window(b);
-        }
-        __syncthreads();   // part is rewritten by the next window
-    }
-    if (p.final_state != nullptr) {
+    if (blockIdx.x > 0) {
+        const int wg = blockIdx.x - 1, nwg = gridDim.x - 1;
+        ZeroPackedGaps(p.out, static_cast<size_t>(p.nheads) * p.dv, p.cu_seqlens, p.batch, p.seqlen, wg, nwg);
+        if (p.final_state == nullptr) return;
         const size_t hkv = static_cast<size_t>(p.nheads) * p.dk * p.dv;
-        for (int b = 0; b < n; ++b) {   // workgroup-uniform
+        for (int b = wg; b < n; b += nwg) {   // workgroup-uniform
             if (chunks(b) > 0) continue;
             float *dst = p.final_state + static_cast<size_t>(b) * hkv;
             const float *src = p.initial_state != nullptr ? p.initial_state + static_cast<size_t>(b) * hkv : nullptr;
             for (size_t i = tid; i < hkv; i += 256) dst[i] = src != nullptr ? src[i] : 0.0f;
         }
+        return;
+    }
+    __shared__ int part[4], most[4];   // per wave: chunks, the longest sequence's
+    const int lane = tid & 63, wave = tid >> 6;
+    const int per = (n + 255) / 256;
+    const int b0 = min(n, tid * per), b1 = min(n, b0 + per);
+    for (int w = 0; w < nwin; ++w) {   // workgroup-uniform
+        int *const off = offs + static_cast<size_t>(w) * (n + 1);
+        auto in_window = [&](int b) { return min(max(chunks(b) - w * win, 0), win); };
+        int sum = 0, longest = 0;
+        for (int b = b0; b < b1; ++b) {
+            const int c = in_window(b);
+            sum += c;
+            longest = max(longest, c);
+        }
+        int incl = sum;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int x = __shfl_up(incl, o);
+            if (lane >= o) incl += x;
+            longest = max(longest, __shfl_xor(longest, o));
+        }
+        if (lane == 63) {
+            part[wave] = incl;
+            most[wave] = longest;
+        }
+        __syncthreads();
+        int acc = incl - sum, total = 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if (i < wave) acc += part[i];
+            total += part[i];
+            longest = max(longest, most[i]);
+        }
+        const bool two = PackedTwoTiles(longest, total, p.nheads, (p.dv + 15) / 16);
+        if (tid == 0) off[n] = total;
+        for (int b = b0; b < b1; ++b) {
+            off[b] = two && b == 0 ? kTwoTilesBit : acc;
+            acc += in_window(b);
+        }
+        __syncthreads();   // part is rewritten by the next window
     }
 }
 
@@ -2018,7 +2024,7 @@ bool LaunchGatedDeltaNet2Chunked(const GatedDeltaNet2Params &p, void *scratch, s
         q.state = carry;
         q.chunk_off = offs;
         XM_NOTE_LAUNCH("Gdn2PackedChunksKernel", {}, );
-        hipLaunchKernelGGL(Gdn2PackedChunksKernel, dim3(1u + std::min(p.seqlen, 255)), dim3(256), 0, stream, q, offs, win,
+        hipLaunchKernelGGL(Gdn2PackedChunksKernel, dim3(1u + std::max(1, std::min(p.seqlen, 255))), dim3(256), 0, stream, q, offs, win,
                            (nchunks + win - 1) / win);
         XM_LAUNCH_CHECK("GatedDeltaNet2Fn packed chunk offsets");
     }
