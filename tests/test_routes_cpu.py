@@ -1,4 +1,4 @@
-"""Which kernel a call takes where an output shares memory with an input, read
+"""Which kernel a call takes, where an output shares memory with an input above all, read
 from xm_last_launches without a GPU: the addresses are made up and nothing runs
 (so the file skips itself where a GPU is visible).  The runs on the GPU, for
 the cases whose result does not depend on the order of the workgroups, are in the
@@ -71,13 +71,13 @@ def test_m3_step_reads_its_tokens_four_at_a_time():
 
 
 def test_ss_segments_with_outputs_over_inputs():
-    """y or the last state over an input, or over each other: one launch of the whole pass, not two of segments."""
+    """y or the last state over an input, or over each other: one launch, not two of segments."""
     u, w, bc = (1, 5120, 2048), (5120, 16), (1, 1, 16, 2048)
     shapes = [u, u, w, bc, bc, (5120,), None, (5120,)]
     for at, two in (({}, True), ({0: (0, 0)}, False), ({1: (2, 0)}, False), ({1: (5, 0)}, False), ({0: (4, 64)}, False),
                     ({1: (7, 5120 * 4 - 4)}, False), ({1: (7, 5120 * 4)}, True)):
         got = launches("selective_scan", shapes, 2, at, return_last_state=1)
-        assert got == ["SelectiveScanFwdKernel"] * (2 if two else 1), (at, xp.last_launches())
+        assert (got == ["SelectiveScanFwdKernel"] * 2) == two and len(got) == 1 + two, (at, xp.last_launches())
 
 
 @pytest.mark.parametrize("at,refused", [(7, False), (0, True), (3, True)])
@@ -90,3 +90,30 @@ def test_noalloc_decode_of_many_heads(at, refused):
     st = xp.lib().xm_gated_deltanet2_forward_noalloc(ins, 7, ctypes.byref(a), (at + 1) << 34, None, err, len(err))
     assert (st == xp.XM_ERR_UNSUPPORTED) == refused, err.value
     assert xp.last_launches() == ([] if refused else ["Gdn2StepKernel<16,8>"])
+
+
+def ss_launches(b, d, l, n, elem=1, var_c=True):
+    row, bc, w = (b, d, l), (b, 1, n, l), (d, n)
+    shapes = [row, row, w, bc, bc if var_c else w, (d,), None, (d,)]
+    data = (0, 1, 3, 4) if var_c else (0, 1, 3)
+    ins = (_capi.XmTensor * 8)(*[xp._desc_from_shape(sh, (i + 1) << 34, elem if i in data else 1) if sh is not None
+                                 else xp._desc_from_tensor(None) for i, sh in enumerate(shapes)])
+    a, err = xp._attrs("selective_scan"), ctypes.create_string_buffer(512)
+    st = xp.lib().xm_selective_scan_forward(ins, 8, ctypes.byref(a), 9 << 34, None, None, err, len(err))
+    names = [k.split("<")[0] for k in xp.last_launches()]
+    return {("SelectiveScanFwdKernel",): "whole", ("SelectiveScanSegKernel",): "parallel",
+            ("SelectiveScanFwdKernel",) * 2: "segments"}[tuple(names)]
+
+
+@pytest.mark.parametrize("call,form", [   # where it was measured the cheapest by a quarter or more
+    ((1, 256, 512, 16), "parallel"), ((1, 1024, 1999, 16), "parallel"), ((1, 5120, 1999, 16), "segments"),
+    ((1, 4096, 1001, 16), "segments"), ((2, 4096, 1999, 16, _capi.XM_ELEM_BFLOAT16), "segments"),
+    ((1, 2048, 1999, 64), "segments"), ((1, 4096, 512, 8), "parallel"), ((8, 5120, 2048, 16), "whole"),
+    # guarded accesses make the whole pass and the segments slower than the sequence-parallel kernel
+    ((8, 3403, 720, 3), "parallel"), ((2, 964, 5616, 8, _capi.XM_ELEM_FLOAT16), "parallel"),
+    # a constant C
+    ((7, 2971, 278, 1, _capi.XM_ELEM_FLOAT16, False), "parallel"), ((2, 12745, 1264, 1, _capi.XM_ELEM_BFLOAT16, False), "parallel"),
+    ((1, 5120, 255, 16), "whole"),
+], ids=str)
+def test_ss_form(call, form):
+    assert ss_launches(*call) == form, xp.last_launches()

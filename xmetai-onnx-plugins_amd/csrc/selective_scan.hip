@@ -27,6 +27,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstdint>
 #include <cstdlib>
 #include <type_traits>
@@ -519,19 +520,30 @@ __global__ __launch_bounds__(kThreads) void SelectiveScanFwdKernel(SelectiveScan
     }
 }
 
-// Lanes per channel and states per lane, with what the forms cost (fp32, one
-// MI355X, interleaved runs of 256 to 4096 tokens at 256 to 20480 channels):
-// the whole pass per token while it has at most one workgroup per CU (ns), the
-// sequence-parallel kernel and the segments per channel and token (ps).
+// Lanes per channel and states per lane, with what the forms cost with variable
+// B and C (one MI355X, fitted to 480 runs of 1 to 330 channel blocks x 256 to
+// 8192 tokens, fp32 and 16-bit; the fits are within 3 to 10% for the whole pass
+// and the segments, up to 20% to 4 states, and 7 to 15% for the
+// sequence-parallel kernel).  [0]: unguarded accesses (FAST), [1]: guarded.
+// 2 x 4, 4 x 4 and 16 x 1 run only under the ss_lpc override.
 struct Config {
     int lpc, spl;
-    float whole_ns, seg_ps, split_ps;
+    float whole_ns[2];   // the whole pass, per token
+    float walk_us, start_us, seq_ps;   // sequence-parallel kernel: per walk, per 1000 channels, per channel and token
+    float split_ps[2];   // segments that fill the chip, per channel and token
+    float chain_ns[2];   // segments that do not, per token of one
 };
 constexpr Config kConfigs[] = {
-    {1, 4, 137.0f, 3.7f, 6.3f},     {2, 4, 105.0f, 5.6f, 5.0f},   {4, 2, 58.0f, 5.6f, 4.6f},
-    {4, 4, 80.0f, 10.0f, 7.5f},     {8, 2, 52.5f, 10.0f, 6.6f},   {16, 1, 45.0f, 10.0f, 9.0f},
-    {8, 4, 81.5f, 18.5f, 11.3f},    {16, 4, 97.0f, 89.0f, 29.0f}, {16, 8, 272.0f, 232.0f, 60.0f},
-    {16, 16, 545.0f, 460.0f, 120.0f},
+    {1, 4, {146.0f, 310.0f}, 0.6f, 0.5f, 2.9f, {6.3f, 10.5f}, {250.0f, 470.0f}},
+    {2, 4, {105.0f, 160.0f}, 0.85f, 0.5f, 4.8f, {5.5f, 9.0f}, {180.0f, 260.0f}},
+    {4, 2, {57.0f, 88.0f}, 0.85f, 0.5f, 4.8f, {4.6f, 8.2f}, {98.0f, 140.0f}},
+    {4, 4, {80.0f, 112.0f}, 1.4f, 0.9f, 8.5f, {8.0f, 11.0f}, {125.0f, 160.0f}},
+    {8, 2, {51.0f, 73.0f}, 1.4f, 0.9f, 8.5f, {6.4f, 9.2f}, {80.0f, 103.0f}},
+    {16, 1, {45.0f, 64.0f}, 1.4f, 0.9f, 8.5f, {9.0f, 12.0f}, {70.0f, 90.0f}},
+    {8, 4, {84.0f, 112.0f}, 1.55f, 1.0f, 15.5f, {11.8f, 12.8f}, {145.0f, 160.0f}},
+    {16, 4, {96.0f, 127.0f}, 3.0f, 1.5f, 85.0f, {27.0f, 33.0f}, {160.0f, 203.0f}},
+    {16, 8, {262.0f, 347.0f}, 6.0f, 0.0f, 180.0f, {130.0f, 99.0f}, {430.0f, 555.0f}},
+    {16, 16, {924.0f, 1085.0f}, 15.0f, 0.0f, 400.0f, {344.0f, 230.0f}, {1400.0f, 1590.0f}},
 };
 Config Layout(int lpc, int spl) {
     for (const Config &c : kConfigs)
@@ -592,19 +604,27 @@ void LaunchLSV(const SelectiveScanParams &p, const SegSplit &split, unsigned blo
 }
 
 template <typename IT, int LPC, int SPL>
-void LaunchLS(const SelectiveScanParams &p, int vec, const SegSplit &split, unsigned blocks, hipStream_t stream) {
-    constexpr int CPW = kThreads / LPC;
-    // the fast path's row descriptors span a workgroup's CPW rows: under 2 GiB
-    const bool rows_fit = static_cast<long long>(CPW) * p.seqlen * static_cast<long long>(sizeof(IT)) < (1LL << 31);
-    if (vec && rows_fit && p.dim_per_group % CPW == 0) LaunchLSV<IT, LPC, SPL, true>(p, split, blocks, stream);
+void LaunchLS(const SelectiveScanParams &p, bool vec, const SegSplit &split, unsigned blocks, hipStream_t stream) {
+    if (vec) LaunchLSV<IT, LPC, SPL, true>(p, split, blocks, stream);
     else LaunchLSV<IT, LPC, SPL, false>(p, split, blocks, stream);
+}
+
+// Every row of the data tensors on a 4-byte boundary: four tokens an access.
+bool AllDwordRows(const SelectiveScanParams &p) {
+    const size_t row = static_cast<size_t>(p.seqlen) * (p.in_type == XM_ELEM_FLOAT ? 4 : 2);
+    return DwordRows(p.u, row) && DwordRows(p.delta, row) && DwordRows(p.out, row) && (!p.b_var || DwordRows(p.B, row)) &&
+           (!p.c_var || DwordRows(p.C, row));
+}
+
+// The fast path of the layout: its row descriptors span a workgroup's channels' rows, under 2 GiB.
+bool FastRows(const SelectiveScanParams &p, int cpw) {
+    const long long row = static_cast<long long>(p.seqlen) * (p.in_type == XM_ELEM_FLOAT ? 4 : 2);
+    return AllDwordRows(p) && cpw * row < (1LL << 31) && p.dim_per_group % cpw == 0;
 }
 
 template <typename IT>
 void LaunchTyped(const SelectiveScanParams &p, const Config &cfg, const SegSplit &split, unsigned blocks, hipStream_t stream) {
-    const size_t row = static_cast<size_t>(p.seqlen) * sizeof(IT);
-    const int vec = DwordRows(p.u, row) && DwordRows(p.delta, row) && DwordRows(p.out, row) &&
-                    (!p.b_var || DwordRows(p.B, row)) && (!p.c_var || DwordRows(p.C, row));
+    const bool vec = FastRows(p, kThreads / cfg.lpc);
     switch (cfg.lpc * 100 + cfg.spl) {
         case 104: LaunchLS<IT, 1, 4>(p, vec, split, blocks, stream); break;
         case 204: LaunchLS<IT, 2, 4>(p, vec, split, blocks, stream); break;
@@ -677,13 +697,16 @@ struct SsPlan {
 // block), the sequence-parallel kernel (one workgroup per channel, 1.3 to 1.8
 // times the arithmetic), or segments of the whole pass (1.6 times, two
 // launches).  With fewer blocks than CUs the whole pass takes its chain's
-// time whatever the channels, the other two grow with the channels; the
-// cheapest by the layout's measured costs runs.  Measured us, whole /
-// sequence-parallel / segments: 1 x 5120 x 1999 107 / 114 / 78, 1 x 2048 x
-// 4096 209 / 88 / 72, 1 x 1024 x 2047 107 / 29 / 33, 1 x 7168 x 512 29 / 44 /
-// 33; 64 states, 1 x 2048 x 2048 199 / 375 / 134.  Above one block per CU a
-// CU steps two (1.4 times the chain); there only 16-bit data gains from
-// segments (their reads are half the bytes): 5 x 2048 x 1024 76 -> 69.
+// time whatever the channels, the other two grow with the channels.  With
+// variable B and C the cheapest by the layout's costs runs; with constant ones
+// (no segments; the whole pass is 0.2 to 0.9 of its cost, the sequence-parallel
+// kernel 0.2 to 0.95) the sequence-parallel kernel wherever there are fewer
+// blocks than CUs.  Measured us, whole / sequence-parallel / segments: 1 x 5120
+// x 1999 105 / 102 / 78, 1 x 4096 x 1001 56 / 51 / 39, 1 x 1024 x 1999 106 / 27 /
+// 35, 1 x 7168 x 512 30 / 42 / 33; bfloat16 rows off 4 bytes, 2 x 4096 x 1999 163 /
+// 468 / 126; guarded, 2 x 12745 x 1264 with one state and constant C 423 / 130 / -;
+// 64 states, 1 x 2048 x 1999 193 / 486 / 132.  Over 480 such runs the rule's
+// choice takes 0.6% more than the best form on average (geometric mean).
 // ss_split override: 1 the whole pass, 2 the sequence-parallel kernel, 3
 // segments wherever the rows hold their records.
 SsPlan ChoosePlan(const SelectiveScanParams &p, const Config &cfg, long long blocks, int64_t forced) {
@@ -693,18 +716,30 @@ SsPlan ChoosePlan(const SelectiveScanParams &p, const Config &cfg, long long blo
     if (forced == 2) return {seg_fits, whole};
     if (forced == 3) return {false, splits ? FitSegments(p, kSplitMax, 32) : whole};
     if (blocks > kSplitMaxChannelBlocks || p.seqlen < kSegMinSeqlen) return {false, whole};
-    const SegSplit split = splits ? FitSegments(p, kSplitTarget / blocks, kSplitMinLen) : whole;
-    const float ct = static_cast<float>(p.batch) * static_cast<float>(p.dim) * 1e-6f;   // us per ps and token
-    const float chain = cfg.whole_ns * 1e-3f;
-    const float t_whole = chain * p.seqlen * (blocks > kSegMaxChannelBlocks ? 1.4f : 1.0f);
-    // the sequence-parallel kernel walks blocks of 512 tokens (1024 to 4 states, 256 above 16)
-    const int walk = p.dstate <= 4 ? 1024 : (p.dstate <= 16 ? 512 : 256);
-    const float t_seg = 3.0f + cfg.seg_ps * ct * (static_cast<float>((p.seqlen + walk - 1) / walk) * walk);
-    const float t_split = 12.0f + std::max(cfg.split_ps * (p.in_type == XM_ELEM_FLOAT ? 1.0f : 0.85f) * ct * p.seqlen,
-                                           1.8f * chain * split.len);
     const bool seg_ok = seg_fits && blocks < kSegMaxChannelBlocks;
-    if (split.count > 1 && t_split < t_whole && (!seg_ok || t_split < t_seg)) return {false, split};
-    return {seg_ok && t_seg < t_whole, whole};
+    if (!p.b_var || !p.c_var) return {seg_ok, whole};
+    const SegSplit split = splits ? FitSegments(p, kSplitTarget / blocks, kSplitMinLen) : whole;
+    const bool f32 = p.in_type == XM_ELEM_FLOAT;
+    const int guarded = FastRows(p, kThreads / cfg.lpc) ? 0 : 1;
+    const float L = static_cast<float>(p.seqlen);
+    const float mch = static_cast<float>(p.batch) * static_cast<float>(p.dim) * 1e-6f;   // million channels: us per ps and token
+    // above one block per CU some CUs step two of them
+    const float t_whole = 3.0f + 1e-3f * cfg.whole_ns[guarded] * L * (blocks > kSegMaxChannelBlocks ? 1.45f : 1.0f);
+    // the sequence-parallel kernel walks blocks of 512 tokens (1024 to 4
+    // states, 256 above 16); above 32 states the tokens past the end cost little
+    const int walk = p.dstate <= 4 ? 1024 : (p.dstate <= 16 ? 512 : 256);
+    const long long walks = (static_cast<long long>(p.seqlen) + walk - 1) / walk;
+    const float seq_ps = cfg.seq_ps * (f32 ? 1.0f : (p.dstate <= 32 ? 0.8f : 0.6f));
+    // rows off 4 bytes are read token by token, lengths off 4 tokens with a mask
+    const float access = !AllDwordRows(p) ? (p.dstate <= 4 ? 2.3f : 3.0f) : (p.seqlen % 4 != 0 ? 1.08f : 1.0f);
+    const float t_seq = 2.5f + access * (cfg.walk_us * static_cast<float>(walks) +
+                                         mch * (1e3f * cfg.start_us + seq_ps * (p.dstate <= 32 ? static_cast<float>(walks * walk) : L)));
+    // the chip's rate or a segment's chain, whichever is longer (a soft maximum), and about 1 us a record to start from
+    const float fill = cfg.split_ps[guarded] * (!f32 && p.dstate <= 16 ? 0.9f : 1.0f) * mch * L;
+    const float chain = 1e-3f * cfg.chain_ns[guarded] * split.len;
+    const float t_split = 4.0f + split.count + std::cbrt(fill * fill * fill + chain * chain * chain);
+    if (split.count > 1 && t_split < t_whole && (!seg_ok || t_split < t_seq)) return {false, split};
+    return {seg_ok && t_seq < t_whole, whole};
 }
 
 }  // namespace
