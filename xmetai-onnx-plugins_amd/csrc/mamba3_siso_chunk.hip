@@ -329,19 +329,23 @@ __global__ __launch_bounds__(64 * (NW + NPW)) void Mamba3ChunkKernel(Mamba3SisoP
     const int nrb = (P + ROWS - 1) / ROWS;
     // the nrb workgroups of one (b,h) prepare the same token vectors: keep them on one XCD
     // (packed sequences: a sequence's heads over all XCDs, XcdSpreadUnit)
-    int wg = XcdLocalBlock(blockIdx.x, gridDim.x);
+    const int wg = XcdLocalBlock(blockIdx.x, gridDim.x);
     const int nseg_wg = MODE == kM3Whole ? 1 : (kState ? (split.maxseg - 1) * (split.ls / split.lf) : split.maxseg);
     const bool packed = PACKED == 1 || (PACKED == 2 && p.cu_seqlens != nullptr);
+    int rb = wg % nrb;
+    int seg = MODE == kM3Whole ? 0 : (wg / nrb) % nseg_wg;   // fine segment (kM3State) or output segment
+    int bh = wg / nrb / nseg_wg;
+    int b = bh / H, h = bh % H;
     if (packed) {
         const XcdUnit u = XcdSpreadUnit(blockIdx.x, nrb);   // units: sequence, segment, head
         const int run = u.unit / H;
         if (run >= p.batch * nseg_wg) return;
-        wg = ((run / nseg_wg * H + u.unit % H) * nseg_wg + run % nseg_wg) * nrb + u.part;
+        rb = u.part;
+        h = u.unit - run * H;
+        b = run / nseg_wg;
+        seg = run - b * nseg_wg;
+        bh = b * H + h;
     }
-    const int rb = wg % nrb;
-    const int seg = MODE == kM3Whole ? 0 : (wg / nrb) % nseg_wg;   // fine segment (kM3State) or output segment
-    const int bh = wg / nrb / nseg_wg;
-    const int b = bh / H, h = bh % H;
     const int gq = h / (H / p.nheads_qk);
     const int r0 = rb * ROWS;
     const float dval = p.D ? p.D[h] : 0.0f;
