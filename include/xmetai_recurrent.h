@@ -102,9 +102,10 @@ void xm_selective_scan_attrs_default(xm_selective_scan_attrs_t *attrs);
 int xm_selective_scan_check_attrs(const xm_selective_scan_attrs_t *attrs, char *errbuf, size_t errlen);
 /* Run-time shape validation without touching the device (reference:
  * Compute, :58-117).  Writes the output shape and the scratch bytes the call
- * will request from the allocator (GatedDeltaNet2Fn: at most; a call of up to
- * 16 tokens requests none, unless an output shares memory with q, k, g or beta
- * or overlaps v or w out of place). */
+ * will request from the allocator (GatedDeltaNet2Fn: at most; a call of a few
+ * tokens, up to 16, requests none where one launch takes it: not with an output
+ * over q, k, g, beta or a shifted part of v or w, nor with thousands of small
+ * heads, which take the chunked path from some tokens on). */
 int xm_selective_scan_validate(const xm_tensor_t *inputs, size_t n_inputs,
                                const xm_selective_scan_attrs_t *attrs, int64_t *out_shape,
                                int32_t *out_rank, size_t *scratch_bytes, char *errbuf, size_t errlen);
@@ -238,8 +239,8 @@ int xm_gated_deltanet2_forward_states(const xm_tensor_t *inputs, size_t n_inputs
  * library runs on holds until the process ends; the chunked path's windows
  * and the preparation chunks of head_k > 512 shrink to fit it, and a call that
  * cannot fit (e.g. a carried state of 64 MiB or more) fails with
- * XM_ERR_UNSUPPORTED before anything is enqueued.  A call of up to 16 tokens
- * that needs no scratch (above) never fails so.  It calls no hipMalloc or
+ * XM_ERR_UNSUPPORTED before anything is enqueued.  A call of a few
+ * tokens that one launch takes (above) uses no scratch and never fails so.  It calls no hipMalloc or
  * hipFree.  Every call on a GPU shares that GPU's array: calls that overlap on
  * one GPU (concurrent streams) race and must be serialised by the caller.
  * Results equal xm_gated_deltanet2_forward's, except where that call splits

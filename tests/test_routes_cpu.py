@@ -117,3 +117,18 @@ def ss_launches(b, d, l, n, elem=1, var_c=True):
 ], ids=str)
 def test_ss_form(call, form):
     assert ss_launches(*call) == form, xp.last_launches()
+
+
+def gdn2_launches(b, t, h, dk, dv):
+    k, v, s = (b, t, h, dk), (b, t, h, dv), (b, h, dk, dv)
+    return launches("gated_deltanet2", [k, k, v, k, k, v, s], 2, scale=1.0, output_final_state=1)
+
+
+@pytest.mark.parametrize("call,step", [
+    ((32, 16, 16, 128, 128), True), ((64, 16, 16, 64, 64), True), ((3072, 16, 1, 128, 64), True), ((1, 16, 4, 512, 8), True),
+    ((3072, 4, 1, 16, 16), True), ((3072, 8, 1, 16, 16), False), ((192, 12, 16, 32, 16), False), ((1024, 6, 1, 512, 16), True),
+    ((1024, 12, 1, 512, 16), False), ((2, 17, 2, 64, 64), False),
+], ids=str)
+def test_gdn2_step_or_chunked(call, step):
+    """Without a GPU the chunked path ends at its scratch, before any launch."""
+    assert gdn2_launches(*call) == (["Gdn2StepKernel"] if step else []), xp.last_launches()

@@ -26,6 +26,8 @@
 // us, the launch (22).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "xm_hip.h"
 #include "xm_matrix.h"
 #include "xm_params.h"
@@ -232,6 +234,25 @@ void LaunchStepKeys(const GatedDeltaNet2Params &p, hipStream_t stream) {
     else LaunchStep<CL, 512 / KG>(p, stream);
 }
 
+long long WideBlocks(const GatedDeltaNet2Params &p) {
+    return static_cast<long long>(p.batch) * p.nheads * ((p.dv + 63) / 64);
+}
+
+// With the chip full a block's tokens take turns, while the chunked path's time
+// hardly depends on how full its chunk is: many small heads are cheaper there
+// from some tokens on.  Both in us, fitted to 500 to 3072 heads of 16 to 512 keys
+// x 8 to 64 columns (within 15%).  Measured, chunked / here: 3072 heads of 16 x 16,
+// 4 tokens 23 / 18, 8 24 / 30, 16 23 / 54; of 128 x 64, 16 tokens 137 / 105; 1024 of
+// 512 x 16, 6 tokens 80 / 71, 12 88 / 118.  Above 384 keys the state leaves room
+// for two waves per SIMD.
+bool StepIsCheaper(const GatedDeltaNet2Params &p) {
+    const double dk = p.dk, rows = static_cast<double>(p.batch) * p.nheads * 1e-3;   // thousands
+    const double state_us = rows * dk * p.dv * 8e-3 / 3.0;                            // in and out at 3 TB/s
+    const double chunked = 16.0 + 0.055 * dk + 0.04 * dk * rows + state_us;
+    const double block_us = p.dk > 384 ? 7.8 : 0.5 + 0.0087 * std::max(dk, 58.0);     // per token of 1000 blocks
+    return 3.0 + 0.3 * state_us + 1e-3 * static_cast<double>(WideBlocks(p)) * block_us * p.seqlen <= chunked;
+}
+
 }  // namespace
 
 bool GatedDeltaNet2StepFits(const GatedDeltaNet2Params &p) {
@@ -252,14 +273,13 @@ bool GatedDeltaNet2StepFits(const GatedDeltaNet2Params &p) {
     for (Override o : {kOverrideGdn2Path, kOverrideGdn2Pairwise, kOverrideGdn2Kpw4, kOverrideGdn2Windowed,
                        kOverrideGdn2Split, kOverrideGdn2Ct})
         if (GetOverride(o) != 0) return false;   // a variant of another path is asked for
-    return true;
+    return WideBlocks(p) < kStepWideBlocks || StepIsCheaper(p);
 }
 
 bool LaunchGatedDeltaNet2Step(const GatedDeltaNet2Params &p, void *stream_v) {
     if (!GatedDeltaNet2StepFits(p)) return false;
     hipStream_t stream = static_cast<hipStream_t>(stream_v);
-    const long long wide = static_cast<long long>(p.batch) * p.nheads * ((p.dv + 63) / 64);
-    if (wide >= kStepWideBlocks) LaunchStepKeys<16>(p, stream);
+    if (WideBlocks(p) >= kStepWideBlocks) LaunchStepKeys<16>(p, stream);
     else LaunchStepKeys<8>(p, stream);
     XM_LAUNCH_CHECK("GatedDeltaNet2Fn (step)");
     return true;

@@ -104,11 +104,12 @@ size_t GatedDeltaNet2ScratchBytes(int batch, int seqlen, int nheads, int dk, int
 // GatedDeltaNet2ScratchBytes chose for cap = scratch_bytes.
 void LaunchGatedDeltaNet2(GatedDeltaNet2Params p, void *scratch, size_t scratch_bytes, void *stream);
 // A few tokens (gated_deltanet2_step.hip): unpacked, seqlen up to
-// kGdn2StepTokens, dk <= kGdn2ChunkKeyLimit, no output over q, k, g or beta, no
-// override that asks for a variant of another path.  No scratch.  Launch: false, launching nothing,
+// kGdn2StepTokens, dk <= kGdn2ChunkKeyLimit, no output over q, k, g or beta, not
+// so many small heads that the chunked path is cheaper, no override that asks for
+// a variant of another path.  No scratch.  Launch: false, launching nothing,
 // when it does not fit.  The limit is one chunk of the chunked path, whose
 // time does not depend on how full the chunk is; at 16 tokens the step kernel
-// is still ahead everywhere measured (us, chunked / step: 32 x 16 heads at
+// is still ahead up to about a thousand heads (us, chunked / step: 32 x 16 heads at
 // 128 x 128 42.8 / 35.2, 1 x 4 heads 22.7 / 15.3, 2 x 8 heads at 256 x 256
 // 29.0 / 19.1, 64 x 16 heads at 64 x 64 33.8 / 27.3), and grows by 1 to 1.5 us
 // a token where a second chunk costs the chunked path about 1.
