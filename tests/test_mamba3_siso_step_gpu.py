@@ -146,7 +146,7 @@ def test_step_states_in_place(p, heads, rows, tokens):
     compare(f"in_place_p{p}_h{heads}_t{tokens}", outs, [x.cpu().numpy() for x in want], TOL_GPU)
 
 
-@pytest.mark.parametrize("tokens", [1, 4, 6])
+@pytest.mark.parametrize("tokens", [1, 4, 5])
 @pytest.mark.parametrize("over", ["V", "Z", "Q", "behind_V"])
 def test_y_over_an_input(over, tokens):
     """y over V or Z, which a block reads only in its own rows and tokens: as ever;

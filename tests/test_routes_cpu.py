@@ -132,3 +132,12 @@ def gdn2_launches(b, t, h, dk, dv):
 def test_gdn2_step_or_chunked(call, step):
     """Without a GPU the chunked path ends at its scratch, before any launch."""
     assert gdn2_launches(*call) == (["Gdn2StepKernel"] if step else []), xp.last_launches()
+
+
+@pytest.mark.parametrize("call,step", [
+    ((2, 16, 128, 64, 128), True), ((1, 5, 104, 64, 16), True), ((1, 8, 104, 64, 16), False), ((298, 8, 1, 32, 32), True),
+    ((298, 14, 1, 32, 32), False), ((61, 10, 6, 16, 64), False), ((61, 8, 6, 16, 64), True), ((720, 16, 1, 64, 32), True),
+], ids=str)
+def test_m3_step_or_chunked(call, step):
+    b, t, h, p, n = call
+    assert (m3_launches(b, t, h, p, n, n // 2) == STEP) == step, xp.last_launches()

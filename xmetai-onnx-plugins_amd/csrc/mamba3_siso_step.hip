@@ -42,8 +42,18 @@ static_assert(kTB == kThreads / 64, "one wave per token");
 constexpr long long kBlocks64 = 512, kBlocks32 = 128;
 // Tokens: up to one chunk of the chunked kernel (kM3StepTokens), half of one
 // where the call has less than a 64-row block per CU: there the chunked kernel
-// takes about 10 us whatever the tokens, and 16 tokens here 10 to 12.
+// takes about 10 us whatever the tokens, and 16 tokens here 10 to 12; also where
+// a block is mostly padding (up to 16 rows, or 32 keys and less than 64 rows),
+// and five with few blocks of up to 32 keys.  Measured us, chunked / here: 298
+// heads of 32 x 32, 14 tokens 7.8 / 11.0; 264 of 48 x 32, 16 tokens 10.6 / 13.1;
+// 720 of 64 x 32, 16 tokens 19.5 / 17.4; 366 of 16 x 64, 10 tokens 8.0 / 9.1; 104 of
+// 64 x 16, 8 tokens 6.0 / 8.4, and 5 tokens of 32 of 96 x 32 5.8 / 5.5.
 constexpr long long kBlocksAllTokens = 256;
+int TokenLimit(const Mamba3SisoParams &p, long long tall) {
+    if (tall < kBlocks32 && p.n <= 32) return 5;
+    if (tall < kBlocksAllTokens || p.p <= 16 || (p.n <= 32 && p.p < 64)) return kM3StepTokens / 2;
+    return kM3StepTokens;
+}
 
 template <int KQ, int RP>   // groups of 64 keys, passes of 16 rows
 __global__ __launch_bounds__(kThreads) void Mamba3StepKernel(Mamba3SisoParams p) {
@@ -329,7 +339,7 @@ bool LaunchMamba3SisoStep(const Mamba3SisoParams &p, void *stream_v) {
     if (shares.with_head && p.p > 64) return false;
     const int one_block = shares.with_head ? p.p : 0;   // rows that must be one block's
     const long long tall = static_cast<long long>(p.batch) * p.nheads * ((p.p + 63) / 64);
-    if (p.seqlen > kM3StepTokens / 2 && tall < kBlocksAllTokens && one_block <= 32) return false;
+    if (p.seqlen > TokenLimit(p, tall) && one_block <= 32) return false;
     hipStream_t stream = static_cast<hipStream_t>(stream_v);
     if (tall >= kBlocks64 || one_block > 32) LaunchStepKeys<4>(p, stream);
     else if (tall >= kBlocks32 || one_block > 16) LaunchStepKeys<2>(p, stream);
