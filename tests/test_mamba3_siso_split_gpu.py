@@ -170,6 +170,28 @@ def test_split_chosen_for_one_prompt():
           TOL_M3, ref32=cref.mamba3_siso(*(inp[k] for k in KEYS), dtype=np.float32))
 
 
+@pytest.mark.parametrize("offsets,heads,split", [([0, 1100, 2000], 8, True), ([0, 40, 2000], 8, True), ([0, 0, 1990], 16, True),
+                                                 ([0, 1000, 2000], 17, False), ([0, 90, 200, 310], 2, False)])
+def test_split_chosen_for_packed_rows(offsets, heads, split):
+    """Packed: up to a quarter of a row block per CU (2 sequences x 16 heads of 64
+    rows here), where sequences of even length would gain; each against itself alone."""
+    s = S(1, offsets[-1], heads, 64, 64, has_z=True)
+    inp = W.mamba3_siso_inputs(s, seed=52)
+    n = len(offsets) - 1
+    states = [to_dev(x) for x in start_states(s, n, 53)]
+    dev = {k: to_dev(inp[k]) for k in KEYS}
+    y, f = xp.mamba3_siso_fn(*dev.values(), return_final_states=True, cu_seqlens=to_dev(np.asarray(offsets, np.int64)),
+                             input_states=tuple(states))
+    assert split_launched() == split, xp.last_launches()
+    for b, (lo, hi) in enumerate(zip(offsets, offsets[1:])):
+        if lo == hi:
+            continue
+        part = [x if k in ("Q_bias", "K_bias", "D") else (x[:, :, lo:hi] if k in ("ADT", "DT", "Trap") else x[:, lo:hi]).contiguous()
+                for k, x in dev.items()]
+        y1, f1 = xp.mamba3_siso_fn(*part, return_final_states=True, input_states=tuple(x[b:b + 1].contiguous() for x in states))
+        compare(f"chosen_packed_h{heads}_{b}", (y[:, lo:hi], *(x[b:b + 1] for x in f)), [x.cpu().numpy() for x in (y1, *f1)], TOL_GPU)
+
+
 def test_output_over_an_input_is_not_split(override):
     import ctypes
     import torch

@@ -68,8 +68,17 @@ def test_step_keys(n, tokens):
 @pytest.mark.parametrize("heads,rows", [(2, 16), (64, 32), (256, 64)])
 def test_step_rows(p, heads, rows):
     got, ref = run(S(2, 3, heads, p, 32, angles=5), seed=p)
-    assert step_rows() in (rows, 2 * rows), xp.last_launches()   # more 64-row blocks above 64 rows
+    assert step_rows() == rows, xp.last_launches()
     compare(f"p{p}_h{heads}", got, ref, TOL_M3)
+
+
+@pytest.mark.parametrize("p,heads,rows", [(64, 127, 16), (64, 128, 32), (65, 63, 16), (65, 64, 32), (64, 511, 32), (64, 512, 64),
+                                          (100, 255, 32), (100, 256, 64)])
+def test_step_row_thresholds(p, heads, rows):
+    """32 rows from 128 blocks of 64 rows on, 64 from 512."""
+    got, ref = run(S(1, 2, heads, p, 32, angles=5), seed=heads)
+    assert step_rows() == rows, xp.last_launches()
+    compare(f"threshold_p{p}_h{heads}", got, ref, TOL_M3)
 
 
 @pytest.mark.parametrize("tokens", [1, 2, 4, 7, 8])

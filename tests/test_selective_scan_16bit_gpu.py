@@ -89,3 +89,31 @@ def test_ss_16bit_matches_fp32_call_on_the_same_values(fmt):
     b = y32.to(tdt).float().cpu().numpy()
     assert np.all(np.abs(a - b) <= ulp(b, MANT[fmt])), float(np.max(np.abs(a - b) / ulp(b, MANT[fmt])))
     assert np.mean(a != b) <= 1e-3, f"{fmt}: {np.mean(a != b):.4f} of y differ from the rounded fp32 result"
+
+
+@pytest.mark.parametrize("fmt", ["float16", "bfloat16"])
+@pytest.mark.parametrize("length", [2, 30, 258, 510, 514, 1026])
+@pytest.mark.parametrize("dstate", [3, 8, 16, 64])
+def test_ss_16bit_sequence_parallel_even_lengths(fmt, length, dstate, override):
+    """Lengths 2 modulo 4 in the sequence-parallel kernel: rows on 4-byte boundaries,
+    the last group of each row cut in two by its end (what follows the last row is
+    infinite)."""
+    import torch
+    from xmetai_onnx_plugins import last_launches
+    tdt = getattr(torch, fmt)
+    inp = W.selective_scan_inputs(W.SelectiveScanShape(1, 20, length, dstate), seed=19)
+    dev, rounded = {}, dict(inp)
+    for k in KEYS:
+        dev[k] = to_dev(inp[k])
+        if k in DATA + ("B", "C") and inp[k] is not None:
+            buf = torch.full((inp[k].size + 8,), float("inf"), dtype=tdt, device="cuda")
+            dev[k] = buf[:inp[k].size].view(inp[k].shape)
+            dev[k].copy_(to_dev(inp[k]))
+            rounded[k] = dev[k].float().cpu().numpy()
+    override("ss_split", 2)
+    y, h = selective_scan_fn(*(dev[k] for k in KEYS), delta_softplus=True, return_last_state=True)
+    assert last_launches()[0].startswith("SelectiveScanSegKernel<") and last_launches()[0].endswith(",1,1,2>"), last_launches()
+    ref_y, ref_h = cref.selective_scan(*(rounded[k] for k in KEYS), delta_softplus=True, dtype=np.float64, return_state=True)
+    err = np.abs(y.float().cpu().numpy() - ref_y)
+    assert np.all(err <= ulp(ref_y, MANT[fmt]) + 1e-5)
+    check(f"selective_scan_{fmt}/parallel_l{length}_n{dstate}/h", h.cpu().numpy(), ref_h, TOL_SS)
