@@ -569,7 +569,7 @@ Config ChooseConfig(int N) {
         // serial work): 8 x 5120 x 2048 0.311 -> 0.256 ms, 4 x 5120 x 2048
         // 0.214 -> 0.168, 1 x 5120 x 2048 (whole pass) 0.207 -> 0.119
         if (N <= 8) return Layout(4, 2);
-        return Layout(8, 2);   // measured: 0.445 ms vs 0.454 ms (4 lanes) at 8 x 5120 x 2048 x 16
+        return Layout(8, 2);   // measured: 0.333 ms vs 0.352 ms (4 lanes) at 8 x 5120 x 2048 x 16
     }
     if (N <= 32) return Layout(8, 4);
     if (N <= 64) return Layout(16, 4);
